@@ -31,6 +31,27 @@ __device__ __forceinline__ u32x4 ld16_cached(const void *p) {
   return *reinterpret_cast<const u32x4 *>(p);
 }
 
+// The same 128-bit accesses at any address that is a multiple of the element
+// size (global memory takes them as one instruction in the unaligned access
+// mode that amdhsa runs in): rows whose length is no multiple of a vector.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+template <bool ANY> __device__ __forceinline__ u32x4 ld16_stream_at(const void *p) {
+  if constexpr (ANY) return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p));
+  return ld16_stream(p);
+}
+template <bool ANY> __device__ __forceinline__ void st16_stream_at(void *p, u32x4 v) {
+  if constexpr (ANY)
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any *>(p));
+  else
+    st16_stream(p, v);
+}
+template <bool ANY> __device__ __forceinline__ u32x4 ld16_cached_at(const void *p) {
+  if constexpr (ANY) return *reinterpret_cast<const u32x4_any *>(p);
+  return ld16_cached(p);
+}
+
 // ---------------------------------------------------------------------------
 // dtype traits: EPV = elements per 16-byte vector.
 // ---------------------------------------------------------------------------
@@ -128,24 +149,25 @@ template <> struct io<_Float16> {
 // A chunk is E consecutive elements handled by one lane: E = 8 whenever a
 // 16-bit type is involved (one 16-byte vector of it), else 4.  A chunk of a
 // wider type spans E * sizeof(T) / 16 vectors.
-template <typename T, int E, bool STREAM = true>
+// ANY: p is a multiple of the element size only.
+template <typename T, int E, bool STREAM = true, bool ANY = false>
 __device__ __forceinline__ void load_chunk(const T *p, float *f) {
   constexpr int NV = E * (int)sizeof(T) / 16;
   static_assert(NV >= 1, "chunk smaller than one vector");
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    u32x4 r = STREAM ? ld16_stream(p + v * io<T>::EPV)
-                     : ld16_cached(p + v * io<T>::EPV);
+    u32x4 r = STREAM ? ld16_stream_at<ANY>(p + v * io<T>::EPV)
+                     : ld16_cached_at<ANY>(p + v * io<T>::EPV);
     io<T>::unpack(r, f + v * io<T>::EPV);
   }
 }
 
-template <typename T, int E>
+template <typename T, int E, bool ANY = false>
 __device__ __forceinline__ void store_chunk(T *p, const float *f) {
   constexpr int NV = E * (int)sizeof(T) / 16;
 #pragma unroll
   for (int v = 0; v < NV; ++v)
-    st16_stream(p + v * io<T>::EPV, io<T>::pack(f + v * io<T>::EPV));
+    st16_stream_at<ANY>(p + v * io<T>::EPV, io<T>::pack(f + v * io<T>::EPV));
 }
 
 // Stores a chunk (p may be null: nothing is written) and replaces f by the
@@ -172,9 +194,9 @@ __device__ __forceinline__ void store_chunk_readback(T *p, float *f) {
 template <typename T, int E> struct RawChunk {
   static constexpr int NV = E * (int)sizeof(T) / 16;
   u32x4 r[NV];
-  __device__ __forceinline__ void load(const T *p) {
+  template <bool ANY = false> __device__ __forceinline__ void load(const T *p) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) r[v] = ld16_stream(p + v * io<T>::EPV);
+    for (int v = 0; v < NV; ++v) r[v] = ld16_stream_at<ANY>(p + v * io<T>::EPV);
   }
   __device__ __forceinline__ void load_cached(const T *p) {
 #pragma unroll

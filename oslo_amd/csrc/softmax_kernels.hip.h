@@ -5,7 +5,9 @@
 // for sk <= 64 * VPL * E); a wavefront processes RPW rows at once so that
 // short rows still keep several 128-bit loads in flight per lane, and rows of
 // at most 32 chunks (256 16-bit keys) lie side by side in a wavefront, 8, 16
-// or 32 lanes each, so that no lane idles.  Keys that
+// or 32 lanes each, so that no lane idles.  Rows whose length is no multiple
+// of a chunk, or whose operands are not 16-byte aligned, take the same kernels
+// in a build that accesses the chunks where they lie (RAG).  Keys that
 // are masked out are never loaded: the causal kernels stop at the diagonal,
 // the masked kernels read the mask bytes of a chunk first and skip the chunk
 // when all of them are set.  Probabilities of masked keys are written as
@@ -158,18 +160,26 @@ __device__ __forceinline__ float row_reduce_max(float a, float *red, int wave,
 }
 
 // Mask bytes of one chunk -> bit e set when key e of the chunk is masked out.
-template <int E>
+template <int E, bool ANY>
 __device__ __forceinline__ uint32_t load_mask_bits(const uint8_t *p) {
   uint32_t bits = 0;
   if constexpr (E == 8) {
-    const u32x2 m = *reinterpret_cast<const u32x2 *>(p);
+    u32x2 m;
+    if constexpr (ANY)
+      m = *reinterpret_cast<const u32x2_any *>(p);
+    else
+      m = *reinterpret_cast<const u32x2 *>(p);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       bits |= ((m.x >> (8 * e)) & 0xffu) ? (1u << e) : 0u;
       bits |= ((m.y >> (8 * e)) & 0xffu) ? (1u << (4 + e)) : 0u;
     }
   } else {
-    const uint32_t m = *reinterpret_cast<const uint32_t *>(p);
+    uint32_t m;
+    if constexpr (ANY)
+      m = *reinterpret_cast<const u32_any *>(p);
+    else
+      m = *reinterpret_cast<const uint32_t *>(p);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       bits |= ((m >> (8 * e)) & 0xffu) ? (1u << e) : 0u;
@@ -177,16 +187,16 @@ __device__ __forceinline__ uint32_t load_mask_bits(const uint8_t *p) {
   return bits;
 }
 
-// Mask bits of chunk c (E keys) of a row that sees `visible` keys through the
-// diagonal: the keys from `visible` on are hidden as well.  Chunks that lie
-// beyond the diagonal altogether do not read their mask bytes.
-template <int E>
-__device__ __forceinline__ uint32_t masked_chunk_bits(const uint8_t *mrow, int c,
+// Mask bits of the chunk of keys i0 .. i0 + E of a row that sees `visible` keys
+// through the diagonal: the keys from `visible` on are hidden as well.  Chunks
+// that lie beyond the diagonal altogether do not read their mask bytes.
+template <int E, bool ANY>
+__device__ __forceinline__ uint32_t masked_chunk_bits(const uint8_t *mrow, int i0,
                                                       int visible) {
   constexpr uint32_t kAllBits = (1u << E) - 1u;
-  const int left = visible - c * E;  // keys of the chunk below the diagonal
+  const int left = visible - i0;  // keys of the chunk below the diagonal
   if (left <= 0) return kAllBits;
-  uint32_t mb = load_mask_bits<E>(mrow + (int64_t)c * E);
+  uint32_t mb = load_mask_bits<E, ANY>(mrow + i0);
   if (left < E) mb |= kAllBits & ~((1u << left) - 1u);
   return mb;
 }
@@ -257,27 +267,27 @@ __device__ __forceinline__ void row_setup(const SoftmaxGeom &g, int64_t r,
 // One chunk of the additive term, E values of the logits' type T or of float
 // (a launch-uniform choice, so one kernel serves both), converted to float as
 // soon as it arrives: the float form is no wider than a float chunk as loaded.
-template <typename T, int E>
-__device__ __forceinline__ void load_bias_chunk(const uint8_t *row, int c, bool f32, float *f) {
+template <typename T, int E, bool ANY>
+__device__ __forceinline__ void load_bias_chunk(const uint8_t *row, int i0, bool f32, float *f) {
   if (sizeof(T) == 4 || f32) {
 #pragma unroll
     for (int v = 0; v < E / 4; ++v)
-      io<float>::unpack(ld16_cached(row + ((int64_t)c * E + 4 * v) * 4), f + 4 * v);
+      io<float>::unpack(ld16_cached_at<ANY>(row + ((int64_t)i0 + 4 * v) * 4), f + 4 * v);
   } else {
-    io<T>::unpack(ld16_cached(row + (int64_t)c * E * (int64_t)sizeof(T)), f);
+    io<T>::unpack(ld16_cached_at<ANY>(row + (int64_t)i0 * (int64_t)sizeof(T)), f);
   }
 }
 
 // The same in two steps, for code that issues all its loads before it
 // converts any of them: the chunk as loaded (E / 4 vectors, the first one only
 // for a 16-bit term), then its conversion.
-template <typename T, int E>
-__device__ __forceinline__ void load_bias_raw(const uint8_t *row, int c, bool f32, u32x4 *r) {
+template <typename T, int E, bool ANY>
+__device__ __forceinline__ void load_bias_raw(const uint8_t *row, int i0, bool f32, u32x4 *r) {
   if (sizeof(T) == 4 || f32) {
 #pragma unroll
-    for (int v = 0; v < E / 4; ++v) r[v] = ld16_cached(row + ((int64_t)c * E + 4 * v) * 4);
+    for (int v = 0; v < E / 4; ++v) r[v] = ld16_cached_at<ANY>(row + ((int64_t)i0 + 4 * v) * 4);
   } else {
-    r[0] = ld16_cached(row + (int64_t)c * E * (int64_t)sizeof(T));
+    r[0] = ld16_cached_at<ANY>(row + (int64_t)i0 * (int64_t)sizeof(T));
   }
 }
 template <typename T, int E>
@@ -307,6 +317,67 @@ __device__ __forceinline__ float bias_at(const uint8_t *row, int i, bool f32) {
   return io<T>::from_scalar(reinterpret_cast<const T *>(row)[i]);
 }
 
+// ---------------------------------------------------------------------------
+// Ragged rows (RAG builds; bound: HBM, with dropout VALU): a row length that is no multiple of a chunk, or
+// operands off the 16-byte grid.  The chunks are counted from the first key of
+// the row and accessed where they lie; the last one ends with the row and
+// overlaps the chunk before it, so that every access is a whole vector inside
+// the row.  Its first dup_keys() keys are held twice: they count once in the
+// sums, and both lanes store the same bits.  (One wave per row with 2-byte
+// accesses before; bf16 causal [51, 1531, 1531]: forward 176 -> 67 us,
+// backward 246 -> 89, with dropout 390 -> 79 and 305 -> 94; fp32 1003 keys
+// 94 -> 78 and 126 -> 96 us.)
+// ---------------------------------------------------------------------------
+template <int E, bool RAG>
+__device__ __forceinline__ int chunk_key(int c, int sk) {
+  const int i0 = c * E;
+  if constexpr (RAG) return i0 < sk - E ? i0 : sk - E;
+  return i0;
+}
+template <int E, bool RAG>
+__device__ __forceinline__ int dup_keys(int c, int sk) {
+  return RAG ? c * E - chunk_key<E, RAG>(c, sk) : 0;
+}
+
+// Dropout of a ragged row: its chunks straddle the groups of eight elements of
+// the flattened tensor.  The lanes of the row (`stride` of them, this one is
+// number `idx`) draw its groups once, one byte of keep bits each, into LDS
+// (kb), as many as reach `keys` keys; a chunk then takes its bits from two
+// neighbouring bytes.
+template <int E>
+__device__ __forceinline__ void draw_row_groups(uint8_t *kb, int64_t row, int sk, int keys,
+                                                int idx, int stride, const DropArgs &d) {
+  const uint64_t flat = (uint64_t)row * (uint64_t)sk;
+  // (all of the last chunk that holds one of the keys)
+  const int upto = keys + E - 1 < sk ? keys + E - 1 : sk;
+  const int groups = keys > 0 ? ((int)(flat & 7u) + upto + 7) >> 3 : 0;
+  for (int t = idx; t < groups; t += stride)
+    kb[t] = (uint8_t)dropout_keep_bits((flat >> 3) + (uint64_t)t, d.seed, d.offset, d.threshold);
+}
+// makes the draws of the row's lanes visible to each other
+__device__ __forceinline__ void row_draws_done(int wpr) {
+  if (wpr > 1) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+__device__ __forceinline__ uint32_t row_keep_bits(const uint8_t *kb, int64_t row, int sk, int i0) {
+  const uint32_t at = ((uint32_t)((uint64_t)row * (uint64_t)sk) & 7u) + (uint32_t)i0;
+  typedef uint16_t u16_any __attribute__((aligned(1)));
+  return (uint32_t)*reinterpret_cast<const u16_any *>(kb + (at >> 3)) >> (at & 7u);
+}
+// v where bit e of the keep bits is set, else +0: two instructions
+__device__ __forceinline__ float keep_or_zero(float v, uint32_t keep, int e) {
+  return __uint_as_float(__float_as_uint(v) &
+                         (uint32_t)__builtin_amdgcn_sbfe((int)keep, e, 1));
+}
+// bytes of keep bits per lane group of a row: one for each chunk it can hold,
+// one for the group that the row's first key shifts past them, one that is
+// read but never used
+constexpr int keep_bytes(int lanes, int vpl) { return lanes * vpl + 2; }
+
 // DROP: dropout is applied to the probabilities before they are written
 // (oslo/transformers/models/gpt2/modeling_gpt2.py:138-142,
 // oslo/transformers/models/bert/modeling_bert.py:306-310) and the row
@@ -317,7 +388,8 @@ __device__ __forceinline__ float bias_at(const uint8_t *row, int i, bool f32) {
 // LPR lanes hold a row: 64 (a row takes whole waves), or 8 / 16 / 32 for rows
 // of at most LPR chunks, where a wave works on 64 / LPR rows side by side
 // (then VPL == 1 and wpr == 1).
-template <typename T, int VPL, int RPW, int MODE, bool DROP, int LPR = kWave>
+template <typename T, int VPL, int RPW, int MODE, bool DROP, int LPR = kWave,
+          bool RAG = false>
 __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     const T *__restrict__ x, const uint8_t *__restrict__ mask,
     T *__restrict__ y, float *__restrict__ stats, SoftmaxGeom g, float scale,
@@ -325,13 +397,15 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
   d = resolve_drop(d);
   constexpr int E = io<T>::EPV;
   constexpr uint32_t kAll = (1u << E) - 1u;
+  static_assert(!RAG || RPW == 1, "ragged rows: one row set per wave");
   __shared__ float red[2][16];
+  extern __shared__ uint8_t kbs[];  // ragged rows with dropout: the rows' keep bits
   const int lane = threadIdx.x & 63;
   // the wave index is uniform: keep it (and the row arithmetic) in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rslot = g.wpr == 1 ? wave : wave / g.wpr;  // (uniform: the division is skipped)
   const int first = rslot * g.wpr;
-  const int nchunks = g.sk / E;
+  const int nchunks = RAG ? (g.sk + E - 1) / E : g.sk / E;
   const int cstride = LPR == kWave ? kWave * g.wpr : LPR;
   constexpr int SUB = kWave / LPR;  // rows side by side in a wave
   const int sl = LPR == kWave ? lane : (lane & (LPR - 1));
@@ -351,6 +425,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
   // gets zeros (its neighbours in the wave may well see keys, so the
   // wave-uniform shortcuts below do not catch it)
   bool nokey[RPW];
+  int vis[RAG ? RPW : 1];  // keys below the diagonal
   const uint8_t *mrow0 = nullptr;
   // additive term (kModeBias): the chunks as loaded, and whether a chunk's
   // logits were left unread
@@ -370,6 +445,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     row[j] = 0;
     if (rvalid[j]) row_setup<MODE>(g, r, mask, row[j], visible, mrow);
     nokey[j] = MODE == kModeBias && rvalid[j] && visible <= 0;
+    if constexpr (RAG) vis[j] = visible;
     // consecutive rows of a wave normally share their mask row (a key-padding
     // mask [b, 1, 1, sk]): its bits are then read and unpacked once
     bool shared = false;
@@ -386,10 +462,10 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
       } else if (rvalid[j] && c < nchunks) {
         if constexpr (MODE == kModeCausal || MODE == kModeBias) {
           // (visible == sk without a diagonal)
-          const int left = visible - c * E;  // visible keys in this chunk
+          const int left = visible - chunk_key<E, RAG>(c, g.sk);  // visible keys in this chunk
           mb = left >= E ? 0u : (left <= 0 ? mb : (mb & ~((1u << left) - 1u)));
         } else {
-          mb = masked_chunk_bits<E>(mrow, c, visible);
+          mb = masked_chunk_bits<E, RAG>(mrow, chunk_key<E, RAG>(c, g.sk), visible);
         }
       }
       mbits[j][k] = mb;
@@ -399,7 +475,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         // (all of them requested before any is converted: a conversion
         //  waits for its load)
         bhid[j][k] = false;
-        if (mb != kAll) load_bias_raw<T, E>(mrow, c, bias_f32, braw[j][k]);
+        if (mb != kAll)
+          load_bias_raw<T, E, RAG>(mrow, chunk_key<E, RAG>(c, g.sk), bias_f32, braw[j][k]);
       }
     }
   }
@@ -427,9 +504,9 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
       //  used: every select below takes the masked branch for it)
       bool want = mbits[j][k] != (1u << E) - 1u;
       if constexpr (MODE == kModeBias) {
-        if (want && !bhid[j][k]) xraw[j][k].load(xr + (int64_t)c * E);
+        if (want && !bhid[j][k]) xraw[j][k].template load<RAG>(xr + chunk_key<E, RAG>(c, g.sk));
       } else {
-        if (want) load_chunk<T, E>(xr + (int64_t)c * E, v[j][k]);
+        if (want) load_chunk<T, E, true, RAG>(xr + chunk_key<E, RAG>(c, g.sk), v[j][k]);
       }
     }
   }
@@ -448,6 +525,14 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
 #pragma unroll
       for (int k = 0; k < VPL; ++k)
         if (mbits[j][k] != kAll && !bhid[j][k]) xraw[j][k].unpack(v[j][k]);
+  }
+
+  // (the draws of a ragged row wait in LDS while its loads are in flight)
+  uint8_t *kb = nullptr;
+  if constexpr (RAG && DROP) {
+    kb = kbs + (LPR == kWave ? rslot : wave * SUB + lane / LPR) *
+                   keep_bytes(LPR == kWave ? kWave * g.wpr : LPR, VPL);
+    if (rvalid[0]) draw_row_groups<E>(kb, row[0], g.sk, vis[0], c0, cstride, d);
   }
 
   // Wave-uniform shortcuts: where no lane of the wave sees a key of chunk
@@ -559,7 +644,10 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         if constexpr (kBias) d = mul_rn(d, kLog2e);
         const float p = __builtin_amdgcn_exp2f(d);
         v[j][k][e] = p;  // exp2(-inf) == 0 for masked keys
-        s += p;
+        if constexpr (RAG)
+          s += e < dup_keys<E, RAG>(c0 + k * cstride, g.sk) ? 0.f : p;
+        else
+          s += p;
       }
     }
     sm[j] = s;
@@ -567,6 +655,12 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
 #pragma unroll
   for (int j = 0; j < RPW; ++j)
     sm[j] = row_reduce_sum<LPR>(sm[j], red[1], wave, first, g.wpr, lane);
+  if constexpr (RAG && DROP) {
+    // a row without a visible key is uniform: all of it is drawn
+    if (rvalid[0] && mx[0] == ninf && !kBias)
+      draw_row_groups<E>(kb, row[0], g.sk, g.sk, c0, cstride, d);
+    row_draws_done(g.wpr);
+  }
 
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
@@ -589,7 +683,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     // 2m + 1, and one DPP swap hands each lane the other's result.  (Rows of a
     // multiple of 8 keys, so that groups do not straddle rows; the row and the
     // conditions below are uniform over the wave, so all lanes are active.)
-    constexpr bool kPairDraw = DROP && E == 4 && LPR == kWave && VPL % 2 == 0;
+    constexpr bool kPairDraw = DROP && !RAG && E == 4 && LPR == kWave && VPL % 2 == 0;
     uint32_t keepk[kPairDraw ? VPL : 1];
     bool paired = false;
     if constexpr (kPairDraw) {
@@ -634,12 +728,14 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         if constexpr (DROP) {
           // exact zeros need no draw (wave-uniform test)
           if (!none_visible[j][k] || empty) {
-            if constexpr (kPairDraw) {
-              const uint32_t keep =
-                  paired ? keepk[k] : chunk_keep_bits<E>(row[j], g.sk, c, d);
+            if constexpr (kPairDraw || RAG) {
+              uint32_t keep;
+              if constexpr (RAG)
+                keep = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk));
+              else
+                keep = paired ? keepk[k] : chunk_keep_bits<E>(row[j], g.sk, c, d);
 #pragma unroll
-              for (int e = 0; e < E; ++e)
-                o[e] = (keep >> e) & 1u ? o[e] * d.scale : 0.f;
+              for (int e = 0; e < E; ++e) o[e] = keep_or_zero(o[e] * d.scale, keep, e);
             } else {
               const KeepWords<E> keep = chunk_keep_words<E>(row[j], g.sk, c, d);
 #pragma unroll
@@ -648,7 +744,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
             }
           }
         }
-        store_chunk<T, E>(yr + (int64_t)c * E, o);
+        store_chunk<T, E, RAG>(yr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }
@@ -658,7 +754,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
 // recomputed as exp2(x * scale * log2 e - stats[row][0]) * stats[row][1], the
 // keep bits are regenerated from (seed, offset), and
 // dx = scale * y * (dp - sum_k dp_k y_k) with dp = keep * dy / (1 - p).
-template <typename T, int VPL, int RPW, int MODE, int LPR = kWave>
+template <typename T, int VPL, int RPW, int MODE, int LPR = kWave, bool RAG = false>
 __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     const T *__restrict__ dy, const T *__restrict__ x,
     const float *__restrict__ stats, const uint8_t *__restrict__ mask,
@@ -666,12 +762,14 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
   d = resolve_drop(d);
   constexpr int E = io<T>::EPV;
   constexpr uint32_t kAll = (1u << E) - 1u;
+  static_assert(!RAG || RPW == 1, "ragged rows: one row set per wave");
   __shared__ float red[16];
+  extern __shared__ uint8_t kbs[];  // ragged rows: the rows' keep bits
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rslot = g.wpr == 1 ? wave : wave / g.wpr;  // (uniform: the division is skipped)
   const int first = rslot * g.wpr;
-  const int nchunks = g.sk / E;
+  const int nchunks = RAG ? (g.sk + E - 1) / E : g.sk / E;
   const int cstride = LPR == kWave ? kWave * g.wpr : LPR;
   constexpr int SUB = kWave / LPR;
   const int sl = LPR == kWave ? lane : (lane & (LPR - 1));
@@ -685,6 +783,7 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
   int64_t row[RPW];
   bool rvalid[RPW];
   float rmax[RPW], rinv[RPW];
+  int vis[RAG ? RPW : 1];  // keys that count below the diagonal
   constexpr bool kBias = MODE == kModeBias;
   float bv[kBias ? RPW : 1][kBias ? VPL : 1][kBias ? E : 1];
   const bool bias_f32 = g.bias_esize == 4;
@@ -706,23 +805,25 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     // uniform row: every key counts (with an additive term there is no such
     // convention: the probabilities are what the arithmetic gives)
     const bool empty = rinv[j] < 0.f && !kBias;
+    if constexpr (RAG) vis[j] = empty ? g.sk : visible;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
+      const int i0 = chunk_key<E, RAG>(c, g.sk);
       uint32_t mb = kAll;
       if (rvalid[j] && c < nchunks) {
         if (empty) {
           mb = 0u;
         } else if constexpr (MODE == kModeCausal || MODE == kModeBias) {
-          const int left = visible - c * E;
+          const int left = visible - i0;
           mb = left >= E ? 0u : (left <= 0 ? mb : (mb & ~((1u << left) - 1u)));
         } else {
-          mb = masked_chunk_bits<E>(mrow, c, visible);
+          mb = masked_chunk_bits<E, RAG>(mrow, i0, visible);
         }
       }
       if constexpr (kBias) {
         if (mb != kAll) {
-          load_bias_chunk<T, E>(mrow, c, bias_f32, bv[j][k]);
+          load_bias_chunk<T, E, RAG>(mrow, i0, bias_f32, bv[j][k]);
           // A chunk whose terms all absorb their logits has probability 0
           // throughout, unless the row's maximum is such a term itself (a
           // row without any other key): skip it altogether
@@ -741,8 +842,8 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
       if (mbits[j][k] != kAll) {
-        load_chunk<T, E>(xr + (int64_t)c * E, yv[j][k]);
-        load_chunk<T, E>(gr + (int64_t)c * E, gv[j][k]);
+        load_chunk<T, E, true, RAG>(xr + chunk_key<E, RAG>(c, g.sk), yv[j][k]);
+        load_chunk<T, E, true, RAG>(gr + chunk_key<E, RAG>(c, g.sk), gv[j][k]);
       } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -751,6 +852,14 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
         }
       }
     }
+  }
+  // (the draws of a ragged row are made while its loads are in flight)
+  uint8_t *kb = nullptr;
+  if constexpr (RAG) {
+    kb = kbs + (LPR == kWave ? rslot : wave * SUB + lane / LPR) *
+                   keep_bytes(LPR == kWave ? kWave * g.wpr : LPR, VPL);
+    if (rvalid[0]) draw_row_groups<E>(kb, row[0], g.sk, vis[0], c0, cstride, d);
+    row_draws_done(g.wpr);
   }
   bool none_loaded[RPW][VPL];
 #pragma unroll
@@ -770,7 +879,15 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
       const int c = c0 + k * cstride;
       // (a chunk without a visible key was not loaded: its gradients are zeros
       //  whatever the draw says)
-      const KeepWords<E> keep = chunk_keep_words<E>(row[j], g.sk, c, d);
+      KeepWords<E> keep;
+      uint32_t keep_bits = 0;
+      int dup = 0;
+      if constexpr (RAG) {
+        keep_bits = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk));
+        dup = dup_keys<E, RAG>(c, g.sk);
+      } else {
+        keep = chunk_keep_words<E>(row[j], g.sk, c, d);
+      }
       const float *bf = nullptr;
       if constexpr (kBias) bf = bv[j][k];
       // (the selects below stay per element: a wave-uniform branch around
@@ -792,10 +909,17 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
         }
         if (empty) p = -rinv[j];
         if ((mbits[j][k] >> e) & 1u) p = 0.f;
-        const float dp = keep.kept(e) ? mul_rn(gv[j][k][e], d.scale) : 0.f;
+        float dp;
+        if constexpr (RAG)
+          dp = keep_or_zero(mul_rn(gv[j][k][e], d.scale), keep_bits, e);
+        else
+          dp = keep.kept(e) ? mul_rn(gv[j][k][e], d.scale) : 0.f;
         yv[j][k][e] = p;
         gv[j][k][e] = dp;
-        a += p * dp;
+        if constexpr (RAG)
+          a += e < dup ? 0.f : p * dp;
+        else
+          a += p * dp;
       }
     }
     s[j] = a;
@@ -821,13 +945,13 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
           for (int e = 0; e < E; ++e)
             o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
         }
-        store_chunk<T, E>(dxr + (int64_t)c * E, o);
+        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }
 }
 
-template <typename T, int VPL, int RPW, int MODE, int LPR = kWave>
+template <typename T, int VPL, int RPW, int MODE, int LPR = kWave, bool RAG = false>
 __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     const T *__restrict__ dy, const T *__restrict__ y,
     const uint8_t *__restrict__ mask, T *__restrict__ dx, SoftmaxGeom g,
@@ -840,7 +964,7 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rslot = g.wpr == 1 ? wave : wave / g.wpr;  // (uniform: the division is skipped)
   const int first = rslot * g.wpr;
-  const int nchunks = g.sk / E;
+  const int nchunks = RAG ? (g.sk + E - 1) / E : g.sk / E;
   const int cstride = LPR == kWave ? kWave * g.wpr : LPR;
   constexpr int SUB = kWave / LPR;
   const int sl = LPR == kWave ? lane : (lane & (LPR - 1));
@@ -866,20 +990,21 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
+      const int i0 = chunk_key<E, RAG>(c, g.sk);
       bool sk_ = true;
       if (rvalid[j] && c < nchunks) {
         if constexpr (MODE == kModeCausal) {
-          sk_ = visible - c * E <= 0;
+          sk_ = visible - i0 <= 0;
         } else if constexpr (MODE == kModeMasked) {
-          sk_ = masked_chunk_bits<E>(mrow, c, visible) == kAll;
+          sk_ = masked_chunk_bits<E, RAG>(mrow, i0, visible) == kAll;
         } else if constexpr (MODE == kModeBias) {
           // beyond the diagonal, or every additive term of the chunk absorbs
           // its logit: the probabilities are zeros (unless the whole row is
           // like that, which the test below catches)
-          sk_ = visible - c * E <= 0;
+          sk_ = visible - i0 <= 0;
           if (!sk_) {
             float bf[E];
-            load_bias_chunk<T, E>(mrow, c, g.bias_esize == 4, bf);
+            load_bias_chunk<T, E, RAG>(mrow, i0, g.bias_esize == 4, bf);
             sk_ = bias_all_hidden<E>(bf);
           }
         } else {
@@ -908,8 +1033,8 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
       if (!skip[j][k]) {
-        load_chunk<T, E>(yr + (int64_t)c * E, yv[j][k]);
-        load_chunk<T, E>(gr + (int64_t)c * E, gv[j][k]);
+        load_chunk<T, E, true, RAG>(yr + chunk_key<E, RAG>(c, g.sk), yv[j][k]);
+        load_chunk<T, E, true, RAG>(gr + chunk_key<E, RAG>(c, g.sk), gv[j][k]);
       } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -935,7 +1060,12 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     for (int k = 0; k < VPL; ++k) {
       if (none_loaded[j][k]) continue;
 #pragma unroll
-      for (int e = 0; e < E; ++e) a += yv[j][k][e] * gv[j][k][e];
+      for (int e = 0; e < E; ++e) {
+        if constexpr (RAG)
+          a += e < dup_keys<E, RAG>(c0 + k * cstride, g.sk) ? 0.f : yv[j][k][e] * gv[j][k][e];
+        else
+          a += yv[j][k][e] * gv[j][k][e];
+      }
     }
     s[j] = a;
   }
@@ -960,14 +1090,14 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
           for (int e = 0; e < E; ++e)
             o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
         }
-        store_chunk<T, E>(dxr + (int64_t)c * E, o);
+        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// generic kernels: any sk / alignment; one 256-thread workgroup per row,
+// generic kernels: rows beyond sixteen waves; one 256-thread workgroup per row,
 // three passes over the (L2-resident) row.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float block_reduce_256(float v, float *sh, bool is_max) {
@@ -1116,168 +1246,60 @@ __global__ __launch_bounds__(256) void softmax_bwd_generic_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// generic rows of at most kWaveRowMax keys: one wavefront per row, the row in
-// registers, no LDS and no barrier.  A lane accesses EW consecutive keys at a
-// time (lane l holds keys EW * (l + 64 k) ...): EW = 4 or 2 when the row
-// length and the pointers allow 8- or 4-byte accesses, else 1 (any length and
-// alignment).  The arithmetic is that of the kernels above, term for term.
+// rows of fewer keys than a chunk (below 8 in a 16-bit type, below 4 in fp32):
+// eight lanes hold a row, one key each.  The arithmetic is that of the kernels
+// above, term for term.
 // ---------------------------------------------------------------------------
-constexpr int kWaveRowMax = 2048;  // 32 elements per lane and operand; builds for 256, 1024, 2048
+constexpr int kTinyLanes = 8;
+constexpr int kTinyRows = 256 / kTinyLanes;  // rows of a workgroup
 
-template <typename T, int EW>
-__device__ __forceinline__ void ld_small(const T *p, float *f) {
-  if constexpr (EW == 1) {
-    f[0] = io<T>::from_scalar(p[0]);
-  } else {
-    T t[EW];
-    if constexpr (EW * sizeof(T) == 4) {
-      const uint32_t raw = *reinterpret_cast<const uint32_t *>(p);
-      __builtin_memcpy(t, &raw, 4);
-    } else {
-      static_assert(EW * sizeof(T) == 8, "at most 8 bytes per access");
-      const u32x2 raw = *reinterpret_cast<const u32x2 *>(p);
-      __builtin_memcpy(t, &raw, 8);
-    }
-#pragma unroll
-    for (int e = 0; e < EW; ++e) f[e] = io<T>::from_scalar(t[e]);
-  }
-}
-
-template <typename T, int EW>
-__device__ __forceinline__ void st_small(T *p, const float *f) {
-  if constexpr (EW == 1) {
-    p[0] = io<T>::to_scalar(f[0]);
-  } else {
-    T t[EW];
-#pragma unroll
-    for (int e = 0; e < EW; ++e) t[e] = io<T>::to_scalar(f[e]);
-    if constexpr (EW * sizeof(T) == 4) {
-      uint32_t raw;
-      __builtin_memcpy(&raw, t, 4);
-      *reinterpret_cast<uint32_t *>(p) = raw;
-    } else {
-      u32x2 raw;
-      __builtin_memcpy(&raw, t, 8);
-      *reinterpret_cast<u32x2 *>(p) = raw;
-    }
-  }
-}
-
-// bit e set: key i0 + e is masked out (EW consecutive mask bytes, EW-aligned)
-template <int EW>
-__device__ __forceinline__ uint32_t ld_mask_small(const uint8_t *p) {
-  if constexpr (EW == 1) {
-    return p[0] != 0 ? 1u : 0u;
-  } else if constexpr (EW == 2) {
-    const uint32_t m = *reinterpret_cast<const uint16_t *>(p);
-    return ((m & 0xffu) ? 1u : 0u) | ((m >> 8) ? 2u : 0u);
-  } else {
-    const uint32_t m = *reinterpret_cast<const uint32_t *>(p);
-    uint32_t bits = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bits |= ((m >> (8 * e)) & 0xffu) ? (1u << e) : 0u;
-    return bits;
-  }
-}
-
-// keep bits of the EW consecutive elements that start at flat index `flat`
-// (a multiple of EW, so they lie inside one dropout group)
-template <int EW>
-__device__ __forceinline__ uint32_t keep_small(int64_t flat, const DropArgs &d) {
-  return dropout_keep_bits((uint64_t)flat >> 3, d.seed, d.offset, d.threshold) >>
-         (uint32_t)(flat & 7);
-}
-
-template <typename T, int MODE, bool DROP, int EW, int ROWMAX>
-__global__ __launch_bounds__(256) void softmax_fwd_wave_kernel(
+template <typename T, int MODE, bool DROP>
+__global__ __launch_bounds__(256) void softmax_fwd_tiny_kernel(
     const T *__restrict__ x, const uint8_t *__restrict__ mask,
     T *__restrict__ y, float *__restrict__ stats, SoftmaxGeom g, float scale,
     DropArgs d) {
   d = resolve_drop(d);
-  constexpr int K = ROWMAX / kWave / EW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = threadIdx.x % kTinyLanes;  // key of this lane
   const float ninf = -__builtin_inff();
-  const float c2 = scale * kLog2e;
-  for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < g.rows;
-       r += (int64_t)gridDim.x * 4) {
-    int64_t row;
-    int visible;
-    const uint8_t *mrow;
-    row_setup<MODE>(g, r, mask, row, visible, mrow);
-    const T *xr = x + row * g.sk;
-    T *yr = y + row * g.sk;
-    constexpr bool kBias = MODE == kModeBias;
-    const bool bias_f32 = g.bias_esize == 4;
-    float v[K][EW];
-    float m = ninf;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-#pragma unroll
-      for (int e = 0; e < EW; ++e) v[k][e] = ninf;
-      if (i0 < g.sk) {
-        // keys beyond the diagonal are not loaded; with a mask tensor the
-        // logits are requested together with the mask bytes (waiting for the
-        // mask first measures 30 % slower than the loads it can save)
-        uint32_t hid = 0;
-        if constexpr (MODE == kModeMasked) hid = ld_mask_small<EW>(mrow + i0);
-        const bool none = i0 >= visible;  // (visible == sk without a diagonal)
-        if (!none) {
-          float t[EW];
-          ld_small<T, EW>(xr + i0, t);
-#pragma unroll
-          for (int e = 0; e < EW; ++e) {
-            const bool hidden =
-                MODE == kModeMasked ? (((hid >> e) & 1u) != 0 || i0 + e >= visible)
-                                    : i0 + e >= visible;
-            if (!hidden) {
-              if constexpr (kBias)
-                v[k][e] = __builtin_fmaf(t[e], scale, bias_at<T>(mrow, i0 + e, bias_f32));
-              else
-                v[k][e] = mul_rn(t[e], c2);
-            }
-            m = fmaxf(m, v[k][e]);
-          }
-        }
-      }
+  constexpr bool kBias = MODE == kModeBias;
+  for (int64_t r0 = (int64_t)blockIdx.x * kTinyRows; r0 < g.rows;
+       r0 += (int64_t)gridDim.x * kTinyRows) {
+    const int64_t r = r0 + threadIdx.x / kTinyLanes;
+    int64_t row = 0;
+    int visible = 0;
+    const uint8_t *mrow = nullptr;
+    if (r < g.rows) row_setup<MODE>(g, r, mask, row, visible, mrow);
+    const bool in_row = r < g.rows && i < g.sk;
+    bool hidden = !in_row || i >= visible;
+    if constexpr (MODE == kModeMasked)
+      if (!hidden) hidden = mrow[i] != 0;
+    float v = ninf;
+    if (!hidden) {
+      const float t = io<T>::from_scalar(x[row * g.sk + i]);
+      if constexpr (kBias)
+        v = __builtin_fmaf(t, scale, bias_at<T>(mrow, i, g.bias_esize == 4));
+      else
+        v = mul_rn(t, scale * kLog2e);
     }
-    m = wave_max(m);
+    const float m = group_allreduce<OpMax, kTinyLanes>(v);
     const bool empty = m == ninf && !kBias;
-    const float off = empty ? 0.f : m;
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-#pragma unroll
-      for (int e = 0; e < EW; ++e) {
-        float dd = sub_rn(v[k][e], off);
-        if constexpr (kBias) dd = mul_rn(dd, kLog2e);
-        const float p = __builtin_amdgcn_exp2f(dd);  // 0 for hidden keys
-        v[k][e] = p;
-        s += p;
-      }
-    s = wave_sum(s);
+    float dd = sub_rn(v, empty ? 0.f : m);
+    if constexpr (kBias) dd = mul_rn(dd, kLog2e);
+    // (0 for hidden keys; a lane beyond the row counts nothing even where the
+    //  row's maximum is -inf or NaN)
+    const float p = in_row ? __builtin_amdgcn_exp2f(dd) : 0.f;
+    const float s = group_allreduce<OpSum, kTinyLanes>(p);
+    if (!in_row) continue;
     const float inv = empty ? 0.f : row_recip(s);
     const float fill = empty ? g.inv_sk : 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-      if (i0 < g.sk) {
-        float o[EW];
-        uint32_t keep = 0xffu;
-        if constexpr (DROP) keep = keep_small<EW>(row * g.sk + i0, d);
-#pragma unroll
-        for (int e = 0; e < EW; ++e) {
-          o[e] = v[k][e] * inv + fill;
-          // (a key beyond the diagonal is an exact zero in a NaN row, too)
-          if (kBias && i0 + e >= visible) o[e] = 0.f;
-          if constexpr (kBias) o[e] = pinned(o[e]);
-          if constexpr (DROP) o[e] = (keep >> e) & 1u ? o[e] * d.scale : 0.f;
-        }
-        st_small<T, EW>(yr + i0, o);
-      }
-    }
+    float o = p * inv + fill;
+    // (a key beyond the diagonal is an exact zero in a NaN row, too)
+    if (kBias && i >= visible) o = 0.f;
+    if constexpr (kBias) o = pinned(o);
+    if constexpr (DROP) o = keep_element(row * g.sk + i, d) ? o * d.scale : 0.f;
+    y[row * g.sk + i] = io<T>::to_scalar(o);
     if constexpr (DROP) {
-      if (lane == 0) {
+      if (i == 0) {
         // (a query that the diagonal leaves without any key: zeros above, and
         //  finite statistics for the backward pass)
         const bool nokey = kBias && visible <= 0;
@@ -1288,155 +1310,70 @@ __global__ __launch_bounds__(256) void softmax_fwd_wave_kernel(
   }
 }
 
-template <typename T, int MODE, int EW, int ROWMAX>
-__global__ __launch_bounds__(256) void softmax_dropout_bwd_wave_kernel(
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void softmax_dropout_bwd_tiny_kernel(
     const T *__restrict__ dy, const T *__restrict__ x,
     const float *__restrict__ stats, const uint8_t *__restrict__ mask,
     T *__restrict__ dx, SoftmaxGeom g, float scale, DropArgs d) {
   d = resolve_drop(d);
-  constexpr int K = ROWMAX / kWave / EW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const float c2 = scale * kLog2e;
-  for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < g.rows;
-       r += (int64_t)gridDim.x * 4) {
-    int64_t row;
-    int visible;
-    const uint8_t *mrow;
-    row_setup<MODE>(g, r, mask, row, visible, mrow);
-    const T *xr = x + row * g.sk;
-    const T *gr = dy + row * g.sk;
-    T *dxr = dx + row * g.sk;
-    const float m = stats[2 * row], inv = stats[2 * row + 1];
-    constexpr bool kBias = MODE == kModeBias;
-    const bool bias_f32 = g.bias_esize == 4;
-    const bool empty = inv < 0.f && !kBias;
-    float pv[K][EW], gv[K][EW];
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-#pragma unroll
-      for (int e = 0; e < EW; ++e) {
-        pv[k][e] = 0.f;
-        gv[k][e] = 0.f;
-      }
-      uint32_t hid = 0;
-      bool none = true;
-      if (i0 < g.sk) {
-        if constexpr (MODE == kModeMasked) hid = ld_mask_small<EW>(mrow + i0);
-        // keys beyond the diagonal contribute nothing and are not loaded
-        // (a row without a visible key is uniform: every key counts)
-        none = !empty && i0 >= visible;
-      }
-      if (!none) {
-        float xt[EW], gt[EW];
-        ld_small<T, EW>(xr + i0, xt);
-        ld_small<T, EW>(gr + i0, gt);
-        const uint32_t keep = keep_small<EW>(row * g.sk + i0, d);
-#pragma unroll
-        for (int e = 0; e < EW; ++e) {
-          const bool hidden =
-              MODE == kModeMasked ? (((hid >> e) & 1u) != 0 || i0 + e >= visible)
-                                  : i0 + e >= visible;
-          float p = 0.f;
-          if (empty) {
-            p = -inv;
-          } else if (!hidden) {
-            if constexpr (kBias) {
-              const float u =
-                  __builtin_fmaf(xt[e], scale, bias_at<T>(mrow, i0 + e, bias_f32));
-              p = __builtin_amdgcn_exp2f(mul_rn(sub_rn(u, m), kLog2e)) * inv;
-            } else {
-              p = __builtin_amdgcn_exp2f(sub_rn(mul_rn(xt[e], c2), m)) * inv;
-            }
-          }
-          pv[k][e] = p;
-          // (a rounded product: fused into the subtraction below it would
-          //  leave the product's rounding error where an exact zero belongs)
-          gv[k][e] = (keep >> e) & 1u ? mul_rn(gt[e], d.scale) : 0.f;
-          s += pv[k][e] * gv[k][e];
+  const int i = threadIdx.x % kTinyLanes;
+  constexpr bool kBias = MODE == kModeBias;
+  for (int64_t r0 = (int64_t)blockIdx.x * kTinyRows; r0 < g.rows;
+       r0 += (int64_t)gridDim.x * kTinyRows) {
+    const int64_t r = r0 + threadIdx.x / kTinyLanes;
+    int64_t row = 0;
+    int visible = 0;
+    const uint8_t *mrow = nullptr;
+    if (r < g.rows) row_setup<MODE>(g, r, mask, row, visible, mrow);
+    const bool in_row = r < g.rows && i < g.sk;
+    float p = 0.f, dp = 0.f;
+    if (in_row) {
+      const float m = stats[2 * row], inv = stats[2 * row + 1];
+      const bool empty = inv < 0.f && !kBias;
+      bool hidden = i >= visible;
+      if constexpr (MODE == kModeMasked)
+        if (!hidden) hidden = mrow[i] != 0;
+      if (empty) {
+        p = -inv;
+      } else if (!hidden) {
+        const float t = io<T>::from_scalar(x[row * g.sk + i]);
+        if constexpr (kBias) {
+          const float u = __builtin_fmaf(t, scale, bias_at<T>(mrow, i, g.bias_esize == 4));
+          p = __builtin_amdgcn_exp2f(mul_rn(sub_rn(u, m), kLog2e)) * inv;
+        } else {
+          p = __builtin_amdgcn_exp2f(sub_rn(mul_rn(t, scale * kLog2e), m)) * inv;
         }
       }
+      // (a rounded product: fused into the subtraction below it would leave the
+      //  product's rounding error where an exact zero belongs; keys beyond the
+      //  diagonal contribute nothing)
+      if ((empty || i < visible) && keep_element(row * g.sk + i, d))
+        dp = mul_rn(io<T>::from_scalar(dy[row * g.sk + i]), d.scale);
     }
-    s = wave_sum(s);
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-      if (i0 < g.sk) {
-        float o[EW];
-#pragma unroll
-        for (int e = 0; e < EW; ++e) o[e] = scale * (pv[k][e] * (gv[k][e] - s));
-        st_small<T, EW>(dxr + i0, o);
-      }
-    }
+    const float s = group_allreduce<OpSum, kTinyLanes>(p * dp);
+    if (in_row) dx[row * g.sk + i] = io<T>::to_scalar(scale * (p * (dp - s)));
   }
 }
 
-template <typename T, int EW, int ROWMAX>
-__global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(
+template <typename T>
+__global__ __launch_bounds__(256) void softmax_bwd_tiny_kernel(
     const T *__restrict__ dy, const T *__restrict__ y, T *__restrict__ dx,
     int64_t rows, int sk, float scale) {
-  constexpr int K = ROWMAX / kWave / EW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < rows;
-       r += (int64_t)gridDim.x * 4) {
-    const T *yr = y + r * sk;
-    const T *gr = dy + r * sk;
-    T *dxr = dx + r * sk;
-    float yv[K][EW], gv[K][EW];
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-#pragma unroll
-      for (int e = 0; e < EW; ++e) {
-        yv[k][e] = 0.f;
-        gv[k][e] = 0.f;
-      }
-      if (i0 < sk) {
-        ld_small<T, EW>(yr + i0, yv[k]);
-        ld_small<T, EW>(gr + i0, gv[k]);
-      }
-#pragma unroll
-      for (int e = 0; e < EW; ++e) s += yv[k][e] * gv[k][e];
-    }
-    s = wave_sum(s);
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int i0 = (lane + kWave * k) * EW;
-      if (i0 < sk) {
-        float o[EW];
-#pragma unroll
-        for (int e = 0; e < EW; ++e) o[e] = scale * (yv[k][e] * (gv[k][e] - s));
-        st_small<T, EW>(dxr + i0, o);
-      }
-    }
+  const int i = threadIdx.x % kTinyLanes;
+  for (int64_t r0 = (int64_t)blockIdx.x * kTinyRows; r0 < rows;
+       r0 += (int64_t)gridDim.x * kTinyRows) {
+    const int64_t row = r0 + threadIdx.x / kTinyLanes;
+    const bool in_row = row < rows && i < sk;
+    const float yv = in_row ? io<T>::from_scalar(y[row * sk + i]) : 0.f;
+    const float gv = in_row ? io<T>::from_scalar(dy[row * sk + i]) : 0.f;
+    const float s = group_allreduce<OpSum, kTinyLanes>(yv * gv);
+    if (in_row) dx[row * sk + i] = io<T>::to_scalar(scale * (yv * (gv - s)));
   }
 }
 
-// Elements per access of the wave-per-row kernels: the widest of 4, 2, 1 for
-// which the row length divides, an access stays within 8 bytes and every
-// pointer (and the mask) is aligned to the access.
-template <typename T>
-static inline int wave_row_ew(int64_t sk, const void *a, const void *b,
-                              const void *c, const uint8_t *mask) {
-  for (int ew = 4; ew > 1; ew >>= 1) {
-    const uintptr_t bytes = (uintptr_t)ew * sizeof(T);
-    if (bytes > 8 || sk % ew != 0) continue;
-    const uintptr_t all = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
-                          reinterpret_cast<uintptr_t>(c);
-    if ((all & (bytes - 1)) != 0) continue;
-    if (mask != nullptr && (reinterpret_cast<uintptr_t>(mask) & (uintptr_t)(ew - 1)) != 0) continue;
-    return ew;
-  }
-  return 1;
-}
-
-// workgroups of a wave-per-row launch (four rows each)
-static inline int64_t wave_row_grid(int64_t rows) {
-  const int64_t want = ceil_div(rows, 4);
-  const int64_t cap = (int64_t)device_cu_count() * 64;
-  return want < cap ? want : cap;
+static inline dim3 tiny_grid(int64_t rows) {
+  const int64_t want = ceil_div(rows, kTinyRows), cap = max_workgroups(256);
+  return dim3((unsigned)(want < cap ? want : cap));
 }
 
 // ---------------------------------------------------------------------------
@@ -1522,6 +1459,80 @@ static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
   while (p.rpb * p.wpr > 16) --p.rpb;
   p.ok = true;
   return p;
+}
+
+// Ragged rows: at least one chunk, at most 64 bytes of an operand per lane and
+// sixteen waves.  Rows of up to 8 and 16 chunks take as many lanes; up to 96
+// chunks a row can be held by 8, 16 or 32 lanes with three chunks each, which
+// idles fewer lanes but reads the row in pieces of 128, 256 or 512 bytes at odd
+// addresses (one line more per piece than aligned), or by one chunk per lane
+// of 32 lanes or a wave, in one piece.  `min_x3` is the smallest lane group
+// that takes three chunks: 8 where the arithmetic is what costs, i.e. with
+// dropout (bf16 180 keys, additive term: forward 118 against 190 us) and in
+// the plain forward, which adds in the order of the forward with dropout (381
+// keys: 91 against 103 us; 180 keys: 119 against 127, causal 140 against 106);
+// none in the plain backward (381 keys: 128 against 102 us; 700: 99 against 88).
+// Two rows (of waves or sets of lane groups) to a workgroup: the line that two
+// rows share is then written through one L2 (bf16 1003 keys: causal backward
+// 102 -> 88 us, dense 156 -> 130 us; four measure the same, and slower beyond
+// 2048 keys).
+static SoftmaxPlan plan_softmax_ragged(int64_t sk, int E, int min_x3) {
+  SoftmaxPlan p{0, 1, 1, 1, kWave, false};
+  if (sk < E) return p;
+  const int64_t nchunks = ceil_div(sk, E);
+  const int64_t wpr = ceil_div(nchunks, kWave * 4);
+  if (wpr > 16) return p;
+  p.ok = true;
+  p.wpr = (int)wpr;
+  p.vpl = 1;
+  if (nchunks <= 8) {
+    p.lpr = 8;
+  } else if (nchunks <= 16) {
+    p.lpr = 16;
+  } else if (nchunks <= 24 && min_x3 <= 8) {
+    p.lpr = 8;
+    p.vpl = 3;
+  } else if (nchunks <= 32) {
+    p.lpr = 32;
+  } else if (nchunks <= 48 && min_x3 <= 16) {
+    p.lpr = 16;
+    p.vpl = 3;
+  } else if (nchunks > 64 && nchunks <= 96 && min_x3 <= 32) {
+    p.lpr = 32;
+    p.vpl = 3;
+  } else {
+    p.vpl = (int)ceil_div(nchunks, kWave * wpr);
+  }
+  p.rpb = g_tune.softmax_rows_per_block > 0 ? g_tune.softmax_rows_per_block : 2;
+  while (p.rpb * p.wpr > 16) --p.rpb;
+  return p;
+}
+#define OSLO_SM_RAGGED_CASES(LAUNCH)       \
+  if (pl.lpr == 8 && pl.vpl == 1) {        \
+    LAUNCH(1, 8);                          \
+  } else if (pl.lpr == 16 && pl.vpl == 1) { \
+    LAUNCH(1, 16);                         \
+  } else if (pl.lpr == 32 && pl.vpl == 1) { \
+    LAUNCH(1, 32);                         \
+  } else if (pl.lpr == 8) {                \
+    LAUNCH(3, 8);                          \
+  } else if (pl.lpr == 16) {               \
+    LAUNCH(3, 16);                         \
+  } else if (pl.lpr == 32) {               \
+    LAUNCH(3, 32);                         \
+  } else if (pl.vpl == 1) {                \
+    LAUNCH(1, kWave);                      \
+  } else if (pl.vpl == 2) {                \
+    LAUNCH(2, kWave);                      \
+  } else if (pl.vpl == 3) {                \
+    LAUNCH(3, kWave);                      \
+  } else {                                 \
+    LAUNCH(4, kWave);                      \
+  }
+// LDS of a ragged launch with dropout: the keep bits of the workgroup's rows
+static inline unsigned ragged_keep_lds(const SoftmaxPlan &pl) {
+  const int lanes = pl.lpr == kWave ? kWave * pl.wpr : pl.lpr;
+  return (unsigned)(pl.rpb * (kWave / pl.lpr) * keep_bytes(lanes, pl.vpl));
 }
 
 constexpr int kFwdMaxElems = 64;  // one operand resident
@@ -1634,37 +1645,22 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
                       (MODE != kModeMasked ||
                        (reinterpret_cast<uintptr_t>(mask) % E) == 0) &&
                       (MODE != kModeBias || bias_vec_ok(g, mask));
-  if (!vec_ok) {
+  const bool ragged = !vec_ok;
+  if (ragged) pl = plan_softmax_ragged(g.sk, E, 8);
+  if (ragged && g.sk < E) {
+    const dim3 grid = tiny_grid(g.rows);
+    if (drop)
+      softmax_fwd_tiny_kernel<T, MODE, true><<<grid, 256, 0, st>>>((const T *)x, mask, (T *)y,
+                                                                   stats, g, scale, d);
+    else
+      softmax_fwd_tiny_kernel<T, MODE, false><<<grid, 256, 0, st>>>((const T *)x, mask, (T *)y,
+                                                                    nullptr, g, scale, d);
+    return check_launch("softmax_fwd_tiny_kernel");
+  }
+  if (!pl.ok) {
     const int64_t grid = g.rows < (int64_t)device_cu_count() * 32
                              ? g.rows
                              : (int64_t)device_cu_count() * 32;
-    if (g.sk <= kWaveRowMax) {
-      const dim3 wgrid((unsigned)wave_row_grid(g.rows));
-      const int ew = wave_row_ew<T>(g.sk, x, y, nullptr, MODE == kModeMasked ? mask : nullptr);
-#define OSLO_SM_WAVE_FWD_R(EW_, RM_)                                       \
-  do {                                                                     \
-    if constexpr (EW_ * sizeof(T) <= 8) {                                  \
-      if (drop)                                                            \
-        softmax_fwd_wave_kernel<T, MODE, true, EW_, RM_><<<wgrid, 256, 0, st>>>(  \
-            (const T *)x, mask, (T *)y, stats, g, scale, d);               \
-      else                                                                 \
-        softmax_fwd_wave_kernel<T, MODE, false, EW_, RM_><<<wgrid, 256, 0, st>>>( \
-            (const T *)x, mask, (T *)y, nullptr, g, scale, d);             \
-    }                                                                      \
-  } while (0)
-#define OSLO_SM_WAVE_FWD(EW_)                                              \
-  do {                                                                     \
-    if (g.sk <= 256) OSLO_SM_WAVE_FWD_R(EW_, 256);                         \
-    else if (g.sk <= 1024) OSLO_SM_WAVE_FWD_R(EW_, 1024);                  \
-    else OSLO_SM_WAVE_FWD_R(EW_, 2048);                                    \
-  } while (0)
-      if (ew == 4) OSLO_SM_WAVE_FWD(4);
-      else if (ew == 2) OSLO_SM_WAVE_FWD(2);
-      else OSLO_SM_WAVE_FWD(1);
-#undef OSLO_SM_WAVE_FWD
-#undef OSLO_SM_WAVE_FWD_R
-      return check_launch("softmax_fwd_wave_kernel");
-    }
     if (drop)
       softmax_fwd_generic_kernel<T, MODE, true>
           <<<dim3((unsigned)grid), 256, 0, st>>>((const T *)x, mask, (T *)y,
@@ -1695,6 +1691,17 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
               (const T *)x, mask, (T *)y, nullptr, g, scale, d);     \
   } else                                                             \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax fwd: no kernel for %d x %d chunks per lane", VPL, RPW)
+#define OSLO_SM_FWD_RAGGED(VPL, LPR_)                                \
+  do {                                                               \
+    if (drop)                                                        \
+      softmax_fwd_kernel<T, VPL, 1, MODE, true, LPR_, true>          \
+          <<<dim3((unsigned)grid), threads, ragged_keep_lds(pl), st>>>( \
+              (const T *)x, mask, (T *)y, stats, g, scale, d);       \
+    else                                                             \
+      softmax_fwd_kernel<T, VPL, 1, MODE, false, LPR_, true>         \
+          <<<dim3((unsigned)grid), threads, 0, st>>>(                \
+              (const T *)x, mask, (T *)y, nullptr, g, scale, d);     \
+  } while (0)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
   int64_t launch_blocks = nblocks;
   if (MODE == kModeBias && g.batch_inner && g_tune.softmax_bias_order == 3 &&
@@ -1704,11 +1711,16 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   }
   for (g.blk0 = 0; g.blk0 < launch_blocks; g.blk0 += per_launch) {
     const int64_t grid = launch_blocks - g.blk0 < per_launch ? launch_blocks - g.blk0 : per_launch;
-    OSLO_SM_CASES(OSLO_SM_FWD)
+    if (ragged) {
+      OSLO_SM_RAGGED_CASES(OSLO_SM_FWD_RAGGED)
+    } else {
+      OSLO_SM_CASES(OSLO_SM_FWD)
+    }
     const int rc = check_launch("softmax_fwd_kernel");
     if (rc != OSLO_OK) return rc;
   }
 #undef OSLO_SM_FWD
+#undef OSLO_SM_FWD_RAGGED
   return OSLO_OK;
 }
 
@@ -1726,32 +1738,17 @@ int launch_softmax_bwd(const void *dy, const void *y,
                       (MODE != kModeMasked ||
                        (reinterpret_cast<uintptr_t>(mask) % E) == 0) &&
                       (MODE != kModeBias || bias_vec_ok(g, mask));
-  if (!vec_ok) {
+  const bool ragged = !vec_ok;
+  if (ragged) pl = plan_softmax_ragged(g.sk, E, kWave);
+  if (ragged && g.sk < E) {
+    softmax_bwd_tiny_kernel<T><<<tiny_grid(g.rows), 256, 0, st>>>(
+        (const T *)dy, (const T *)y, (T *)dx, g.rows, g.sk, scale);
+    return check_launch("softmax_bwd_tiny_kernel");
+  }
+  if (!pl.ok) {
     const int64_t grid = g.rows < (int64_t)device_cu_count() * 32
                              ? g.rows
                              : (int64_t)device_cu_count() * 32;
-    if (g.sk <= kWaveRowMax) {
-      const dim3 wgrid((unsigned)wave_row_grid(g.rows));
-      const int ew = wave_row_ew<T>(g.sk, dy, y, dx, nullptr);
-#define OSLO_SM_WAVE_BWD_R(EW_, RM_)                                       \
-  do {                                                                     \
-    if constexpr (EW_ * sizeof(T) <= 8)                                    \
-      softmax_bwd_wave_kernel<T, EW_, RM_><<<wgrid, 256, 0, st>>>(         \
-          (const T *)dy, (const T *)y, (T *)dx, g.rows, g.sk, scale);      \
-  } while (0)
-#define OSLO_SM_WAVE_BWD(EW_)                                              \
-  do {                                                                     \
-    if (g.sk <= 256) OSLO_SM_WAVE_BWD_R(EW_, 256);                         \
-    else if (g.sk <= 1024) OSLO_SM_WAVE_BWD_R(EW_, 1024);                  \
-    else OSLO_SM_WAVE_BWD_R(EW_, 2048);                                    \
-  } while (0)
-      if (ew == 4) OSLO_SM_WAVE_BWD(4);
-      else if (ew == 2) OSLO_SM_WAVE_BWD(2);
-      else OSLO_SM_WAVE_BWD(1);
-#undef OSLO_SM_WAVE_BWD
-#undef OSLO_SM_WAVE_BWD_R
-      return check_launch("softmax_bwd_wave_kernel");
-    }
     softmax_bwd_generic_kernel<T><<<dim3((unsigned)grid), 256, 0, st>>>(
         (const T *)dy, (const T *)y, (T *)dx, g.rows, g.sk, scale);
     return check_launch("softmax_bwd_generic_kernel");
@@ -1771,13 +1768,25 @@ int launch_softmax_bwd(const void *dy, const void *y,
             (const T *)dy, (const T *)y, mask, (T *)dx, g, scale); \
   else                                                     \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
+#define OSLO_SM_BWD_RAGGED(VPL, LPR_)                      \
+  if constexpr (VPL == 1 || LPR_ == kWave)                 \
+    softmax_bwd_kernel<T, VPL, 1, MODE, LPR_, true>        \
+        <<<dim3((unsigned)grid), threads, 0, st>>>(        \
+            (const T *)dy, (const T *)y, mask, (T *)dx, g, scale); \
+  else                                                     \
+    return fail(OSLO_ERR_UNSUPPORTED, "softmax bwd: no kernel for %d chunks in %d lanes", VPL, LPR_)
   for (g.blk0 = 0; g.blk0 < nblocks; g.blk0 += per_launch) {
     const int64_t grid = nblocks - g.blk0 < per_launch ? nblocks - g.blk0 : per_launch;
-    OSLO_SM_CASES(OSLO_SM_BWD)
+    if (ragged) {
+      OSLO_SM_RAGGED_CASES(OSLO_SM_BWD_RAGGED)
+    } else {
+      OSLO_SM_CASES(OSLO_SM_BWD)
+    }
     const int rc = check_launch("softmax_bwd_kernel");
     if (rc != OSLO_OK) return rc;
   }
 #undef OSLO_SM_BWD
+#undef OSLO_SM_BWD_RAGGED
   return OSLO_OK;
 }
 
@@ -1798,32 +1807,17 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
                       (MODE != kModeMasked ||
                        (reinterpret_cast<uintptr_t>(mask) % E) == 0) &&
                       (MODE != kModeBias || bias_vec_ok(g, mask));
-  if (!vec_ok) {
+  const bool ragged = !vec_ok;
+  if (ragged) pl = plan_softmax_ragged(g.sk, E, 8);
+  if (ragged && g.sk < E) {
+    softmax_dropout_bwd_tiny_kernel<T, MODE><<<tiny_grid(g.rows), 256, 0, st>>>(
+        (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d);
+    return check_launch("softmax_dropout_bwd_tiny_kernel");
+  }
+  if (!pl.ok) {
     const int64_t grid = g.rows < (int64_t)device_cu_count() * 32
                              ? g.rows
                              : (int64_t)device_cu_count() * 32;
-    if (g.sk <= kWaveRowMax) {
-      const dim3 wgrid((unsigned)wave_row_grid(g.rows));
-      const int ew = wave_row_ew<T>(g.sk, dy, x, dx, MODE == kModeMasked ? mask : nullptr);
-#define OSLO_SM_WAVE_DBWD_R(EW_, RM_)                                      \
-  do {                                                                     \
-    if constexpr (EW_ * sizeof(T) <= 8)                                    \
-      softmax_dropout_bwd_wave_kernel<T, MODE, EW_, RM_><<<wgrid, 256, 0, st>>>( \
-          (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d); \
-  } while (0)
-#define OSLO_SM_WAVE_DBWD(EW_)                                             \
-  do {                                                                     \
-    if (g.sk <= 256) OSLO_SM_WAVE_DBWD_R(EW_, 256);                        \
-    else if (g.sk <= 1024) OSLO_SM_WAVE_DBWD_R(EW_, 1024);                 \
-    else OSLO_SM_WAVE_DBWD_R(EW_, 2048);                                   \
-  } while (0)
-      if (ew == 4) OSLO_SM_WAVE_DBWD(4);
-      else if (ew == 2) OSLO_SM_WAVE_DBWD(2);
-      else OSLO_SM_WAVE_DBWD(1);
-#undef OSLO_SM_WAVE_DBWD
-#undef OSLO_SM_WAVE_DBWD_R
-      return check_launch("softmax_dropout_bwd_wave_kernel");
-    }
     softmax_dropout_bwd_generic_kernel<T, MODE>
         <<<dim3((unsigned)grid), 256, 0, st>>>((const T *)dy, (const T *)x,
                                                stats, mask, (T *)dx, g, scale,
@@ -1846,6 +1840,10 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
             scale, d);                                              \
   else                                                              \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax dropout bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
+#define OSLO_SM_DBWD_RAGGED(VPL, LPR_)                              \
+  softmax_dropout_bwd_kernel<T, VPL, 1, MODE, LPR_, true>           \
+      <<<dim3((unsigned)grid), threads, ragged_keep_lds(pl), st>>>( \
+          (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
   int64_t launch_blocks = nblocks;
   if (MODE == kModeBias && g.batch_inner && g_tune.softmax_bias_order == 3 &&
@@ -1855,11 +1853,16 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
   }
   for (g.blk0 = 0; g.blk0 < launch_blocks; g.blk0 += per_launch) {
     const int64_t grid = launch_blocks - g.blk0 < per_launch ? launch_blocks - g.blk0 : per_launch;
-    OSLO_SM_CASES(OSLO_SM_DBWD)
+    if (ragged) {
+      OSLO_SM_RAGGED_CASES(OSLO_SM_DBWD_RAGGED)
+    } else {
+      OSLO_SM_CASES(OSLO_SM_DBWD)
+    }
     const int rc = check_launch("softmax_dropout_bwd_kernel");
     if (rc != OSLO_OK) return rc;
   }
 #undef OSLO_SM_DBWD
+#undef OSLO_SM_DBWD_RAGGED
   return OSLO_OK;
 }
 
