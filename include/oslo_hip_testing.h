@@ -62,7 +62,9 @@ int oslo_wave_reduce_selftest(float *out4, void *stream);
  * oslo_colsum_finalize_probe), "colsum_slices" (slices of the partial rows
  * that a workgroup of the column-sum reduction adds side by side: 64 or 128,
  * the default, with eight lanes per slice and 32 columns per workgroup, or
- * 256 with four lanes per slice and 16 columns);
+ * 256 with four lanes per slice and 16 columns), "softmax_waves_per_cu" (waves
+ * of a softmax launch kept on a compute unit, 1..32; by default from the bytes
+ * that a wave requests);
  * value 0 restores the default.  Other values must be ones the launch code
  * has a kernel build and a valid workgroup shape for, else
  * OSLO_ERR_INVALID_ARGUMENT: chunks per lane (*_vpl: 1, 2, 4, forward also 8,

@@ -51,6 +51,7 @@ struct Tuning {
   int softmax_causal_order;
   int softmax_bias_group;
   int colsum_slices;
+  int softmax_waves_per_cu;
 };
 // oslo_tune() writes a process-wide table under a lock; every entry point
 // copies that table into a per-thread snapshot before it plans a launch

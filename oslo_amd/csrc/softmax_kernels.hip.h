@@ -159,46 +159,57 @@ __device__ __forceinline__ float row_reduce_max(float a, float *red, int wave,
   return a;
 }
 
-// Mask bytes of one chunk -> bit e set when key e of the chunk is masked out.
-template <int E, bool ANY>
-__device__ __forceinline__ uint32_t load_mask_bits(const uint8_t *p) {
-  uint32_t bits = 0;
-  if constexpr (E == 8) {
-    u32x2 m;
-    if constexpr (ANY)
-      m = *reinterpret_cast<const u32x2_any *>(p);
-    else
-      m = *reinterpret_cast<const u32x2 *>(p);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      bits |= ((m.x >> (8 * e)) & 0xffu) ? (1u << e) : 0u;
-      bits |= ((m.y >> (8 * e)) & 0xffu) ? (1u << (4 + e)) : 0u;
+// Mask bytes of one chunk as loaded, and their bits: bit e set when key e of
+// the chunk is masked out.  (In two steps, like every operand of these
+// kernels: all loads of a row are requested before any is converted.  A
+// conversion next to its load, inside the branch that decides about the load,
+// makes the wave wait for one chunk before it requests the next.)
+template <int E, bool ANY> struct MaskChunk {
+  uint32_t w[E / 4];
+  __device__ __forceinline__ void load(const uint8_t *p) {
+    if constexpr (E == 8) {
+      u32x2 m;
+      if constexpr (ANY)
+        m = *reinterpret_cast<const u32x2_any *>(p);
+      else
+        m = *reinterpret_cast<const u32x2 *>(p);
+      w[0] = m.x;
+      w[1] = m.y;
+    } else {
+      if constexpr (ANY)
+        w[0] = *reinterpret_cast<const u32_any *>(p);
+      else
+        w[0] = *reinterpret_cast<const uint32_t *>(p);
     }
-  } else {
-    uint32_t m;
-    if constexpr (ANY)
-      m = *reinterpret_cast<const u32_any *>(p);
-    else
-      m = *reinterpret_cast<const uint32_t *>(p);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      bits |= ((m >> (8 * e)) & 0xffu) ? (1u << e) : 0u;
   }
-  return bits;
-}
+  // bit 7 of every byte that is not zero
+  static __device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v) {
+    return (((v & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v) & 0x80808080u;
+  }
+  // (the flags of four bytes at a time, then gathered: 14 instructions where
+  //  testing the eight bytes one by one takes 24)
+  __device__ __forceinline__ uint32_t bits() const {
+    uint32_t x = nonzero_bytes(w[0]) >> 7;
+    if constexpr (E == 8) x |= nonzero_bytes(w[1]) >> 3;
+    x |= (x >> 7) | (x >> 14) | (x >> 21);
+    return x & ((1u << E) - 1u);
+  }
+};
 
-// Mask bits of the chunk of keys i0 .. i0 + E of a row that sees `visible` keys
-// through the diagonal: the keys from `visible` on are hidden as well.  Chunks
-// that lie beyond the diagonal altogether do not read their mask bytes.
-template <int E, bool ANY>
-__device__ __forceinline__ uint32_t masked_chunk_bits(const uint8_t *mrow, int i0,
-                                                      int visible) {
+// All outstanding vector loads have arrived.  The kernels say so once, between
+// the loads of a row and their use (and, where they have to look at mask bytes or
+// terms before they know which logits to request, between the two): the
+// compiler otherwise carries a load inside a branch as possibly outstanding
+// through all later branches and waits again in front of each, by then for the
+// loads or the stores in between.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
+// Bits of the keys i0 .. i0 + E that lie at or beyond `visible`.
+template <int E>
+__device__ __forceinline__ uint32_t beyond_bits(int i0, int visible) {
   constexpr uint32_t kAllBits = (1u << E) - 1u;
   const int left = visible - i0;  // keys of the chunk below the diagonal
-  if (left <= 0) return kAllBits;
-  uint32_t mb = load_mask_bits<E, ANY>(mrow + i0);
-  if (left < E) mb |= kAllBits & ~((1u << left) - 1u);
-  return mb;
+  return left >= E ? 0u : (left <= 0 ? kAllBits : kAllBits & ~((1u << left) - 1u));
 }
 
 // Row bookkeeping shared by forward and backward.  Rows are numbered so that
@@ -265,22 +276,8 @@ __device__ __forceinline__ void row_setup(const SoftmaxGeom &g, int64_t r,
 }
 
 // One chunk of the additive term, E values of the logits' type T or of float
-// (a launch-uniform choice, so one kernel serves both), converted to float as
-// soon as it arrives: the float form is no wider than a float chunk as loaded.
-template <typename T, int E, bool ANY>
-__device__ __forceinline__ void load_bias_chunk(const uint8_t *row, int i0, bool f32, float *f) {
-  if (sizeof(T) == 4 || f32) {
-#pragma unroll
-    for (int v = 0; v < E / 4; ++v)
-      io<float>::unpack(ld16_cached_at<ANY>(row + ((int64_t)i0 + 4 * v) * 4), f + 4 * v);
-  } else {
-    io<T>::unpack(ld16_cached_at<ANY>(row + (int64_t)i0 * (int64_t)sizeof(T)), f);
-  }
-}
-
-// The same in two steps, for code that issues all its loads before it
-// converts any of them: the chunk as loaded (E / 4 vectors, the first one only
-// for a 16-bit term), then its conversion.
+// (a launch-uniform choice, so one kernel serves both): as loaded (E / 4
+// vectors, the first one only for a 16-bit term), then its conversion.
 template <typename T, int E, bool ANY>
 __device__ __forceinline__ void load_bias_raw(const uint8_t *row, int i0, bool f32, u32x4 *r) {
   if (sizeof(T) == 4 || f32) {
@@ -425,14 +422,15 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
   // gets zeros (its neighbours in the wave may well see keys, so the
   // wave-uniform shortcuts below do not catch it)
   bool nokey[RPW];
-  int vis[RAG ? RPW : 1];  // keys below the diagonal
-  const uint8_t *mrow0 = nullptr;
+  int vis[RPW];  // keys below the diagonal
+  const uint8_t *mrows[RPW];
+  bool shared[RPW];  // the row's mask bits are those of the wave's first row
+  MaskChunk<E, RAG> mraw[MODE == kModeMasked ? RPW : 1][MODE == kModeMasked ? VPL : 1];
   // additive term (kModeBias): the chunks as loaded, and whether a chunk's
   // logits were left unread
   constexpr bool kBias = MODE == kModeBias;
-  float bv[kBias ? RPW : 1][kBias ? VPL : 1][kBias ? E : 1];
   u32x4 braw[kBias ? RPW : 1][kBias ? VPL : 1][kBias ? E / 4 : 1];
-  RawChunk<T, E> xraw[kBias ? RPW : 1][kBias ? VPL : 1];
+  RawChunk<T, E> xraw[RPW][VPL];
   bool bhid[kBias ? RPW : 1][kBias ? VPL : 1];
   const bool bias_f32 = g.bias_esize == 4;
 
@@ -440,43 +438,45 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
   for (int j = 0; j < RPW; ++j) {
     const int64_t r = rbase + j * SUB;
     rvalid[j] = r < g.rows;
-    int visible = 0;
-    const uint8_t *mrow = nullptr;
+    vis[j] = 0;
+    mrows[j] = nullptr;
     row[j] = 0;
-    if (rvalid[j]) row_setup<MODE>(g, r, mask, row[j], visible, mrow);
-    nokey[j] = MODE == kModeBias && rvalid[j] && visible <= 0;
-    if constexpr (RAG) vis[j] = visible;
+    if (rvalid[j]) row_setup<MODE>(g, r, mask, row[j], vis[j], mrows[j]);
+    nokey[j] = MODE == kModeBias && rvalid[j] && vis[j] <= 0;
     // consecutive rows of a wave normally share their mask row (a key-padding
     // mask [b, 1, 1, sk]): its bits are then read and unpacked once
-    bool shared = false;
-    if constexpr (MODE == kModeMasked && RPW > 1) {
-      if (j == 0) mrow0 = mrow;
-      shared = j > 0 && rvalid[j] && rvalid[0] && mrow == mrow0 && !g.causal;
+    shared[j] = false;
+    if constexpr (MODE == kModeMasked && RPW > 1)
+      shared[j] = j > 0 && rvalid[j] && rvalid[0] && mrows[j] == mrows[0] && !g.causal;
+    if constexpr (MODE == kModeMasked) {
+      // (chunks beyond the diagonal do not read their mask bytes)
+#pragma unroll
+      for (int k = 0; k < VPL; ++k) {
+        const int c = c0 + k * cstride;
+        const int i0 = chunk_key<E, RAG>(c, g.sk);
+        if (!shared[j] && rvalid[j] && c < nchunks && i0 < vis[j]) mraw[j][k].load(mrows[j] + i0);
+      }
     }
+  }
+  if constexpr (MODE == kModeMasked) wait_loads();
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
-      uint32_t mb = (1u << E) - 1u;
-      if (shared) {
-        mb = mbits[0][k];
-      } else if (rvalid[j] && c < nchunks) {
-        if constexpr (MODE == kModeCausal || MODE == kModeBias) {
-          // (visible == sk without a diagonal)
-          const int left = visible - chunk_key<E, RAG>(c, g.sk);  // visible keys in this chunk
-          mb = left >= E ? 0u : (left <= 0 ? mb : (mb & ~((1u << left) - 1u)));
-        } else {
-          mb = masked_chunk_bits<E, RAG>(mrow, chunk_key<E, RAG>(c, g.sk), visible);
-        }
+      const int i0 = chunk_key<E, RAG>(c, g.sk);
+      uint32_t mb = kAll;
+      if (rvalid[j] && c < nchunks) {
+        mb = beyond_bits<E>(i0, vis[j]);  // (vis == sk without a diagonal)
+        if constexpr (MODE == kModeMasked)
+          if (mb != kAll) mb |= shared[j] ? mbits[0][k] : mraw[j][k].bits();
       }
       mbits[j][k] = mb;
       if constexpr (MODE == kModeBias) {
         // the additive term of every chunk that has a key below the diagonal
         // (cached loads: its rows are normally shared by many rows of logits)
-        // (all of them requested before any is converted: a conversion
-        //  waits for its load)
         bhid[j][k] = false;
-        if (mb != kAll)
-          load_bias_raw<T, E, RAG>(mrow, chunk_key<E, RAG>(c, g.sk), bias_f32, braw[j][k]);
+        if (mb != kAll) load_bias_raw<T, E, RAG>(mrows[j], i0, bias_f32, braw[j][k]);
       }
     }
   }
@@ -484,13 +484,15 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     // a chunk whose terms all absorb their logits takes the terms as its
     // sums: the logits are not read
     if (g.bias_skip) {
+      wait_loads();
 #pragma unroll
       for (int j = 0; j < RPW; ++j)
 #pragma unroll
         for (int k = 0; k < VPL; ++k)
           if (mbits[j][k] != kAll) {
-            unpack_bias_raw<T, E>(braw[j][k], bias_f32, bv[j][k]);
-            bhid[j][k] = bias_all_hidden<E>(bv[j][k]);
+            float bf[E];
+            unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
+            bhid[j][k] = bias_all_hidden<E>(bf);
           }
     }
   }
@@ -502,31 +504,11 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
       const int c = c0 + k * cstride;
       // (a chunk without a visible key is not loaded; its registers are never
       //  used: every select below takes the masked branch for it)
-      bool want = mbits[j][k] != (1u << E) - 1u;
-      if constexpr (MODE == kModeBias) {
-        if (want && !bhid[j][k]) xraw[j][k].template load<RAG>(xr + chunk_key<E, RAG>(c, g.sk));
-      } else {
-        if (want) load_chunk<T, E, true, RAG>(xr + chunk_key<E, RAG>(c, g.sk), v[j][k]);
-      }
+      bool want = mbits[j][k] != kAll;
+      if constexpr (MODE == kModeBias) want = want && !bhid[j][k];
+      if (want) xraw[j][k].template load<RAG>(xr + chunk_key<E, RAG>(c, g.sk));
     }
   }
-  if constexpr (MODE == kModeBias) {
-    // (without the test above the logits were requested together with the
-    //  terms: the terms are converted only now)
-    if (!g.bias_skip) {
-#pragma unroll
-      for (int j = 0; j < RPW; ++j)
-#pragma unroll
-        for (int k = 0; k < VPL; ++k)
-          if (mbits[j][k] != kAll) unpack_bias_raw<T, E>(braw[j][k], bias_f32, bv[j][k]);
-    }
-#pragma unroll
-    for (int j = 0; j < RPW; ++j)
-#pragma unroll
-      for (int k = 0; k < VPL; ++k)
-        if (mbits[j][k] != kAll && !bhid[j][k]) xraw[j][k].unpack(v[j][k]);
-  }
-
   // (the draws of a ragged row wait in LDS while its loads are in flight)
   uint8_t *kb = nullptr;
   if constexpr (RAG && DROP) {
@@ -534,6 +516,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
                    keep_bytes(LPR == kWave ? kWave * g.wpr : LPR, VPL);
     if (rvalid[0]) draw_row_groups<E>(kb, row[0], g.sk, vis[0], c0, cstride, d);
   }
+  if constexpr (VPL * RPW > 1) wait_loads();
 
   // Wave-uniform shortcuts: where no lane of the wave sees a key of chunk
   // slot (j, k) the arithmetic is skipped altogether; where every lane sees
@@ -566,7 +549,11 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         // the sum scale * x + term as one fused multiply-add, kept in the
         // natural domain: a large negative term (-10000) then costs the logit
         // one rounding, as in a float evaluation of the unfused chain
-        const float *bf = bv[j][k];
+        // (the terms are converted here, a slot at a time: kept converted next to
+        //  the logits they cost a wave per SIMD)
+        float bf[E];
+        unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
+        xraw[j][k].unpack(v[j][k]);
         // (wave-uniform: no lane of the wave left the logits of this slot unread)
         const bool no_skip = __builtin_amdgcn_ballot_w64(bhid[j][k]) == 0;
         if (DROP && no_skip && all_visible[j][k]) {
@@ -592,6 +579,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         }
         continue;
       }
+      xraw[j][k].unpack(v[j][k]);
       if (all_visible[j][k]) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -783,52 +771,68 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
   int64_t row[RPW];
   bool rvalid[RPW];
   float rmax[RPW], rinv[RPW];
-  int vis[RAG ? RPW : 1];  // keys that count below the diagonal
+  int vis[RPW];  // keys that count below the diagonal
+  const uint8_t *mrows[RPW];
+  MaskChunk<E, RAG> mraw[MODE == kModeMasked ? RPW : 1][MODE == kModeMasked ? VPL : 1];
+  RawChunk<T, E> xraw[RPW][VPL], graw[RPW][VPL];
   constexpr bool kBias = MODE == kModeBias;
-  float bv[kBias ? RPW : 1][kBias ? VPL : 1][kBias ? E : 1];
+  u32x4 braw[kBias ? RPW : 1][kBias ? VPL : 1][kBias ? E / 4 : 1];
   const bool bias_f32 = g.bias_esize == 4;
 
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
     const int64_t r = rbase + j * SUB;
     rvalid[j] = r < g.rows;
-    int visible = 0;
-    const uint8_t *mrow = nullptr;
+    vis[j] = 0;
+    mrows[j] = nullptr;
     row[j] = 0;
     rmax[j] = 0.f;
     rinv[j] = 0.f;
     if (rvalid[j]) {
-      row_setup<MODE>(g, r, mask, row[j], visible, mrow);
+      row_setup<MODE>(g, r, mask, row[j], vis[j], mrows[j]);
       rmax[j] = stats[2 * row[j]];
       rinv[j] = stats[2 * row[j] + 1];
     }
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const int c = c0 + k * cstride;
+      const int i0 = chunk_key<E, RAG>(c, g.sk);
+      const bool want = rvalid[j] && c < nchunks && i0 < vis[j];
+      if constexpr (MODE == kModeMasked) {
+        if (want) mraw[j][k].load(mrows[j] + i0);
+      }
+      if constexpr (kBias) {
+        if (want) load_bias_raw<T, E, RAG>(mrows[j], i0, bias_f32, braw[j][k]);
+      }
+    }
+  }
+  if constexpr (MODE == kModeMasked) wait_loads();
+  if constexpr (kBias)
+    if (g.bias_skip) wait_loads();
+#pragma unroll
+  for (int j = 0; j < RPW; ++j) {
     // uniform row: every key counts (with an additive term there is no such
     // convention: the probabilities are what the arithmetic gives)
     const bool empty = rinv[j] < 0.f && !kBias;
-    if constexpr (RAG) vis[j] = empty ? g.sk : visible;
+    if (empty) vis[j] = g.sk;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
       const int i0 = chunk_key<E, RAG>(c, g.sk);
       uint32_t mb = kAll;
       if (rvalid[j] && c < nchunks) {
-        if (empty) {
-          mb = 0u;
-        } else if constexpr (MODE == kModeCausal || MODE == kModeBias) {
-          const int left = visible - i0;
-          mb = left >= E ? 0u : (left <= 0 ? mb : (mb & ~((1u << left) - 1u)));
-        } else {
-          mb = masked_chunk_bits<E, RAG>(mrow, i0, visible);
-        }
+        mb = beyond_bits<E>(i0, vis[j]);
+        if constexpr (MODE == kModeMasked)
+          if (mb != kAll && !empty) mb |= mraw[j][k].bits();
       }
       if constexpr (kBias) {
-        if (mb != kAll) {
-          load_bias_chunk<T, E, RAG>(mrow, i0, bias_f32, bv[j][k]);
-          // A chunk whose terms all absorb their logits has probability 0
-          // throughout, unless the row's maximum is such a term itself (a
-          // row without any other key): skip it altogether
-          if (g.bias_skip && rmax[j] > kBiasHidden && bias_all_hidden<E>(bv[j][k]))
-            mb = kAll;
+        // A chunk whose terms all absorb their logits has probability 0
+        // throughout, unless the row's maximum is such a term itself (a
+        // row without any other key): skip it altogether
+        if (g.bias_skip && mb != kAll) {
+          float bf[E];
+          unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
+          if (rmax[j] > kBiasHidden && bias_all_hidden<E>(bf)) mb = kAll;
         }
       }
       mbits[j][k] = mb;
@@ -840,16 +844,13 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     const T *gr = dy + row[j] * g.sk;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
-      const int c = c0 + k * cstride;
+      const int i0 = chunk_key<E, RAG>(c0 + k * cstride, g.sk);
+      // (a chunk without a visible key is not loaded: its gradients are zeros
+      //  whatever the draw says, its logits are never used)
+      graw[j][k].zero();
       if (mbits[j][k] != kAll) {
-        load_chunk<T, E, true, RAG>(xr + chunk_key<E, RAG>(c, g.sk), yv[j][k]);
-        load_chunk<T, E, true, RAG>(gr + chunk_key<E, RAG>(c, g.sk), gv[j][k]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          yv[j][k][e] = 0.f;
-          gv[j][k][e] = 0.f;
-        }
+        xraw[j][k].template load<RAG>(xr + i0);
+        graw[j][k].template load<RAG>(gr + i0);
       }
     }
   }
@@ -861,6 +862,7 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     if (rvalid[0]) draw_row_groups<E>(kb, row[0], g.sk, vis[0], c0, cstride, d);
     row_draws_done(g.wpr);
   }
+  if constexpr (VPL * RPW > 1) wait_loads();
   bool none_loaded[RPW][VPL];
 #pragma unroll
   for (int j = 0; j < RPW; ++j)
@@ -877,8 +879,6 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
     for (int k = 0; k < VPL; ++k) {
       if (none_loaded[j][k]) continue;
       const int c = c0 + k * cstride;
-      // (a chunk without a visible key was not loaded: its gradients are zeros
-      //  whatever the draw says)
       KeepWords<E> keep;
       uint32_t keep_bits = 0;
       int dup = 0;
@@ -888,8 +888,10 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
       } else {
         keep = chunk_keep_words<E>(row[j], g.sk, c, d);
       }
-      const float *bf = nullptr;
-      if constexpr (kBias) bf = bv[j][k];
+      float bf[kBias ? E : 1];
+      if constexpr (kBias) unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
+      xraw[j][k].unpack(yv[j][k]);
+      graw[j][k].unpack(gv[j][k]);
       // (the selects below stay per element: a wave-uniform branch around
       //  them for slots in which every lane sees all its keys measured 12 %
       //  slower at [256, 2048, 2048], 690 -> 772 us)
@@ -977,6 +979,10 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
   bool skip[RPW][VPL];
   int64_t row[RPW];
   bool rvalid[RPW];
+  constexpr bool kBias = MODE == kModeBias;
+  MaskChunk<E, RAG> mraw[MODE == kModeMasked ? VPL : 1];
+  u32x4 braw[kBias ? VPL : 1][kBias ? E / 4 : 1];
+  RawChunk<T, E> yraw[RPW][VPL], graw[RPW][VPL];
 
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
@@ -991,28 +997,33 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     for (int k = 0; k < VPL; ++k) {
       const int c = c0 + k * cstride;
       const int i0 = chunk_key<E, RAG>(c, g.sk);
-      bool sk_ = true;
-      if (rvalid[j] && c < nchunks) {
-        if constexpr (MODE == kModeCausal) {
-          sk_ = visible - i0 <= 0;
-        } else if constexpr (MODE == kModeMasked) {
-          sk_ = masked_chunk_bits<E, RAG>(mrow, i0, visible) == kAll;
-        } else if constexpr (MODE == kModeBias) {
-          // beyond the diagonal, or every additive term of the chunk absorbs
-          // its logit: the probabilities are zeros (unless the whole row is
-          // like that, which the test below catches)
-          sk_ = visible - i0 <= 0;
-          if (!sk_) {
-            float bf[E];
-            load_bias_chunk<T, E, RAG>(mrow, i0, g.bias_esize == 4, bf);
-            sk_ = bias_all_hidden<E>(bf);
-          }
-        } else {
-          sk_ = false;
+      const bool want = rvalid[j] && c < nchunks && (MODE == kModeDense || i0 < visible);
+      skip[j][k] = !want;
+      if constexpr (MODE == kModeMasked) {
+        if (want) mraw[k].load(mrow + i0);
+      }
+      if constexpr (kBias) {
+        if (want) load_bias_raw<T, E, RAG>(mrow, i0, g.bias_esize == 4, braw[k]);
+      }
+    }
+    if constexpr (MODE == kModeMasked || kBias) wait_loads();
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      if constexpr (MODE == kModeMasked) {
+        const int i0 = chunk_key<E, RAG>(c0 + k * cstride, g.sk);
+        if (!skip[j][k]) skip[j][k] = (mraw[k].bits() | beyond_bits<E>(i0, visible)) == kAll;
+      }
+      if constexpr (kBias) {
+        // every additive term of the chunk absorbs its logit: the
+        // probabilities are zeros (unless the whole row is like that, which
+        // the test below catches)
+        if (!skip[j][k]) {
+          float bf[E];
+          unpack_bias_raw<T, E>(braw[k], g.bias_esize == 4, bf);
+          skip[j][k] = bias_all_hidden<E>(bf);
         }
       }
-      skip[j][k] = sk_;
-      if (!sk_) anyvis = 1.f;
+      if (!skip[j][k]) anyvis = 1.f;
     }
     if constexpr (MODE != kModeDense) {
       // a row with no visible key holds the uniform distribution: read it all
@@ -1031,19 +1042,16 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     const T *gr = dy + row[j] * g.sk;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
-      const int c = c0 + k * cstride;
+      const int i0 = chunk_key<E, RAG>(c0 + k * cstride, g.sk);
+      yraw[j][k].zero();
+      graw[j][k].zero();
       if (!skip[j][k]) {
-        load_chunk<T, E, true, RAG>(yr + chunk_key<E, RAG>(c, g.sk), yv[j][k]);
-        load_chunk<T, E, true, RAG>(gr + chunk_key<E, RAG>(c, g.sk), gv[j][k]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          yv[j][k][e] = 0.f;
-          gv[j][k][e] = 0.f;
-        }
+        yraw[j][k].template load<RAG>(yr + i0);
+        graw[j][k].template load<RAG>(gr + i0);
       }
     }
   }
+  if constexpr (VPL * RPW > 1) wait_loads();
   // wave-uniform: no lane of the wave loaded chunk slot (j, k) -> no arithmetic
   bool none_loaded[RPW][VPL];
 #pragma unroll
@@ -1059,6 +1067,8 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       if (none_loaded[j][k]) continue;
+      yraw[j][k].unpack(yv[j][k]);
+      graw[j][k].unpack(gv[j][k]);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         if constexpr (RAG)
@@ -1535,6 +1545,59 @@ static inline unsigned ragged_keep_lds(const SoftmaxPlan &pl) {
   return (unsigned)(pl.rpb * (kWave / pl.lpr) * keep_bytes(lanes, pl.vpl));
 }
 
+// Waves of a launch to keep on a CU, 0 for as many as fit.  A wave requests its
+// whole row at once, so the waves on a CU decide how much of the operands is
+// requested at a time, and the memory serves a launch fastest when that is some
+// 64 KB per CU (forward) or 96 KB (backward): less leaves it idle, more widens
+// the window of addresses that is open at once.  Measured at 1 GB tensors, waves
+// that fit -> waves kept: bf16 causal 2048 keys forward 252 -> 241 us (16),
+// backward 328 -> 307 (12); 1024 keys backward 318 -> 308 (24); fp32 1024 keys
+// 253 -> 235 (14) and 338 -> 309 (12); [256, 2048, 2048] forward 547 -> 508,
+// backward 694 -> 655.
+// Launches that spend the time on arithmetic (dropout on 16-bit rows), on mask
+// bytes, or on the barrier between the waves of a row want more waves: with
+// dropout 160 KB in the backward (20 waves of 2048 keys: 317 us, 12: 343) and no
+// limit in the 16-bit forward, causal with a key mask 160 KB (314 against 342 us),
+// rows of several waves 160 and 96 KB (4096 keys backward 322 against 348 us),
+// ragged rows, two to a workgroup, 128 KB.
+template <typename T, int MODE>
+static int softmax_waves_per_cu(const SoftmaxPlan &pl, bool backward, bool drop, bool causal,
+                                bool ragged) {
+  constexpr bool k16 = sizeof(T) == 2;
+  int kb;
+  if (backward) {
+    kb = MODE == kModeDense || MODE == kModeBias ? 112 : 96;
+    if (ragged) kb = 128;
+    if (drop) kb = k16 ? 160 : 112;
+    if (pl.wpr > 1 || (MODE == kModeMasked && causal)) kb = 160;
+  } else {
+    kb = MODE == kModeMasked ? 112 : 64;
+    if (drop) kb = 96;
+    if (pl.wpr > 1 && kb < 96) kb = 96;
+    if (drop && k16) return 0;
+  }
+  int waves = kb / (pl.vpl * pl.rpw * (backward ? 2 : 1));  // (1 KB per chunk slot and operand)
+  // forward rows that would leave room for more than 28 waves: 3-5 % faster
+  // with 28, but for 16-bit causal rows of whole waves (1024 keys: 3 % slower)
+  // and ragged rows (197 keys: 5 % slower)
+  if (!backward && !drop && !ragged && waves > 28 &&
+      !(MODE == kModeCausal && k16 && pl.lpr == kWave))
+    waves = 28;
+  return waves;
+}
+
+// LDS that a launch of `nblocks` workgroups reserves in order to keep at most
+// `waves` of its waves on a CU.  (Not for workgroups of a third of the CU and
+// more, and not for launches of a few rounds, whose tail would grow.)
+static inline unsigned occupancy_lds(int waves, int threads, int64_t nblocks) {
+  const bool asked = g_tune.softmax_waves_per_cu > 0;
+  if (asked) waves = g_tune.softmax_waves_per_cu;
+  const int blocks = waves * kWave / threads;
+  if (waves <= 0 || waves >= 32 || blocks < 3) return 0;
+  if (!asked && nblocks < (int64_t)device_cu_count() * blocks * 4) return 0;
+  return (unsigned)(160 * 1024 / blocks - 512);
+}
+
 constexpr int kFwdMaxElems = 64;  // one operand resident
 constexpr int kBwdMaxElems = 32;  // two operands resident
 
@@ -1676,18 +1739,21 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   if (g_tune.softmax_causal_order == 0 && pl.wpr > 1) g.causal_order = 1;
   g.rpb = pl.rpb;
   const int threads = kWave * pl.wpr * pl.rpb;
+  const unsigned keep_lds = ragged_keep_lds(pl);
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
+  const unsigned occ = occupancy_lds(
+      softmax_waves_per_cu<T, MODE>(pl, false, drop, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_FWD(VPL, RPW, LPR_)                                  \
   if constexpr (VPL * RPW * E <= (MODE == kModeBias ? kBiasMaxElems : kFwdMaxElems)) { \
     if (drop)                                                        \
       softmax_fwd_kernel<T, VPL, RPW, MODE, true, LPR_>              \
-          <<<dim3((unsigned)grid), threads, 0, st>>>(                \
+          <<<dim3((unsigned)grid), threads, occ, st>>>(                \
               (const T *)x, mask, (T *)y, stats, g, scale, d);       \
     else                                                             \
       softmax_fwd_kernel<T, VPL, RPW, MODE, false, LPR_>             \
-          <<<dim3((unsigned)grid), threads, 0, st>>>(                \
+          <<<dim3((unsigned)grid), threads, occ, st>>>(                \
               (const T *)x, mask, (T *)y, nullptr, g, scale, d);     \
   } else                                                             \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax fwd: no kernel for %d x %d chunks per lane", VPL, RPW)
@@ -1695,11 +1761,11 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   do {                                                               \
     if (drop)                                                        \
       softmax_fwd_kernel<T, VPL, 1, MODE, true, LPR_, true>          \
-          <<<dim3((unsigned)grid), threads, ragged_keep_lds(pl), st>>>( \
+          <<<dim3((unsigned)grid), threads, keep_lds > occ ? keep_lds : occ, st>>>( \
               (const T *)x, mask, (T *)y, stats, g, scale, d);       \
     else                                                             \
       softmax_fwd_kernel<T, VPL, 1, MODE, false, LPR_, true>         \
-          <<<dim3((unsigned)grid), threads, 0, st>>>(                \
+          <<<dim3((unsigned)grid), threads, occ, st>>>(                \
               (const T *)x, mask, (T *)y, nullptr, g, scale, d);     \
   } while (0)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
@@ -1760,18 +1826,20 @@ int launch_softmax_bwd(const void *dy, const void *y,
   const int threads = kWave * pl.wpr * pl.rpb;
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
+  const unsigned occ = occupancy_lds(
+      softmax_waves_per_cu<T, MODE>(pl, true, false, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_BWD(VPL, RPW, LPR_)                        \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_))       \
     softmax_bwd_kernel<T, VPL, RPW, MODE, LPR_>            \
-        <<<dim3((unsigned)grid), threads, 0, st>>>(        \
+        <<<dim3((unsigned)grid), threads, occ, st>>>(        \
             (const T *)dy, (const T *)y, mask, (T *)dx, g, scale); \
   else                                                     \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
 #define OSLO_SM_BWD_RAGGED(VPL, LPR_)                      \
   if constexpr (VPL == 1 || LPR_ == kWave)                 \
     softmax_bwd_kernel<T, VPL, 1, MODE, LPR_, true>        \
-        <<<dim3((unsigned)grid), threads, 0, st>>>(        \
+        <<<dim3((unsigned)grid), threads, occ, st>>>(        \
             (const T *)dy, (const T *)y, mask, (T *)dx, g, scale); \
   else                                                     \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax bwd: no kernel for %d chunks in %d lanes", VPL, LPR_)
@@ -1829,20 +1897,23 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
   if (g_tune.softmax_causal_order == 0 && pl.wpr > 1) g.causal_order = 1;
   g.rpb = pl.rpb;
   const int threads = kWave * pl.wpr * pl.rpb;
+  const unsigned keep_lds = ragged_keep_lds(pl);
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
+  const unsigned occ = occupancy_lds(
+      softmax_waves_per_cu<T, MODE>(pl, true, true, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_DBWD(VPL, RPW, LPR_)                                \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_) && (MODE != kModeBias || RPW <= 2)) \
     softmax_dropout_bwd_kernel<T, VPL, RPW, MODE, LPR_>             \
-        <<<dim3((unsigned)grid), threads, 0, st>>>(                 \
+        <<<dim3((unsigned)grid), threads, occ, st>>>(                 \
             (const T *)dy, (const T *)x, stats, mask, (T *)dx, g,   \
             scale, d);                                              \
   else                                                              \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax dropout bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
 #define OSLO_SM_DBWD_RAGGED(VPL, LPR_)                              \
   softmax_dropout_bwd_kernel<T, VPL, 1, MODE, LPR_, true>           \
-      <<<dim3((unsigned)grid), threads, ragged_keep_lds(pl), st>>>( \
+      <<<dim3((unsigned)grid), threads, keep_lds > occ ? keep_lds : occ, st>>>( \
           (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
   int64_t launch_blocks = nblocks;
