@@ -491,7 +491,8 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
   static_assert(LPR == kWave || VPL == 1 || VPL == 3, "side-by-side rows: one or three chunks per lane");
   static_assert(UNIT == kWave || (UNIT == 32 && LPR == kWave && VPL == 1 && EVEN),
                 "half-wave units: whole-unit rows, one chunk per lane");
-  extern __shared__ __align__(16) float xslot[];  // [n2] when rpb > 1
+  // gamma chunks during the rows, then the column sums of the row slots
+  extern __shared__ __align__(16) float xslot[];
   __shared__ float red[2][64];
   const int lane = UNIT == kWave ? (threadIdx.x & 63) : (threadIdx.x & 31);
   // the wave index is uniform: keep it (and the row arithmetic) in scalar registers
@@ -514,8 +515,7 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
   // gamma then live in LDS, each lane reading back what it wrote (no barrier).
   constexpr int GREG = VPL * E >= 16 ? (sizeof(V) == 4 ? 1 : 0) : VPL;
   RawChunk<V, E> gmraw[GREG > 0 ? GREG : 1];
-  RawChunk<V, E> *const gslot =
-      reinterpret_cast<RawChunk<V, E> *>(xslot + (rpb > SUB ? n2 : 0));
+  RawChunk<V, E> *const gslot = reinterpret_cast<RawChunk<V, E> *>(xslot);
   float acc_g[VPL][E], acc_b[VPL][E];
   float acc_d[FUSE ? VPL : 1][E];  // bias gradient of the fused epilogue
 #pragma unroll
@@ -603,7 +603,9 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
 #pragma unroll
       for (int k = 0; k < VPL; ++k) f.extra[k].unpack(extra[k]);
     }
-    fetch(f, base + PF * rstride);
+    // (a workgroup of a small batch has one or two iterations: a prefetch past
+    //  the end would double or triple what it reads)
+    if (base + PF * rstride < n1) fetch(f, base + PF * rstride);
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
@@ -688,7 +690,7 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
   } else {
     RowFetch f0, f1;
     fetch(f0, base0);
-    fetch(f1, base0 + rstride);
+    if (base0 + rstride < n1) fetch(f1, base0 + rstride);
     for (int64_t base = base0; base < n1; base += 2 * rstride) {
       process(f0, base);
       if (base + rstride >= n1) break;  // uniform over the workgroup
@@ -698,7 +700,11 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
 
   if (part == nullptr) return;  // uniform: no parameter gradients wanted
 
-  // Fold the row slots of this workgroup into slot 0, one slot at a time.
+  // The row slots of this workgroup are summed through LDS, one chunk per lane
+  // and array at a time: every slot writes its columns, then each column is
+  // summed over the slots in order by one thread (128-bit accesses, two
+  // barriers; slot after slot into the first took two barriers per slot, 28 to
+  // 42 in a row for rows of 768 elements).
   // Arrays: 0 = dgamma, then dbeta (LayerNorm only), then the bias gradient of
   // the fused epilogue (last, when wanted).
   constexpr int NARR = RMS ? 1 : 2;
@@ -707,6 +713,8 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
   // registers: none of them is indexed by a run-time value)
   const int wslots = LPR == kWave ? rpb : rpb / SUB;  // wave-level row slots
   const bool lead = LPR == kWave || lane < LPR;        // first lane group
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  f32x4 *const fold = reinterpret_cast<f32x4 *>(xslot);  // [wslots][cstride][E / 4]
   auto fold_and_store = [&](auto &acc, int a) {
     if constexpr (LPR < kWave) {
       // the lane groups of a wave hold the same columns: sum them into the
@@ -721,36 +729,31 @@ __global__ __launch_bounds__(MAXT) void norm_bwd_reg_kernel(
           acc[k][e] = t;
         }
     }
-    for (int s = 1; s < wslots; ++s) {
-      __syncthreads();
-      if (wslot == s && lead) {
-#pragma unroll
-        for (int k = 0; k < VPL; ++k) {
-          const int c = c0 + k * cstride;
-          if (c < nchunks) {
-#pragma unroll
-            for (int e = 0; e < E; ++e) xslot[c * E + e] = acc[k][e];
-          }
-        }
-      }
-      __syncthreads();
-      if (wslot == 0 && lead) {
-#pragma unroll
-        for (int k = 0; k < VPL; ++k) {
-          const int c = c0 + k * cstride;
-          if (c < nchunks) {
-#pragma unroll
-            for (int e = 0; e < E; ++e) acc[k][e] += xslot[c * E + e];
-          }
-        }
-      }
-    }
-    if (wslot == 0 && lead) {
-      float *prow = part + ((int64_t)a * P + blockIdx.x) * n2;
+    float *prow = part + ((int64_t)a * P + blockIdx.x) * n2;
+    if (wslots == 1) {
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
         const int c = c0 + k * cstride;
-        if (c < nchunks) store_chunk<float, E>(prow + (int64_t)c * E, acc[k]);
+        if (lead && c < nchunks) store_chunk<float, E>(prow + (int64_t)c * E, acc[k]);
+      }
+      return;
+    }
+    constexpr int Q = E / 4;  // quads per chunk
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      __syncthreads();
+      if (lead) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          fold[(wslot * cstride + c0) * Q + q] =
+              f32x4{acc[k][4 * q], acc[k][4 * q + 1], acc[k][4 * q + 2], acc[k][4 * q + 3]};
+      }
+      __syncthreads();
+      for (int q = threadIdx.x; q < cstride * Q; q += blockDim.x) {
+        if (k * cstride + q / Q >= nchunks) break;
+        f32x4 t = fold[q];
+        for (int s = 1; s < wslots; ++s) t += fold[s * cstride * Q + q];
+        *reinterpret_cast<f32x4 *>(prow + (int64_t)k * cstride * E + 4 * q) = t;
       }
     }
   };
@@ -1231,9 +1234,13 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
       if (cap > 16 / E) cap = 16 / E;
       sp = split_row(n2 / E, cap, allowed, nallowed, waves);
     } else {
-      // measured best on MI355X: 8 elements per lane wherever a row then
-      // fits one workgroup, else 16 elements per lane
-      sp = split_row(n2 / E, 8 / E, allowed, nallowed, waves);
+      // the narrowest split that fits one workgroup: one chunk per lane, then
+      // two (fp32 only), then 16 elements.  (fp32 with 8 elements per lane,
+      // where 4 would do, left a quarter of the lanes of a 768-element row
+      // idle and did not fit the registers of the fused epilogue: [2048, 768]
+      // 26 -> 12 us, [4096, 4096] 102 -> 64; plain 10.0 -> 9.3, 40 -> 39)
+      sp = split_row(n2 / E, 1, allowed, nallowed, waves);
+      if (!sp.ok && E == 4) sp = split_row(n2 / E, 2, allowed, nallowed, waves);
       if (!sp.ok) {
         const RowSplit wide = split_row(n2 / E, 16 / E, allowed, nallowed, waves);
         if (wide.ok) sp = wide;
@@ -1298,6 +1305,13 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
     sp.wpr = upr;
     sp.rpb = 32 / upr;
   }
+  // With fewer rows than slots on the chip, slots give way to workgroups on
+  // idle CUs ([512, 1024] fp16: 64 workgroups of 8 slots -> 256 of 2)
+  const int64_t rows_per_cu = ceil_div(n1, (int64_t)device_cu_count());
+  if (sp.rpb > rows_per_cu) {
+    sp.rpb = (int)rows_per_cu;
+    if (upr > 0) sp.rpb += sp.rpb & 1;  // (two units to a wave)
+  }
   // short rows side by side in a wave: the row slots of a workgroup multiply
   // (the three-chunks-per-lane mapping of the forward kernel does not pay
   //  here: its 24 elements per lane and operand need a 512-thread workgroup,
@@ -1323,12 +1337,15 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
     part = (float *)ws;
   }
   const int threads = (upr > 0 ? 32 : kWave) * sp.wpr * wave_slots;
-  // LDS: one row of column partials when a workgroup holds several row
-  // slots, and behind it the chunks of gamma that 16 elements per lane move
-  // out of the registers (one of four with 4-byte parameters, else all)
-  size_t lds = wave_slots > 1 ? (size_t)n2 * sizeof(float) : 0;
-  if (sp.vpl * E >= 16)
-    lds += (size_t)(sp.vpl - (sizeof(V) == 4 ? 1 : 0)) * threads * E * sizeof(V);
+  // LDS: the chunks of gamma that 16 elements per lane move out of the
+  // registers (one of four with 4-byte parameters, else all), and after the
+  // last row, in the same place, the column sums of one chunk per lane when a
+  // workgroup holds several row slots (at most 32 KB)
+  size_t lds = wave_slots > 1 ? (size_t)threads * E * sizeof(float) : 0;
+  if (sp.vpl * E >= 16) {
+    const size_t gl = (size_t)(sp.vpl - (sizeof(V) == 4 ? 1 : 0)) * threads * E * sizeof(V);
+    if (gl > lds) lds = gl;
+  }
   const bool even = upr > 0 ? true
                   : lpr < kWave ? (n2 / E) == lpr
                                 : (n2 / E) == (int64_t)sp.vpl * kWave * sp.wpr;
@@ -1337,8 +1354,11 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
   // else one (a wave that owns whole rows measures 6 % slower with two)
   // (plain workgroups of twelve waves, rows of 3072 and 6144 16-bit
   //  elements, measure 2.5 % faster with one; with the fused epilogue 8 %
-  //  slower)
-  int pf = sp.vpl * E <= 8 && sp.wpr >= 2 && (fused || threads != 12 * kWave) ? 2 : 1;
+  //  slower.  fp32 rows are not packed: two of them with three operands and
+  //  three accumulators spill at 8 elements per lane ([8192, 768] 59 us
+  //  against 34) and gain nothing at 4)
+  int pf = sp.vpl * E <= 8 && sp.wpr >= 2 &&
+                   (fused ? E == 8 : threads != 12 * kWave) ? 2 : 1;
   if (g_tune.norm_bwd_prefetch > 0) pf = g_tune.norm_bwd_prefetch >= 2 ? 2 : 1;
 #define OSLO_BWD_LAUNCH_T(VPL, EVEN_, PF_, MAXT_)                          \
   do {                                                                     \
