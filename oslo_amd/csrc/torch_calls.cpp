@@ -1,0 +1,909 @@
+// The per-call host work of the layer ops, in native code: argument checks,
+// output allocation, the launch through the C ABI (include/oslo_hip.h) and
+// nothing else.  One function per method of the kernel objects in
+// oslo_amd/torch/_C/__init__.py, which document the semantics and own the
+// workspaces; the autograd Functions above them stay in Python.
+//
+// Why native: a decoding step or a small layer is bound by the host.  Checks
+// and allocations in Python with a ctypes call of twelve to eighteen arguments
+// took 9-11 us of a norm's 14.6 us a call, of which the launch is about 3.
+//
+// The GIL is held while the arguments are read and released from the first
+// allocation to the launch, so that a launch that blocks (a full queue) does
+// not stop other Python threads.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <optional>
+#include <vector>
+
+#include "../../include/oslo_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// ---------------------------------------------------------------- arguments
+struct Args {
+  PyObject *const *a;
+  Py_ssize_t n, i = 0;
+
+  PyObject *next() {
+    TORCH_CHECK_TYPE(i < n, "too few arguments");
+    return a[i++];
+  }
+  const Tensor &tensor() {
+    PyObject *o = next();
+    TORCH_CHECK_TYPE(THPVariable_Check(o), "argument ", i, " must be a Tensor, not ", Py_TYPE(o)->tp_name);
+    return THPVariable_Unpack(o);
+  }
+  // undefined for None
+  Tensor optional() {
+    if (a[i < n ? i : 0] == Py_None) {
+      next();
+      return Tensor();
+    }
+    return tensor();
+  }
+  bool flag() {
+    const int r = PyObject_IsTrue(next());
+    if (r < 0) throw python_error();
+    return r != 0;
+  }
+  // None -> -1, else the truth value
+  int tristate() {
+    if (i < n && a[i] == Py_None) {
+      ++i;
+      return -1;
+    }
+    return flag() ? 1 : 0;
+  }
+  double real() {
+    const double v = PyFloat_AsDouble(next());
+    if (v == -1.0 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+  int64_t integer() {
+    const int64_t v = PyLong_AsLongLong(next());
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+  // any integer, modulo 2^64
+  uint64_t word() {
+    PyObject *o = PyNumber_Long(next());
+    if (o == nullptr) throw python_error();
+    const uint64_t v = PyLong_AsUnsignedLongLongMask(o);
+    Py_DECREF(o);
+    if (v == (uint64_t)-1 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+  std::vector<int64_t> sizes() {
+    PyObject *o = PySequence_Fast(next(), "normalized_shape must be a sequence of integers");
+    if (o == nullptr) throw python_error();
+    std::vector<int64_t> v;
+    for (Py_ssize_t k = 0; k < PySequence_Fast_GET_SIZE(o); ++k) {
+      PyObject *e = PyNumber_Long(PySequence_Fast_GET_ITEM(o, k));
+      v.push_back(e != nullptr ? PyLong_AsLongLong(e) : -1);
+      Py_XDECREF(e);
+      if (PyErr_Occurred()) {
+        Py_DECREF(o);
+        throw python_error();
+      }
+    }
+    Py_DECREF(o);
+    return v;
+  }
+};
+
+struct NoGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+PyObject *wrap(const Tensor &t) {
+  if (t.defined()) return THPVariable_Wrap(t);
+  Py_RETURN_NONE;
+}
+
+PyObject *wrap_all(std::initializer_list<Tensor> ts, bool list) {
+  const Py_ssize_t n = (Py_ssize_t)ts.size();
+  PyObject *o = list ? PyList_New(n) : PyTuple_New(n);
+  if (o == nullptr) throw python_error();
+  Py_ssize_t k = 0;
+  for (const Tensor &t : ts) {
+    PyObject *e = wrap(t);
+    if (e == nullptr) {
+      Py_DECREF(o);
+      throw python_error();
+    }
+    if (list) PyList_SET_ITEM(o, k++, e);
+    else PyTuple_SET_ITEM(o, k++, e);
+  }
+  return o;
+}
+
+// ---------------------------------------------------------------- checks
+std::string dtype_name(at::ScalarType t) { return "torch." + c10::getDtypeNames(t).first; }
+
+int dtype_code(const Tensor &t, const char *what, bool f64 = false) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return OSLO_DTYPE_F32;
+    case at::kHalf: return OSLO_DTYPE_F16;
+    case at::kBFloat16: return OSLO_DTYPE_BF16;
+    case at::kDouble:
+      if (f64) return OSLO_DTYPE_F64;
+      break;
+    default: break;
+  }
+  TORCH_CHECK(false, what, ": dtype ", dtype_name(t.scalar_type()),
+              " is not supported by the HIP kernels (float32, float16 and bfloat16 are",
+              f64 ? "" : "; float64 only by the norms", ")");
+}
+
+// CHECK_INPUT of FusedLayerNormBinder.cpp:8-14
+void check_input(const Tensor &t, const char *name) {
+  TORCH_CHECK(t.is_cuda(), name, " must be a CUDA tensor");
+  TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+}
+
+void check_param(const Tensor &t, const std::vector<int64_t> &shape, const char *name) {
+  if (t.defined())
+    TORCH_CHECK(t.sizes() == at::IntArrayRef(shape), name, " of shape ", t.sizes(),
+                " does not match normalized_shape=", at::IntArrayRef(shape));
+}
+
+// check_args / compute_n1_n2 of FusedLayerNormBinder.cpp:19-36, 59-93
+void rows_and_length(const Tensor &x, const std::vector<int64_t> &shape, int64_t &n1, int64_t &n2) {
+  const int64_t nd = (int64_t)shape.size();
+  TORCH_CHECK(nd >= 1,
+              "Expected normalized_shape to be at least 1-dimensional, i.e., containing at "
+              "least one element, but got normalized_shape=", at::IntArrayRef(shape));
+  TORCH_CHECK(x.dim() >= nd && x.sizes().slice(x.dim() - nd) == at::IntArrayRef(shape),
+              "Given normalized_shape=", at::IntArrayRef(shape), ", expected input with shape [*, ",
+              c10::Join(", ", shape), "], but got input of size", x.sizes());
+  n2 = 1;
+  for (int64_t s : shape) n2 *= s;
+  n1 = n2 > 0 ? x.numel() / n2 : 0;
+}
+
+void check_rc(int rc) { TORCH_CHECK(rc == 0, oslo_hip_last_error()); }
+
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+// FusedLayerNormBinder.cpp:146-152: the statistics are fp32 for 16-bit inputs
+// and have the input's type otherwise
+at::ScalarType stat_type(const Tensor &t) { return t.scalar_type() == at::kDouble ? at::kDouble : at::kFloat; }
+
+Tensor new_f32(const Tensor &like, at::IntArrayRef shape) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+
+// The operand's device made current for one call, and torch's current stream on it.
+struct OnDevice {
+  c10::DeviceGuard guard;
+  void *stream;
+  explicit OnDevice(const Tensor &t)
+      : guard(t.device()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+};
+
+// An output of the softmax: from 64 MiB on it starts k * (1 MiB + 4 KiB) past
+// a 2 MiB boundary (empty_staggered of the Python module says why).
+Tensor softmax_out(const Tensor &like, int k) {
+  constexpr int64_t kMin = 64ll << 20, kStep = (1 << 20) + 4096, kRound = 2 << 20;
+  const int64_t nbytes = like.numel() * (int64_t)like.element_size();
+  if (nbytes < kMin) return at::empty(like.sizes(), like.options());
+  const Tensor base = at::empty({nbytes + kRound}, like.options().dtype(at::kByte));
+  const int64_t phase = (int64_t)(reinterpret_cast<uintptr_t>(base.data_ptr()) % kRound);
+  const int64_t off = ((k * kStep - phase) % kRound + kRound) % kRound;
+  return base.slice(0, off, off + nbytes).view(like.scalar_type()).view(like.sizes());
+}
+
+// ---------------------------------------------------------------- norms
+// (rms, input, normalized_shape, gamma, beta, eps, mixed) -> [output, (mean,) invvar]
+PyObject *norm_forward(Args &g) {
+  const bool rms = g.flag();
+  const Tensor &x = g.tensor();
+  const auto shape = g.sizes();
+  const Tensor gamma = g.optional(), beta = g.optional();
+  const double eps = g.real();
+  const bool mixed = g.flag();
+  check_input(x, "input");
+  int64_t n1, n2;
+  rows_and_length(x, shape, n1, n2);
+  check_param(gamma, shape, "gamma");
+  check_param(beta, shape, "beta");
+  const int din = dtype_code(x, "input", true);
+  const at::ScalarType out_type = mixed ? gamma.scalar_type() : x.scalar_type();
+  const std::pair<const char *, const Tensor *> params[] = {{"gamma", &gamma}, {"beta", &beta}};
+  for (const auto &[name, t] : params)
+    if (t->defined()) {
+      check_input(*t, name);
+      TORCH_CHECK(t->scalar_type() == out_type, name, " has dtype ", dtype_name(t->scalar_type()),
+                  " but the output dtype is ", dtype_name(out_type));
+    }
+  const int dout = mixed ? dtype_code(gamma, "output", true) : din;
+  Tensor out, mean, inv;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    out = at::empty(x.sizes(), x.options().dtype(out_type));
+    const auto stats = x.options().dtype(stat_type(x));
+    inv = at::empty({n1}, stats);
+    if (rms) {
+      check_rc(oslo_rms_fwd(ptr(x), ptr(gamma), ptr(out), ptr(inv), n1, n2, eps, din, dout, on.stream));
+    } else {
+      mean = at::empty({n1}, stats);
+      check_rc(oslo_ln_fwd(ptr(x), ptr(gamma), ptr(beta), ptr(out), ptr(mean), ptr(inv), n1, n2, eps, din,
+                           dout, on.stream));
+    }
+  }
+  return rms ? wrap_all({out, inv}, true) : wrap_all({out, mean, inv}, true);
+}
+
+// (rms, dout, mean, invvar, input, normalized_shape, gamma, beta, workspace, nbytes)
+// -> (grad_input, grad_gamma, grad_beta)
+PyObject *norm_backward(Args &g) {
+  const bool rms = g.flag();
+  const Tensor &dy = g.tensor();
+  const Tensor mean = g.optional();
+  const Tensor &inv = g.tensor();
+  const Tensor &x = g.tensor();
+  const auto shape = g.sizes();
+  const Tensor gamma = g.optional(), beta = g.optional(), ws = g.optional();
+  const int64_t nbytes = g.integer();
+  check_input(dy, "dout");
+  check_input(inv, "invvar");
+  check_input(x, "input");
+  if (!rms) {
+    TORCH_CHECK(mean.defined(), "mean is missing");
+    check_input(mean, "mean");
+  }
+  int64_t n1, n2;
+  rows_and_length(x, shape, n1, n2);
+  TORCH_CHECK(dy.sizes() == x.sizes(), "dout of size ", dy.sizes(), " does not match input of size ", x.sizes());
+  const int din = dtype_code(x, "input", true), dcode = dtype_code(dy, "dout", true);
+  const std::pair<const char *, const Tensor *> stats[] = {{"invvar", &inv}, {"mean", &mean}};
+  for (const auto &[name, t] : stats)
+    if (t->defined()) {
+      TORCH_CHECK(t->scalar_type() == stat_type(x), name, " has dtype ", dtype_name(t->scalar_type()),
+                  ", expected ", dtype_name(stat_type(x)));
+      TORCH_CHECK(t->numel() == n1, name, " has ", t->numel(), " elements for ", n1, " rows of input");
+    }
+  if (gamma.defined()) {
+    check_input(gamma, "gamma");
+    check_param(gamma, shape, "gamma");
+    TORCH_CHECK(gamma.scalar_type() == dy.scalar_type(), "gamma has dtype ", dtype_name(gamma.scalar_type()),
+                " but dout has dtype ", dtype_name(dy.scalar_type()));
+  }
+  Tensor dx, dg, db;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    dx = at::empty(x.sizes(), x.options());
+    if (gamma.defined()) {
+      dg = at::empty_like(gamma);
+      if (!rms) db = at::empty_like(beta.defined() ? beta : gamma);
+    }
+    check_rc(rms ? oslo_rms_bwd(ptr(dy), ptr(x), ptr(inv), ptr(gamma), ptr(dx), ptr(dg), ptr(ws), nbytes, n1,
+                                n2, din, dcode, on.stream)
+                 : oslo_ln_bwd(ptr(dy), ptr(x), ptr(mean), ptr(inv), ptr(gamma), ptr(dx), ptr(dg), ptr(db),
+                               ptr(ws), nbytes, n1, n2, din, dcode, on.stream));
+  }
+  return wrap_all({dx, dg, db}, false);
+}
+
+// (rms, input, bias, residual, normalized_shape, gamma, beta, eps, p, seed, offset, want_h)
+// -> [y, h, mean, invvar]
+PyObject *residual_norm_forward(Args &g) {
+  const bool rms = g.flag();
+  const Tensor &x = g.tensor();
+  const Tensor bias = g.optional(), res = g.optional();
+  const auto shape = g.sizes();
+  const Tensor gamma = g.optional(), beta = g.optional();
+  const double eps = g.real(), p = g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool want_h = g.flag();
+  check_input(x, "input");
+  int64_t n1, n2;
+  rows_and_length(x, shape, n1, n2);
+  const std::pair<const char *, const Tensor *> ops[] = {
+      {"gamma", &gamma}, {"beta", &beta}, {"bias", &bias}, {"residual", &res}};
+  for (const auto &[name, t] : ops)
+    if (t->defined()) {
+      check_input(*t, name);
+      if (t != &res) check_param(*t, shape, name);
+    }
+  TORCH_CHECK(!res.defined() || res.sizes() == x.sizes(), "residual and input differ in shape");
+  for (const auto &[name, t] : ops)
+    TORCH_CHECK(!t->defined() || t->scalar_type() == x.scalar_type(), name, " has dtype ",
+                dtype_name(t->scalar_type()), " but input has dtype ", dtype_name(x.scalar_type()));
+  const int code = dtype_code(x, "input");
+  Tensor y, h, mean, inv;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    y = at::empty(x.sizes(), x.options());
+    if (want_h) h = at::empty(x.sizes(), x.options());
+    inv = new_f32(x, {n1});
+    if (!rms) mean = new_f32(x, {n1});
+    check_rc(oslo_bias_dropout_add_norm_fwd(ptr(x), ptr(bias), ptr(res), ptr(gamma), ptr(beta), ptr(h), ptr(y),
+                                            (float *)ptr(mean), (float *)ptr(inv), n1, n2, eps, (float)p, seed, offset, rms, code,
+                                            on.stream));
+  }
+  return wrap_all({y, h, mean, inv}, true);
+}
+
+// (rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma, p, seed, offset,
+//  need_bias_grad, workspace, nbytes)
+// -> (grad_residual, grad_input, grad_gamma, grad_beta, grad_bias)
+PyObject *residual_norm_backward(Args &g) {
+  const bool rms = g.flag();
+  const Tensor &dy = g.tensor();
+  const Tensor extra = g.optional();
+  const Tensor &h = g.tensor();
+  const Tensor mean = g.optional();
+  const Tensor &inv = g.tensor();
+  const auto shape = g.sizes();
+  const Tensor gamma = g.optional();
+  const double p = g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool want_bias = g.flag();
+  const Tensor ws = g.optional();
+  const int64_t nbytes = g.integer();
+  check_input(dy, "dout");
+  check_input(h, "h");
+  check_input(inv, "invvar");
+  int64_t n1, n2;
+  rows_and_length(h, shape, n1, n2);
+  TORCH_CHECK(dy.sizes() == h.sizes() && dy.scalar_type() == h.scalar_type(), "dout and h differ in shape or dtype");
+  if (!rms) {
+    TORCH_CHECK(mean.defined(), "mean is missing");
+    check_input(mean, "mean");
+  }
+  const auto check_stat = [&](const Tensor &t, const char *name) {
+    TORCH_CHECK(t.scalar_type() == at::kFloat && t.numel() == n1, name,
+                " must be float32 with one element per row of h");
+  };
+  check_stat(inv, "invvar");
+  if (!rms) check_stat(mean, "mean");
+  if (extra.defined()) {
+    check_input(extra, "dh_extra");
+    TORCH_CHECK(extra.sizes() == h.sizes() && extra.scalar_type() == h.scalar_type(),
+                "dh_extra and h differ in shape or dtype");
+  }
+  const int code = dtype_code(h, "h");
+  if (gamma.defined()) {
+    check_input(gamma, "gamma");
+    check_param(gamma, shape, "gamma");
+    TORCH_CHECK(gamma.scalar_type() == h.scalar_type(), "gamma has dtype ", dtype_name(gamma.scalar_type()),
+                " but h has dtype ", dtype_name(h.scalar_type()));
+  }
+  Tensor dres, dx, dg, db, dbias;
+  {
+    NoGil nogil;
+    const OnDevice on(h);
+    dres = at::empty(h.sizes(), h.options());
+    if (p > 0.0) dx = at::empty(h.sizes(), h.options());
+    if (gamma.defined()) {
+      dg = at::empty_like(gamma);
+      if (!rms) db = at::empty_like(gamma);
+    }
+    if (want_bias) dbias = at::empty(shape, h.options());
+    check_rc(oslo_bias_dropout_add_norm_bwd(ptr(dy), ptr(extra), ptr(h), rms ? nullptr : (const float *)ptr(mean), (const float *)ptr(inv),
+                                            ptr(gamma), ptr(dres), ptr(dx), ptr(dg), ptr(db), ptr(dbias), ptr(ws),
+                                            nbytes, n1, n2, (float)p, seed, offset, rms, code, on.stream));
+  }
+  return wrap_all({dres, dx.defined() ? dx : dres, dg, db, dbias}, false);
+}
+
+// ---------------------------------------------------------------- softmax
+void check_same(const Tensor &a, const char *na, const Tensor &b, const char *nb) {
+  check_input(a, na);
+  check_input(b, nb);
+  TORCH_CHECK(a.scalar_type() == b.scalar_type(), na, " and ", nb, " differ in dtype");
+  TORCH_CHECK(a.sizes() == b.sizes(), na, " and ", nb, " differ in shape");
+}
+
+// A boolean mask (non-zero = hidden) as contiguous bytes.
+Tensor mask_bytes(const Tensor &mask, const Tensor &like) {
+  TORCH_CHECK(mask.device() == like.device(), "mask is on ", mask.device().str(), " but the softmax operand is on ",
+              like.device().str());
+  if (mask.scalar_type() == at::kBool || mask.scalar_type() == at::kByte) return mask.contiguous();
+  return mask.ne(0).contiguous();
+}
+
+void check_mask_dims(const Tensor &x, const Tensor &mask) {
+  TORCH_CHECK(x.dim() == 4 && mask.dim() == 4, "expected 4D tensor");
+  TORCH_CHECK(mask.size(1) == 1 && mask.size(3) == x.size(3) && (mask.size(0) == 1 || mask.size(0) == x.size(0)) &&
+                  (mask.size(2) == 1 || mask.size(2) == x.size(2)),
+              "mask of size ", mask.sizes(), " does not broadcast to [", x.size(0), ", 1, ", x.size(2), ", ",
+              x.size(3), "]");
+}
+
+// (input, scale) -> out
+PyObject *causal_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const float scale = (float)g.real();
+  TORCH_CHECK(x.dim() == 3, "expected 3D tensor");
+  check_input(x, "input");
+  const int code = dtype_code(x, "input");
+  Tensor out;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    out = softmax_out(x, 1);
+    check_rc(oslo_softmax_causal_fwd(ptr(x), ptr(out), x.size(0), x.size(1), x.size(2), scale, code, on.stream));
+  }
+  return wrap(out);
+}
+
+// (output_grads, softmax_results, scale, inplace) -> grad_input
+PyObject *causal_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &y = g.tensor();
+  const float scale = (float)g.real();
+  const bool inplace = g.flag();
+  TORCH_CHECK(dy.dim() == 3 && y.dim() == 3, "expected 3D tensor");
+  check_same(dy, "output_grads", y, "softmax_results");
+  const int code = dtype_code(dy, "output_grads");
+  Tensor dx;
+  {
+    NoGil nogil;
+    const OnDevice on(dy);
+    dx = inplace ? dy : softmax_out(dy, 2);
+    check_rc(oslo_softmax_causal_bwd(ptr(dy), ptr(y), ptr(dx), y.size(0), y.size(1), y.size(2), scale, code,
+                                     on.stream));
+  }
+  return wrap(dx);
+}
+
+// (input, mask, scale, causal) -> out
+PyObject *masked_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor &mask = g.tensor();
+  const float scale = (float)g.real();
+  const bool causal = g.flag();
+  check_mask_dims(x, mask);
+  check_input(x, "input");
+  const int code = dtype_code(x, "input");
+  Tensor out;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Tensor m = mask_bytes(mask, x);
+    out = softmax_out(x, 1);
+    check_rc((causal ? oslo_softmax_causal_masked_fwd : oslo_softmax_masked_fwd)(
+        ptr(x), (const uint8_t *)ptr(m), ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), mask.size(0),
+        mask.size(2), scale, code, on.stream));
+  }
+  return wrap(out);
+}
+
+// (output_grads, softmax_results, scale, mask, inplace, causal) -> grad_input
+PyObject *masked_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &y = g.tensor();
+  const float scale = (float)g.real();
+  const Tensor mask = g.optional();
+  const bool inplace = g.flag(), causal = g.flag();
+  TORCH_CHECK(dy.dim() == 4 && y.dim() == 4, "expected 4D tensor");
+  check_same(dy, "output_grads", y, "softmax_results");
+  if (mask.defined()) check_mask_dims(y, mask);
+  const int code = dtype_code(dy, "output_grads");
+  Tensor dx;
+  {
+    NoGil nogil;
+    const OnDevice on(dy);
+    const Tensor m = mask.defined() ? mask_bytes(mask, y) : Tensor();
+    dx = inplace ? dy : softmax_out(dy, 2);
+    check_rc((causal ? oslo_softmax_causal_masked_bwd : oslo_softmax_masked_bwd)(
+        ptr(dy), ptr(y), (const uint8_t *)ptr(m), ptr(dx), y.size(0), y.size(1), y.size(2), y.size(3),
+        mask.defined() ? mask.size(0) : 1, mask.defined() ? mask.size(2) : 1, scale, code, on.stream));
+  }
+  return wrap(dx);
+}
+
+int64_t row_count(const Tensor &x) { return x.numel() > 0 ? x.numel() / x.size(-1) : 0; }
+
+// (input, mask, scale, p, seed, offset, causal) -> [out, stats]
+PyObject *dropout_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor mask = g.optional();
+  const float scale = (float)g.real(), p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool causal = g.flag();
+  check_input(x, "input");
+  if (mask.defined()) check_mask_dims(x, mask);
+  else TORCH_CHECK(x.dim() == 3, "expected 3D tensor");
+  const int code = dtype_code(x, "input");
+  Tensor out, stats;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Tensor m = mask.defined() ? mask_bytes(mask, x) : Tensor();
+    out = softmax_out(x, 1);
+    stats = new_f32(x, {row_count(x), 2});
+    float *st = stats.data_ptr<float>();
+    check_rc(!mask.defined()
+                 ? oslo_softmax_causal_dropout_fwd(ptr(x), ptr(out), st, x.size(0), x.size(1), x.size(2), scale, p,
+                                                   seed, offset, code, on.stream)
+                 : (causal ? oslo_softmax_causal_masked_dropout_fwd : oslo_softmax_masked_dropout_fwd)(
+                       ptr(x), (const uint8_t *)ptr(m), ptr(out), st, x.size(0), x.size(1), x.size(2), x.size(3),
+                       mask.size(0), mask.size(2), scale, p, seed, offset, code, on.stream));
+  }
+  return wrap_all({out, stats}, true);
+}
+
+void check_dropout_operands(const Tensor &dy, const Tensor &x, const Tensor &stats) {
+  check_input(dy, "output_grads");
+  check_input(x, "input");
+  check_input(stats, "stats");
+  TORCH_CHECK(dy.scalar_type() == x.scalar_type() && dy.sizes() == x.sizes(),
+              "output_grads and input differ in dtype or shape");
+  TORCH_CHECK(stats.scalar_type() == at::kFloat && stats.numel() == 2 * row_count(x),
+              "stats must be float32 [rows, 2]");
+}
+
+// (output_grads, input, stats, mask, scale, p, seed, offset, inplace, causal) -> grad_input
+PyObject *dropout_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &x = g.tensor();
+  const Tensor &stats = g.tensor();
+  const Tensor mask = g.optional();
+  const float scale = (float)g.real(), p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool inplace = g.flag(), causal = g.flag();
+  check_dropout_operands(dy, x, stats);
+  if (mask.defined()) check_mask_dims(x, mask);
+  else TORCH_CHECK(x.dim() == 3, "expected 3D tensor");
+  const int code = dtype_code(x, "input");
+  Tensor dx;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Tensor m = mask.defined() ? mask_bytes(mask, x) : Tensor();
+    dx = inplace ? dy : softmax_out(dy, 2);
+    const float *st = stats.data_ptr<float>();
+    check_rc(!mask.defined()
+                 ? oslo_softmax_causal_dropout_bwd(ptr(dy), ptr(x), st, ptr(dx), x.size(0), x.size(1), x.size(2),
+                                                   scale, p, seed, offset, code, on.stream)
+                 : (causal ? oslo_softmax_causal_masked_dropout_bwd : oslo_softmax_masked_dropout_bwd)(
+                       ptr(dy), ptr(x), (const uint8_t *)ptr(m), st, ptr(dx), x.size(0), x.size(1), x.size(2),
+                       x.size(3), mask.size(0), mask.size(2), scale, p, seed, offset, code, on.stream));
+  }
+  return wrap(dx);
+}
+
+// The additive term as the kernel addresses it: four dimensions, its strides
+// along batch, heads and queries (0 = broadcast; expanded views have it), the
+// keys contiguous, the input's dtype or fp32.
+struct Term {
+  Tensor t;
+  int64_t sb, sh, sq;
+  int code;
+  Term(const Tensor &term, const Tensor &x) : t(term) {
+    while (t.dim() < 4) t = t.unsqueeze(0);
+    const int64_t sk = x.size(3);
+    if (t.size(3) != sk) t = t.expand({-1, -1, -1, sk}).contiguous();
+    if (t.scalar_type() != x.scalar_type() && t.scalar_type() != at::kFloat) t = t.to(at::kFloat);
+    if (sk > 1 && t.stride(3) != 1) t = t.contiguous();
+    const auto stride = [&](int64_t d) { return t.size(d) == 1 ? 0 : t.stride(d); };
+    sb = stride(0), sh = stride(1), sq = stride(2);
+    code = dtype_code(t, "the additive term");
+  }
+  static void check(const Tensor &t, const Tensor &x) {
+    TORCH_CHECK(x.dim() == 4, "expected 4D tensor");
+    TORCH_CHECK(t.is_floating_point(), "the additive term must be a floating-point tensor");
+    TORCH_CHECK(t.device() == x.device(), "the additive term is on ", t.device().str(),
+                " but the softmax operand is on ", x.device().str());
+    TORCH_CHECK(t.dim() <= 4, "the additive term has more than four dimensions");
+    bool fits = true;
+    for (int64_t d = 0; d < t.dim(); ++d) fits &= t.size(d) == 1 || t.size(d) == x.size(d + 4 - t.dim());
+    TORCH_CHECK(fits, "additive term of size ", t.sizes(), " does not broadcast to ", x.sizes());
+  }
+};
+
+// `skip` -1 is the default: the test for hidden keys in the backward passes
+// only, and there only where the term is small next to the logits (shared by
+// the heads or by the queries), where a hidden chunk saves two loads.  (Waiting
+// for the term before the logits are requested costs a forward pass more than
+// the unread logits save: [16, 16, 1024, 1024] fp16 with 48 % of the keys under
+// -inf 159 us with the test, 163 without; with a -10000 mask, which hides
+// nothing, 190-210 against 163.)
+int term_flags(bool causal, int skip, int64_t sh, int64_t sq, bool forward) {
+  const bool test = skip < 0 ? !forward && (sh == 0 || sq == 0) : skip != 0;
+  return (causal ? OSLO_SOFTMAX_CAUSAL : 0) | (test ? OSLO_SOFTMAX_SKIP_HIDDEN : 0);
+}
+
+// (bias, input) -> (term, stride_b, stride_h, stride_q, dtype code)
+PyObject *bias_operand(Args &g) {
+  const Tensor &bias = g.tensor();
+  const Tensor &x = g.tensor();
+  Term::check(bias, x);
+  const Term t(bias, x);
+  PyObject *o = THPVariable_Wrap(t.t);
+  if (o == nullptr) throw python_error();
+  return Py_BuildValue("NLLLi", o, (long long)t.sb, (long long)t.sh, (long long)t.sq, t.code);
+}
+
+// (causal, skip_hidden, stride_h, stride_q, forward) -> flags
+PyObject *bias_flags(Args &g) {
+  const bool causal = g.flag();
+  const int skip = g.tristate();
+  const int64_t sh = g.integer(), sq = g.integer();
+  return PyLong_FromLong(term_flags(causal, skip, sh, sq, g.flag()));
+}
+
+// (input, bias, scale, causal, skip_hidden) -> out
+PyObject *bias_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor &bias = g.tensor();
+  const float scale = (float)g.real();
+  const bool causal = g.flag();
+  const int skip = g.tristate();
+  check_input(x, "input");
+  Term::check(bias, x);
+  const int code = dtype_code(x, "input");
+  Tensor out;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Term t(bias, x);
+    const int flags = term_flags(causal, skip, t.sh, t.sq, true);
+    out = softmax_out(x, 1);
+    check_rc(oslo_softmax_bias_fwd(ptr(x), ptr(t.t), ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), t.sb,
+                                   t.sh, t.sq, t.code, flags, scale, code, on.stream));
+  }
+  return wrap(out);
+}
+
+// (output_grads, softmax_results, scale, bias, causal, skip_hidden, inplace) -> grad_input
+PyObject *bias_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &y = g.tensor();
+  const float scale = (float)g.real();
+  const Tensor bias = g.optional();
+  const bool causal = g.flag();
+  const int skip = g.tristate();
+  const bool inplace = g.flag();
+  TORCH_CHECK(dy.dim() == 4 && y.dim() == 4, "expected 4D tensor");
+  check_same(dy, "output_grads", y, "softmax_results");
+  const int code = dtype_code(y, "softmax_results");
+  if (bias.defined()) Term::check(bias, y);
+  Tensor dx;
+  {
+    NoGil nogil;
+    const OnDevice on(dy);
+    std::optional<Term> t;
+    int flags = causal ? OSLO_SOFTMAX_CAUSAL : 0;
+    if (bias.defined()) {
+      t.emplace(bias, y);
+      flags = term_flags(causal, skip, t->sh, t->sq, false);
+      if (!(flags & OSLO_SOFTMAX_SKIP_HIDDEN)) t.reset();  // (only the test reads the term)
+    }
+    dx = inplace ? dy : softmax_out(dy, 2);
+    check_rc(oslo_softmax_bias_bwd(ptr(dy), ptr(y), t ? ptr(t->t) : nullptr, ptr(dx), y.size(0), y.size(1),
+                                   y.size(2), y.size(3), t ? t->sb : 0, t ? t->sh : 0, t ? t->sq : 0,
+                                   t ? t->code : code, flags, scale, code,
+                                   on.stream));
+  }
+  return wrap(dx);
+}
+
+// (input, bias, scale, p, seed, offset, causal, skip_hidden) -> [out, stats]
+PyObject *bias_dropout_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor &bias = g.tensor();
+  const float scale = (float)g.real(), p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool causal = g.flag();
+  const int skip = g.tristate();
+  check_input(x, "input");
+  Term::check(bias, x);
+  const int code = dtype_code(x, "input");
+  Tensor out, stats;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Term t(bias, x);
+    const int flags = term_flags(causal, skip, t.sh, t.sq, true);
+    out = softmax_out(x, 1);
+    stats = new_f32(x, {x.size(0) * x.size(1) * x.size(2), 2});
+    check_rc(oslo_softmax_bias_dropout_fwd(ptr(x), ptr(t.t), ptr(out), stats.data_ptr<float>(), x.size(0), x.size(1),
+                                           x.size(2), x.size(3), t.sb, t.sh, t.sq, t.code, flags, scale, p, seed,
+                                           offset, code, on.stream));
+  }
+  return wrap_all({out, stats}, true);
+}
+
+// (output_grads, input, bias, stats, scale, p, seed, offset, causal, skip_hidden, inplace) -> grad_input
+PyObject *bias_dropout_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &x = g.tensor();
+  const Tensor &bias = g.tensor();
+  const Tensor &stats = g.tensor();
+  const float scale = (float)g.real(), p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool causal = g.flag();
+  const int skip = g.tristate();
+  const bool inplace = g.flag();
+  check_input(dy, "output_grads");
+  check_input(x, "input");
+  check_input(stats, "stats");
+  TORCH_CHECK(dy.scalar_type() == x.scalar_type() && dy.sizes() == x.sizes(),
+              "output_grads and input differ in dtype or shape");
+  Term::check(bias, x);
+  TORCH_CHECK(stats.scalar_type() == at::kFloat && stats.numel() == 2 * x.size(0) * x.size(1) * x.size(2),
+              "stats must be float32 [rows, 2]");
+  const int code = dtype_code(x, "input");
+  Tensor dx;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    const Term t(bias, x);
+    const int flags = term_flags(causal, skip, t.sh, t.sq, false);
+    dx = inplace ? dy : softmax_out(dy, 2);
+    check_rc(oslo_softmax_bias_dropout_bwd(ptr(dy), ptr(x), ptr(t.t), stats.data_ptr<float>(), ptr(dx), x.size(0),
+                                           x.size(1), x.size(2), x.size(3), t.sb, t.sh, t.sq, t.code, flags, scale,
+                                           p, seed, offset, code, on.stream));
+  }
+  return wrap(dx);
+}
+
+// ---------------------------------------------------------------- element-wise
+void rows_and_cols(const Tensor &x, const Tensor &bias, int64_t &rows, int64_t &cols) {
+  cols = x.dim() > 0 ? x.size(-1) : 1;
+  if (bias.defined())
+    TORCH_CHECK(bias.dim() == 1 && bias.size(0) == cols, "bias of size ", bias.sizes(),
+                " does not match the last dimension of input of size ", x.sizes());
+  rows = cols > 0 ? x.numel() / cols : 0;
+}
+
+void check_bias(const Tensor &bias, const Tensor &x) {
+  if (!bias.defined()) return;
+  check_input(bias, "bias");
+  TORCH_CHECK(bias.scalar_type() == x.scalar_type(), "bias and input differ in dtype");
+}
+
+// (input, bias) -> out
+PyObject *gelu_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor bias = g.optional();
+  check_input(x, "input");
+  check_bias(bias, x);
+  int64_t rows, cols;
+  rows_and_cols(x, bias, rows, cols);
+  const int code = dtype_code(x, "input");
+  Tensor out;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    out = at::empty(x.sizes(), x.options());
+    check_rc(oslo_bias_gelu_fwd(ptr(x), ptr(bias), ptr(out), rows, cols, code, on.stream));
+  }
+  return wrap(out);
+}
+
+// (grad_output, input, bias, need_bias_grad, workspace, nbytes) -> (grad_input, grad_bias)
+PyObject *gelu_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const Tensor &x = g.tensor();
+  const Tensor bias = g.optional();
+  const bool want_bias = g.flag();
+  const Tensor ws = g.optional();
+  const int64_t nbytes = g.integer();
+  check_input(dy, "grad_output");
+  check_input(x, "input");
+  TORCH_CHECK(dy.scalar_type() == x.scalar_type() && dy.sizes() == x.sizes(), "grad_output does not match input");
+  check_bias(bias, x);
+  int64_t rows, cols;
+  rows_and_cols(x, bias, rows, cols);
+  const int code = dtype_code(x, "input");
+  Tensor dx, db;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    dx = at::empty(x.sizes(), x.options());
+    if (bias.defined() && want_bias) db = at::empty_like(bias);
+    check_rc(oslo_bias_gelu_bwd(ptr(dy), ptr(x), ptr(bias), ptr(dx), ptr(db), ptr(ws), nbytes, rows, cols, code,
+                                on.stream));
+  }
+  return wrap_all({dx, db}, false);
+}
+
+// (input, bias, residual, p, seed, offset, out, return_mask) -> (out, mask or None)
+PyObject *dropout_add_forward(Args &g) {
+  const Tensor &x = g.tensor();
+  const Tensor bias = g.optional(), res = g.optional();
+  const float p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  Tensor out = g.optional();
+  const bool want_mask = g.flag();
+  check_input(x, "input");
+  check_bias(bias, x);
+  if (res.defined()) {
+    check_input(res, "residual");
+    TORCH_CHECK(res.scalar_type() == x.scalar_type(), "residual and input differ in dtype");
+    TORCH_CHECK(res.sizes() == x.sizes(), "residual does not match input");
+  }
+  int64_t rows, cols;
+  rows_and_cols(x, bias, rows, cols);
+  const int code = dtype_code(x, "input");
+  Tensor mask;
+  {
+    NoGil nogil;
+    const OnDevice on(x);
+    if (!out.defined()) out = at::empty(x.sizes(), x.options());
+    if (want_mask) mask = at::empty(x.sizes(), x.options().dtype(at::kByte));
+    check_rc(oslo_bias_dropout_add_fwd(ptr(x), ptr(bias), ptr(res), ptr(out), (uint8_t *)ptr(mask), rows, cols, p,
+                                       seed, offset, code, on.stream));
+  }
+  return wrap_all({out, mask}, false);
+}
+
+// (grad_output, p, seed, offset, need_input_grad, need_bias_grad, workspace, nbytes)
+// -> (grad_input, grad_bias)
+PyObject *dropout_add_backward(Args &g) {
+  const Tensor &dy = g.tensor();
+  const float p = (float)g.real();
+  const uint64_t seed = g.word(), offset = g.word();
+  const bool want_input = g.flag(), want_bias = g.flag();
+  const Tensor ws = g.optional();
+  const int64_t nbytes = g.integer();
+  check_input(dy, "grad_output");
+  int64_t rows, cols;
+  rows_and_cols(dy, Tensor(), rows, cols);
+  Tensor dx, db;
+  if (want_input || want_bias) {
+    const int code = dtype_code(dy, "grad_output");
+    NoGil nogil;
+    const OnDevice on(dy);
+    if (want_input) dx = at::empty(dy.sizes(), dy.options());
+    if (want_bias) db = at::empty({cols}, dy.options());
+    check_rc(oslo_bias_dropout_add_bwd(ptr(dy), ptr(dx), ptr(db), ptr(ws), nbytes, rows, cols, p, seed, offset, code,
+                                       on.stream));
+  }
+  return wrap_all({dx, db}, false);
+}
+
+// ---------------------------------------------------------------- module
+template <PyObject *(*F)(Args &)>
+PyObject *entry(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args args{a, n};
+  return F(args);
+  END_HANDLE_TH_ERRORS
+}
+
+#define OSLO_METHOD(F) {#F, (PyCFunction)(void (*)(void))entry<F>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    OSLO_METHOD(norm_forward),
+    OSLO_METHOD(norm_backward),
+    OSLO_METHOD(residual_norm_forward),
+    OSLO_METHOD(residual_norm_backward),
+    OSLO_METHOD(causal_forward),
+    OSLO_METHOD(causal_backward),
+    OSLO_METHOD(masked_forward),
+    OSLO_METHOD(masked_backward),
+    OSLO_METHOD(dropout_forward),
+    OSLO_METHOD(dropout_backward),
+    OSLO_METHOD(bias_operand),
+    OSLO_METHOD(bias_flags),
+    OSLO_METHOD(bias_forward),
+    OSLO_METHOD(bias_backward),
+    OSLO_METHOD(bias_dropout_forward),
+    OSLO_METHOD(bias_dropout_backward),
+    OSLO_METHOD(gelu_forward),
+    OSLO_METHOD(gelu_backward),
+    OSLO_METHOD(dropout_add_forward),
+    OSLO_METHOD(dropout_add_backward),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "oslo_torch_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_oslo_torch_calls() { return PyModule_Create(&module); }

@@ -7,15 +7,20 @@ there) whose methods have the signatures of the reference's pybind modules
 Instead of JIT-compiling CUDA through ``torch.utils.cpp_extension`` the shared
 library is built ahead of time by ``hipcc`` for gfx950 and bound with ctypes;
 tensors cross the boundary as raw device pointers and every output and
-workspace is allocated here, by torch's caching allocator.
+workspace is allocated on this side, by torch's caching allocator.  The methods
+of the layer ops do that in native code (``csrc/torch_calls.cpp``: checks,
+allocation, launch): in Python they cost three times the launch itself.
 
 A missing or unloadable library raises ``EnvironmentError`` (the reference's
 exception type, ``_C/__init__.py:200-204``); there is no fallback for GPU
 tensors.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import subprocess
+import sys
 import threading
 
 import torch
@@ -24,6 +29,7 @@ _CSRC_DIR = os.path.normpath(
     os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "..", "csrc")
 )
 LIBRARY_PATH = os.path.join(_CSRC_DIR, "liboslo_hip.so")
+CALLS_PATH = os.path.join(_CSRC_DIR, "oslo_torch_calls.so")
 
 OSLO_OP_LN_BWD = 1
 OSLO_OP_RMS_BWD = 2
@@ -38,6 +44,7 @@ OSLO_DTYPE_F64 = 3  # LayerNorm / RMSNorm only
 OSLO_LN_BWD_STATIC_SCRATCH_BYTES = 16 * 1024 * 1024
 
 _lib = None
+_calls = None
 _lib_lock = threading.Lock()
 
 _p = ctypes.c_void_p
@@ -200,8 +207,9 @@ EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 
 def build_library(force=False):
-    """Compiles ``liboslo_hip.so`` in place with hipcc (``make`` in ``csrc``)."""
-    cmd = ["make", "-C", _CSRC_DIR, "-j8"]
+    """Compiles ``liboslo_hip.so`` and the native side of this module in place
+    with hipcc (``make`` in ``csrc``)."""
+    cmd = ["make", "-C", _CSRC_DIR, "-j8", "PYTHON=" + sys.executable]
     if force:
         subprocess.run(["make", "-C", _CSRC_DIR, "clean"], check=True,
                        stdout=subprocess.DEVNULL)
@@ -244,6 +252,31 @@ def load_library():
     return _lib
 
 
+def load_calls():
+    """Returns the extension module with the native side of the kernel objects."""
+    global _calls
+    if _calls is not None:
+        return _calls
+    load_library()
+    with _lib_lock:
+        if _calls is not None:
+            return _calls
+        if not os.path.exists(CALLS_PATH):
+            build_library()
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("oslo_torch_calls", CALLS_PATH)
+            module = importlib.util.module_from_spec(
+                importlib.util.spec_from_loader("oslo_torch_calls", loader))
+            loader.exec_module(module)
+        except (ImportError, OSError) as exc:
+            raise EnvironmentError(
+                "Failed loading the HIP kernels (%s): %s. Rebuild with "
+                "`make -C %s`." % (CALLS_PATH, exc, _CSRC_DIR)
+            ) from exc
+        _calls = module
+    return _calls
+
+
 def _check(rc, lib):
     if rc != 0:
         raise RuntimeError(lib.oslo_hip_last_error().decode("utf-8", "replace"))
@@ -282,23 +315,15 @@ def _device_of(t):
     return torch.cuda.device_of(t)
 
 
-def _dtype_code(t, what, allow_f64=False):
-    if allow_f64 and t.dtype == torch.float64:
-        return OSLO_DTYPE_F64
+def _dtype_code(t, what):
     try:
         return _DTYPE_CODE[t.dtype]
     except KeyError:
         raise RuntimeError(
             "%s: dtype %s is not supported by the HIP kernels "
-            "(float32, float16 and bfloat16 are%s)"
-            % (what, t.dtype, "" if allow_f64 else "; float64 only by the norms")
+            "(float32, float16 and bfloat16 are; float64 only by the norms)"
+            % (what, t.dtype)
         ) from None
-
-
-def _stat_dtype(t):
-    # FusedLayerNormBinder.cpp:146-152: the statistics are fp32 for 16-bit
-    # inputs and have the input's type otherwise
-    return torch.float64 if t.dtype == torch.float64 else torch.float32
 
 
 def _check_input(t, name):
@@ -409,6 +434,14 @@ def _workspace(lib, op, n1, n2, device):
     return _ws_cache.lease(index, stream, op, nbytes)
 
 
+def _norm_workspace(lib, op, input, normalized_shape):
+    """Lease for a norm backward; the native call refuses what is not on the GPU."""
+    if not input.is_cuda:
+        return _NO_WORKSPACE
+    n1, n2 = _compute_n1_n2(input, normalized_shape)
+    return _workspace(lib, op, n1, n2, input.device)
+
+
 class device_rng:
     """Within the block, the dropout entry points called on this host thread
     read (seed, offset) from ``state`` -- two 64-bit integers in device memory --
@@ -476,129 +509,43 @@ def _compute_n1_n2(input, normalized_shape):
     return n1, n2
 
 
-def _check_param(p, normalized_shape, name):
-    if p is not None and tuple(p.shape) != tuple(int(s) for s in normalized_shape):
-        raise RuntimeError(
-            "%s of shape %s does not match normalized_shape=%s"
-            % (name, list(p.shape), list(normalized_shape))
-        )
-
-
 class _LayerNormKernel:
     """The ten functions of the reference's ``oslo_fused_layer_norm`` module."""
 
     def __init__(self, lib):
         self._lib = lib
+        self._calls = load_calls()
 
     # -- forward ----------------------------------------------------------
-    def _forward(self, rms, input, normalized_shape, gamma, beta, eps, out_dtype):
-        lib = self._lib
-        _check_input(input, "input")
-        n1, n2 = _compute_n1_n2(input, normalized_shape)
-        if gamma is not None:
-            _check_param(gamma, normalized_shape, "gamma")
-            _check_param(beta, normalized_shape, "beta")
-        din = _dtype_code(input, "input", allow_f64=True)
-        output = torch.empty_like(input, dtype=out_dtype)
-        dout = _dtype_code(output, "output", allow_f64=True)
-        for name, t in (("gamma", gamma), ("beta", beta)):
-            if t is not None:
-                _check_input(t, name)
-                if t.dtype != out_dtype:
-                    raise RuntimeError(
-                        "%s has dtype %s but the output dtype is %s"
-                        % (name, t.dtype, out_dtype)
-                    )
-        invvar = torch.empty(n1, dtype=_stat_dtype(input), device=input.device)
-        with _device_of(input):
-            if rms:
-                rc = lib.oslo_rms_fwd(
-                    _ptr(input), _ptr(gamma), _ptr(output), _ptr(invvar),
-                    n1, n2, float(eps), din, dout, _stream(input),
-                )
-                _check(rc, lib)
-                return [output, invvar]
-            mean = torch.empty(n1, dtype=_stat_dtype(input), device=input.device)
-            rc = lib.oslo_ln_fwd(
-                _ptr(input), _ptr(gamma), _ptr(beta), _ptr(output), _ptr(mean),
-                _ptr(invvar), n1, n2, float(eps), din, dout, _stream(input),
-            )
-            _check(rc, lib)
-        return [output, mean, invvar]
-
     def layer_norm_forward(self, input, normalized_shape, eps):
-        return self._forward(False, input, normalized_shape, None, None, eps, input.dtype)
+        return self._calls.norm_forward(False, input, normalized_shape, None, None, eps, False)
 
     def layer_norm_forward_affine(self, input, normalized_shape, gamma, beta, eps):
-        return self._forward(False, input, normalized_shape, gamma, beta, eps, input.dtype)
+        return self._calls.norm_forward(False, input, normalized_shape, gamma, beta, eps, False)
 
     def layer_norm_forward_affine_mixed_dtypes(self, input, normalized_shape, gamma, beta, eps):
-        return self._forward(False, input, normalized_shape, gamma, beta, eps, gamma.dtype)
+        return self._calls.norm_forward(False, input, normalized_shape, gamma, beta, eps, True)
 
     def rms_norm_forward(self, input, normalized_shape, eps):
-        return self._forward(True, input, normalized_shape, None, None, eps, input.dtype)
+        return self._calls.norm_forward(True, input, normalized_shape, None, None, eps, False)
 
     def rms_norm_forward_affine(self, input, normalized_shape, gamma, eps):
-        return self._forward(True, input, normalized_shape, gamma, None, eps, input.dtype)
+        return self._calls.norm_forward(True, input, normalized_shape, gamma, None, eps, False)
 
     def rms_norm_forward_affine_mixed_dtypes(self, input, normalized_shape, gamma, eps):
-        return self._forward(True, input, normalized_shape, gamma, None, eps, gamma.dtype)
+        return self._calls.norm_forward(True, input, normalized_shape, gamma, None, eps, True)
 
     # -- backward ---------------------------------------------------------
     def _backward(self, rms, dout, mean, invvar, input, normalized_shape, gamma, beta):
-        lib = self._lib
-        for name, t in (("dout", dout), ("invvar", invvar), ("input", input)):
-            _check_input(t, name)
-        if not rms:
-            _check_input(mean, "mean")
-        n1, n2 = _compute_n1_n2(input, normalized_shape)
-        if dout.shape != input.shape:
-            raise RuntimeError(
-                "dout of size %s does not match input of size %s"
-                % (list(dout.shape), list(input.shape))
-            )
-        din = _dtype_code(input, "input", allow_f64=True)
-        dcode = _dtype_code(dout, "dout", allow_f64=True)
-        for name, t in (("invvar", invvar), ("mean", mean)):
-            if t is not None and t.dtype != _stat_dtype(input):
-                raise RuntimeError(
-                    "%s has dtype %s, expected %s" % (name, t.dtype, _stat_dtype(input))
-                )
-            if t is not None and t.numel() != n1:
-                raise RuntimeError(
-                    "%s has %d elements for %d rows of input" % (name, t.numel(), n1)
-                )
-        grad_input = torch.empty_like(input)
-        grad_gamma = grad_beta = None
         lease = _NO_WORKSPACE
         if gamma is not None:
-            _check_input(gamma, "gamma")
-            _check_param(gamma, normalized_shape, "gamma")
-            if gamma.dtype != dout.dtype:
-                raise RuntimeError(
-                    "gamma has dtype %s but dout has dtype %s" % (gamma.dtype, dout.dtype)
-                )
-            grad_gamma = torch.empty_like(gamma)
-            if not rms:
-                grad_beta = torch.empty_like(beta if beta is not None else gamma)
-            lease = _workspace(
-                lib, OSLO_OP_RMS_BWD if rms else OSLO_OP_LN_BWD, n1, n2, input.device
+            op = OSLO_OP_RMS_BWD if rms else OSLO_OP_LN_BWD
+            lease = _norm_workspace(self._lib, op, input, normalized_shape)
+        with lease as ws:
+            return self._calls.norm_backward(
+                rms, dout, mean, invvar, input, normalized_shape, gamma, beta,
+                ws.tensor, ws.nbytes,
             )
-        with _device_of(input), lease as ws:
-            if rms:
-                rc = lib.oslo_rms_bwd(
-                    _ptr(dout), _ptr(input), _ptr(invvar), _ptr(gamma), _ptr(grad_input),
-                    _ptr(grad_gamma), _ptr(ws.tensor), ws.nbytes, n1, n2, din, dcode,
-                    _stream(input),
-                )
-            else:
-                rc = lib.oslo_ln_bwd(
-                    _ptr(dout), _ptr(input), _ptr(mean), _ptr(invvar), _ptr(gamma),
-                    _ptr(grad_input), _ptr(grad_gamma), _ptr(grad_beta), _ptr(ws.tensor),
-                    ws.nbytes, n1, n2, din, dcode, _stream(input),
-                )
-            _check(rc, lib)
-        return grad_input, grad_gamma, grad_beta
 
     def layer_norm_backward(self, dout, mean, invvar, input, normalized_shape, eps):
         return self._backward(False, dout, mean, invvar, input, normalized_shape, None, None)[0]
@@ -632,35 +579,9 @@ class _LayerNormKernel:
         Returns ``[y, h, mean, invvar]`` (``h`` None when ``want_h`` is false,
         ``mean`` None for RMSNorm).  One dtype throughout.
         """
-        lib = self._lib
-        _check_input(input, "input")
-        n1, n2 = _compute_n1_n2(input, normalized_shape)
-        for name, t in (("gamma", gamma), ("beta", beta), ("bias", bias)):
-            if t is not None:
-                _check_input(t, name)
-                _check_param(t, normalized_shape, name)
-        if residual is not None:
-            _check_input(residual, "residual")
-            if residual.shape != input.shape:
-                raise RuntimeError("residual and input differ in shape")
-        for name, t in (("gamma", gamma), ("beta", beta), ("bias", bias), ("residual", residual)):
-            if t is not None and t.dtype != input.dtype:
-                raise RuntimeError(
-                    "%s has dtype %s but input has dtype %s" % (name, t.dtype, input.dtype)
-                )
-        code = _dtype_code(input, "input")
-        y = torch.empty_like(input)
-        h = torch.empty_like(input) if want_h else None
-        invvar = torch.empty(n1, dtype=torch.float32, device=input.device)
-        mean = None if rms else torch.empty(n1, dtype=torch.float32, device=input.device)
-        with _device_of(input):
-            rc = lib.oslo_bias_dropout_add_norm_fwd(
-                _ptr(input), _ptr(bias), _ptr(residual), _ptr(gamma), _ptr(beta), _ptr(h),
-                _ptr(y), _ptr(mean), _ptr(invvar), n1, n2, float(eps), float(p),
-                int(seed), int(offset), 1 if rms else 0, code, _stream(input),
-            )
-            _check(rc, lib)
-        return [y, h, mean, invvar]
+        return self._calls.residual_norm_forward(
+            rms, input, bias, residual, normalized_shape, gamma, beta, eps, p, seed, offset, want_h
+        )
 
     def bias_dropout_add_norm_backward(
         self, rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma,
@@ -668,53 +589,16 @@ class _LayerNormKernel:
     ):
         """Returns ``(grad_residual, grad_input, grad_gamma, grad_beta, grad_bias)``;
         ``grad_input`` is ``grad_residual`` itself when ``p == 0``."""
-        lib = self._lib
-        for name, t in (("dout", dout), ("h", h), ("invvar", invvar)):
-            _check_input(t, name)
-        n1, n2 = _compute_n1_n2(h, normalized_shape)
-        if dout.shape != h.shape or dout.dtype != h.dtype:
-            raise RuntimeError("dout and h differ in shape or dtype")
-        if not rms:
-            _check_input(mean, "mean")
-        for name, t in (("invvar", invvar), ("mean", None if rms else mean)):
-            if t is not None and (t.dtype != torch.float32 or t.numel() != n1):
-                raise RuntimeError("%s must be float32 with one element per row of h" % name)
-        if dh_extra is not None:
-            _check_input(dh_extra, "dh_extra")
-            if dh_extra.shape != h.shape or dh_extra.dtype != h.dtype:
-                raise RuntimeError("dh_extra and h differ in shape or dtype")
-        code = _dtype_code(h, "h")
-        grad_res = torch.empty_like(h)
-        grad_in = torch.empty_like(h) if p > 0.0 else None
-        grad_gamma = grad_beta = grad_bias = None
-        if gamma is not None:
-            _check_input(gamma, "gamma")
-            _check_param(gamma, normalized_shape, "gamma")
-            if gamma.dtype != h.dtype:
-                raise RuntimeError(
-                    "gamma has dtype %s but h has dtype %s" % (gamma.dtype, h.dtype)
-                )
-            grad_gamma = torch.empty_like(gamma)
-            if not rms:
-                grad_beta = torch.empty_like(gamma)
-        if need_bias_grad:
-            grad_bias = torch.empty(n2, dtype=h.dtype, device=h.device)
         lease = _NO_WORKSPACE
         if gamma is not None or need_bias_grad:
-            lease = _workspace(lib, OSLO_OP_BIAS_DROPOUT_ADD_NORM_BWD, n1, n2, h.device)
-        with _device_of(h), lease as ws:
-            rc = lib.oslo_bias_dropout_add_norm_bwd(
-                _ptr(dout), _ptr(dh_extra), _ptr(h), _ptr(mean), _ptr(invvar), _ptr(gamma),
-                _ptr(grad_res), _ptr(grad_in), _ptr(grad_gamma), _ptr(grad_beta),
-                _ptr(grad_bias), _ptr(ws.tensor), ws.nbytes, n1, n2, float(p), int(seed),
-                int(offset), 1 if rms else 0, code, _stream(h),
+            lease = _norm_workspace(
+                self._lib, OSLO_OP_BIAS_DROPOUT_ADD_NORM_BWD, h, normalized_shape
             )
-            _check(rc, lib)
-        if grad_in is None:
-            grad_in = grad_res
-        if grad_bias is not None:
-            grad_bias = grad_bias.view(tuple(int(s) for s in normalized_shape))
-        return grad_res, grad_in, grad_gamma, grad_beta, grad_bias
+        with lease as ws:
+            return self._calls.residual_norm_backward(
+                rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma, p, seed, offset,
+                need_bias_grad, ws.tensor, ws.nbytes,
+            )
 
 
 # ---------------------------------------------------------------------------
@@ -749,10 +633,6 @@ def empty_staggered(shape, dtype, device, k):
     return base[off:off + nbytes].view(dtype).view(tuple(shape))
 
 
-def _softmax_out(like, k):
-    return empty_staggered(like.shape, like.dtype, like.device, k)
-
-
 class _SoftmaxKernel:
     """The five functions of ``FusedScaleMaskSoftmaxBinder.cpp:111-127``.
 
@@ -764,69 +644,22 @@ class _SoftmaxKernel:
 
     def __init__(self, lib):
         self._lib = lib
-
-    @staticmethod
-    def _mask_u8(mask, like):
-        """The mask as contiguous bytes (non-zero = masked out); it has to live
-        on the device of ``like``, since the kernel reads it through a raw pointer."""
-        if mask.device != like.device:
-            raise RuntimeError(
-                "mask is on %s but the softmax operand is on %s" % (mask.device, like.device)
-            )
-        if mask.dtype == torch.bool:
-            return mask.contiguous().view(torch.uint8)
-        if mask.dtype == torch.uint8:
-            return mask.contiguous()
-        return (mask != 0).contiguous().view(torch.uint8)
+        self._calls = load_calls()
 
     def fused_scaled_masked_softmax_forward(self, input, mask, scale_factor, causal=False):
         """``causal=True`` (not in the reference's shim) hides the keys beyond
         the diagonal as well: causal attention on a padded batch."""
-        lib = self._lib
-        b, np_, sq, sk, mb, msq = self._masked_dims(input, mask)
-        _check_input(input, "input")
-        m8 = self._mask_u8(mask, input)
-        out = _softmax_out(input, 1)
-        with _device_of(input):
-            fn = lib.oslo_softmax_causal_masked_fwd if causal else lib.oslo_softmax_masked_fwd
-            rc = fn(
-                _ptr(input), _ptr(m8), _ptr(out), b, np_, sq, sk, mb, msq,
-                float(scale_factor), _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return out
+        return self._calls.masked_forward(input, mask, scale_factor, causal)
 
     def fused_scaled_masked_softmax_backward(
         self, output_grads, softmax_results, scale_factor, mask=None, inplace=False,
         causal=False,
     ):
-        lib = self._lib
-        if output_grads.dim() != 4 or softmax_results.dim() != 4:
-            raise RuntimeError("expected 4D tensor")
-        _check_input(output_grads, "output_grads")
-        _check_input(softmax_results, "softmax_results")
-        if output_grads.dtype != softmax_results.dtype:
-            raise RuntimeError("output_grads and softmax_results differ in dtype")
-        if output_grads.shape != softmax_results.shape:
-            raise RuntimeError("output_grads and softmax_results differ in shape")
-        b, np_, sq, sk = softmax_results.shape
-        mb = msq = 1
-        m8 = None
-        if mask is not None:
-            _, _, _, _, mb, msq = self._masked_dims(softmax_results, mask)
-            m8 = self._mask_u8(mask, softmax_results)
         # inplace=True overwrites output_grads, as the kernel this shim was
         # written for does
-        grad_input = output_grads if inplace else _softmax_out(output_grads, 2)
-        with _device_of(output_grads):
-            fn = lib.oslo_softmax_causal_masked_bwd if causal else lib.oslo_softmax_masked_bwd
-            rc = fn(
-                _ptr(output_grads), _ptr(softmax_results), _ptr(m8), _ptr(grad_input),
-                b, np_, sq, sk, mb, msq, float(scale_factor),
-                _dtype_code(output_grads, "output_grads"), _stream(output_grads),
-            )
-            _check(rc, lib)
-        return grad_input
+        return self._calls.masked_backward(
+            output_grads, softmax_results, scale_factor, mask, inplace, causal
+        )
 
     def get_batch_per_block(self, query_seq_len, key_seq_len, batches, attn_heads):
         lib = self._lib
@@ -838,58 +671,16 @@ class _SoftmaxKernel:
         return int(rc)
 
     def fused_scaled_upper_triang_masked_softmax_forward(self, input, scale_factor):
-        lib = self._lib
-        if input.dim() != 3:
-            raise RuntimeError("expected 3D tensor")
-        _check_input(input, "input")
-        ab, sq, sk = input.shape
-        out = _softmax_out(input, 1)
-        with _device_of(input):
-            rc = lib.oslo_softmax_causal_fwd(
-                _ptr(input), _ptr(out), ab, sq, sk, float(scale_factor),
-                _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return out
+        return self._calls.causal_forward(input, scale_factor)
 
     def fused_scaled_upper_triang_masked_softmax_backward(
         self, output_grads, softmax_results, scale_factor, inplace=False
     ):
-        lib = self._lib
-        if output_grads.dim() != 3 or softmax_results.dim() != 3:
-            raise RuntimeError("expected 3D tensor")
-        _check_input(output_grads, "output_grads")
-        _check_input(softmax_results, "softmax_results")
-        if output_grads.dtype != softmax_results.dtype:
-            raise RuntimeError("output_grads and softmax_results differ in dtype")
-        if output_grads.shape != softmax_results.shape:
-            raise RuntimeError("output_grads and softmax_results differ in shape")
-        ab, sq, sk = softmax_results.shape
-        grad_input = output_grads if inplace else _softmax_out(output_grads, 2)
-        with _device_of(output_grads):
-            rc = lib.oslo_softmax_causal_bwd(
-                _ptr(output_grads), _ptr(softmax_results), _ptr(grad_input), ab, sq, sk,
-                float(scale_factor), _dtype_code(output_grads, "output_grads"),
-                _stream(output_grads),
-            )
-            _check(rc, lib)
-        return grad_input
+        return self._calls.causal_backward(output_grads, softmax_results, scale_factor, inplace)
 
     # -- softmax with the attention dropout fused in (no counterpart in the
     #    reference's shim: the models apply nn.Dropout to the probabilities,
     #    oslo/transformers/models/gpt2/modeling_gpt2.py:138-142) -------------
-    def _masked_dims(self, input, mask):
-        if input.dim() != 4 or mask.dim() != 4:
-            raise RuntimeError("expected 4D tensor")
-        b, np_, sq, sk = input.shape
-        mb, mh, msq, msk = mask.shape
-        if mh != 1 or msk != sk or mb not in (1, b) or msq not in (1, sq):
-            raise RuntimeError(
-                "mask of size %s does not broadcast to [%d, 1, %d, %d]"
-                % (list(mask.shape), b, sq, sk)
-            )
-        return b, np_, sq, sk, mb, msq
-
     def softmax_dropout_forward(self, input, mask, scale_factor, p, seed, offset, causal=False):
         """``dropout(softmax(mask(scale * input)), p)`` -> ``[out, stats]``.
 
@@ -899,72 +690,17 @@ class _SoftmaxKernel:
         hidden as well).  ``stats`` (float32 ``[rows, 2]``) and ``input`` are
         what the backward pass needs.
         """
-        lib = self._lib
-        _check_input(input, "input")
-        out = _softmax_out(input, 1)
-        rows = input.numel() // input.shape[-1] if input.numel() else 0
-        stats = torch.empty((rows, 2), dtype=torch.float32, device=input.device)
-        with _device_of(input):
-            if mask is None:
-                if input.dim() != 3:
-                    raise RuntimeError("expected 3D tensor")
-                ab, sq, sk = input.shape
-                rc = lib.oslo_softmax_causal_dropout_fwd(
-                    _ptr(input), _ptr(out), _ptr(stats), ab, sq, sk,
-                    float(scale_factor), float(p), int(seed), int(offset),
-                    _dtype_code(input, "input"), _stream(input),
-                )
-            else:
-                b, np_, sq, sk, mb, msq = self._masked_dims(input, mask)
-                m8 = self._mask_u8(mask, input)
-                fn = (lib.oslo_softmax_causal_masked_dropout_fwd if causal
-                      else lib.oslo_softmax_masked_dropout_fwd)
-                rc = fn(
-                    _ptr(input), _ptr(m8), _ptr(out), _ptr(stats), b, np_, sq, sk,
-                    mb, msq, float(scale_factor), float(p), int(seed), int(offset),
-                    _dtype_code(input, "input"), _stream(input),
-                )
-            _check(rc, lib)
-        return [out, stats]
+        return self._calls.dropout_forward(
+            input, mask, scale_factor, p, seed, offset, causal
+        )
 
     def softmax_dropout_backward(
         self, output_grads, input, stats, mask, scale_factor, p, seed, offset,
         inplace=False, causal=False,
     ):
-        lib = self._lib
-        _check_input(output_grads, "output_grads")
-        _check_input(input, "input")
-        _check_input(stats, "stats")
-        if output_grads.dtype != input.dtype or output_grads.shape != input.shape:
-            raise RuntimeError("output_grads and input differ in dtype or shape")
-        rows = input.numel() // input.shape[-1] if input.numel() else 0
-        if stats.dtype != torch.float32 or stats.numel() != 2 * rows:
-            raise RuntimeError("stats must be float32 [rows, 2]")
-        grad_input = output_grads if inplace else _softmax_out(output_grads, 2)
-        with _device_of(input):
-            if mask is None:
-                if input.dim() != 3:
-                    raise RuntimeError("expected 3D tensor")
-                ab, sq, sk = input.shape
-                rc = lib.oslo_softmax_causal_dropout_bwd(
-                    _ptr(output_grads), _ptr(input), _ptr(stats), _ptr(grad_input),
-                    ab, sq, sk, float(scale_factor), float(p), int(seed), int(offset),
-                    _dtype_code(input, "input"), _stream(input),
-                )
-            else:
-                b, np_, sq, sk, mb, msq = self._masked_dims(input, mask)
-                m8 = self._mask_u8(mask, input)
-                fn = (lib.oslo_softmax_causal_masked_dropout_bwd if causal
-                      else lib.oslo_softmax_masked_dropout_bwd)
-                rc = fn(
-                    _ptr(output_grads), _ptr(input), _ptr(m8), _ptr(stats),
-                    _ptr(grad_input), b, np_, sq, sk, mb, msq, float(scale_factor),
-                    float(p), int(seed), int(offset), _dtype_code(input, "input"),
-                    _stream(input),
-                )
-            _check(rc, lib)
-        return grad_input
-
+        return self._calls.dropout_backward(
+            output_grads, input, stats, mask, scale_factor, p, seed, offset, inplace, causal
+        )
 
     # -- softmax with an additive floating-point term (no counterpart in the
     #    reference's shim; its models add the term to the scores with torch,
@@ -976,53 +712,11 @@ class _SoftmaxKernel:
         ``input``: up to four dimensions, each of the leading three either 1 or
         the full size (expanded views are fine: their stride is 0), the keys
         contiguous; its dtype becomes the input's or float32."""
-        if input.dim() != 4:
-            raise RuntimeError("expected 4D tensor")
-        if not bias.is_floating_point():
-            raise RuntimeError("the additive term must be a floating-point tensor")
-        if bias.device != input.device:
-            raise RuntimeError(
-                "the additive term is on %s but the softmax operand is on %s"
-                % (bias.device, input.device)
-            )
-        if bias.dim() > 4:
-            raise RuntimeError("the additive term has more than four dimensions")
-        while bias.dim() < 4:
-            bias = bias.unsqueeze(0)
-        b, np_, sq, sk = input.shape
-        for d, full in enumerate((b, np_, sq)):
-            if bias.size(d) not in (1, full):
-                raise RuntimeError(
-                    "additive term of size %s does not broadcast to %s"
-                    % (list(bias.shape), list(input.shape))
-                )
-        if bias.size(3) != sk:
-            if bias.size(3) != 1:
-                raise RuntimeError(
-                    "additive term of size %s does not broadcast to %s"
-                    % (list(bias.shape), list(input.shape))
-                )
-            bias = bias.expand(-1, -1, -1, sk).contiguous()
-        if bias.dtype != input.dtype and bias.dtype != torch.float32:
-            bias = bias.float()
-        if sk > 1 and bias.stride(3) != 1:
-            bias = bias.contiguous()
-        strides = [0 if bias.size(d) == 1 else bias.stride(d) for d in range(3)]
-        return bias, strides[0], strides[1], strides[2], _DTYPE_CODE[bias.dtype]
+        return load_calls().bias_operand(bias, input)
 
     @staticmethod
     def _bias_flags(causal, skip_hidden, strides, forward):
-        if skip_hidden is None:
-            # Reading the term first pays in the backward passes when the term is
-            # small next to the logits (a mask shared by the heads or by the
-            # queries): a hidden chunk saves two loads there.  In the forward
-            # pass it does not: the loads of the logits then wait for the term,
-            # which costs more than the unread logits save (measured at
-            # [16,16,1024,1024] fp16 with 48 % of the keys under -inf: 159 us
-            # with the test, 163 us without; with a -10000 mask, which hides
-            # nothing, 190-210 us against 163 us).
-            skip_hidden = (not forward) and (strides[1] == 0 or strides[2] == 0)
-        return (1 if causal else 0) | (2 if skip_hidden else 0)
+        return load_calls().bias_flags(causal, skip_hidden, strides[1], strides[2], forward)
 
     def softmax_bias_forward(self, input, bias, scale_factor, causal=False, skip_hidden=None):
         """``softmax(scale * input + bias)`` over the last dimension of the
@@ -1030,19 +724,7 @@ class _SoftmaxKernel:
         as well.  ``skip_hidden`` (default: off in the forward passes, on in the
         backward passes when the term is shared by heads or queries) lets the
         kernel leave logits unread whose term is -inf or the lowest finite value."""
-        lib = self._lib
-        _check_input(input, "input")
-        bias, sb, sh, sq_, bcode = self._bias_operand(bias, input)
-        b, np_, sq, sk = input.shape
-        out = _softmax_out(input, 1)
-        flags = self._bias_flags(causal, skip_hidden, (sb, sh, sq_), True)
-        with _device_of(input):
-            rc = lib.oslo_softmax_bias_fwd(
-                _ptr(input), _ptr(bias), _ptr(out), b, np_, sq, sk, sb, sh, sq_, bcode,
-                flags, float(scale_factor), _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return out
+        return self._calls.bias_forward(input, bias, scale_factor, causal, skip_hidden)
 
     def softmax_bias_backward(
         self, output_grads, softmax_results, scale_factor, bias=None, causal=False,
@@ -1050,197 +732,74 @@ class _SoftmaxKernel:
     ):
         """``scale * y * (g - sum(g * y))``; ``bias`` (optional) only lets the
         kernel skip loads, as in the forward pass."""
-        lib = self._lib
-        if output_grads.dim() != 4 or softmax_results.dim() != 4:
-            raise RuntimeError("expected 4D tensor")
-        _check_input(output_grads, "output_grads")
-        _check_input(softmax_results, "softmax_results")
-        if output_grads.dtype != softmax_results.dtype:
-            raise RuntimeError("output_grads and softmax_results differ in dtype")
-        if output_grads.shape != softmax_results.shape:
-            raise RuntimeError("output_grads and softmax_results differ in shape")
-        b, np_, sq, sk = softmax_results.shape
-        sb = sh = sq_ = 0
-        bcode = _dtype_code(softmax_results, "softmax_results")
-        flags = 1 if causal else 0
-        if bias is not None:
-            bias, sb, sh, sq_, bcode = self._bias_operand(bias, softmax_results)
-            flags = self._bias_flags(causal, skip_hidden, (sb, sh, sq_), False)
-            if not flags & 2:
-                bias = None
-        grad_input = output_grads if inplace else _softmax_out(output_grads, 2)
-        with _device_of(output_grads):
-            rc = lib.oslo_softmax_bias_bwd(
-                _ptr(output_grads), _ptr(softmax_results), _ptr(bias), _ptr(grad_input),
-                b, np_, sq, sk, sb, sh, sq_, bcode, flags, float(scale_factor),
-                _dtype_code(output_grads, "output_grads"), _stream(output_grads),
-            )
-            _check(rc, lib)
-        return grad_input
+        return self._calls.bias_backward(
+            output_grads, softmax_results, scale_factor, bias, causal, skip_hidden, inplace
+        )
 
     def softmax_bias_dropout_forward(
         self, input, bias, scale_factor, p, seed, offset, causal=False, skip_hidden=None
     ):
         """``dropout(softmax(scale * input + bias), p)`` -> ``[out, stats]``."""
-        lib = self._lib
-        _check_input(input, "input")
-        bias, sb, sh, sq_, bcode = self._bias_operand(bias, input)
-        b, np_, sq, sk = input.shape
-        out = _softmax_out(input, 1)
-        stats = torch.empty((b * np_ * sq, 2), dtype=torch.float32, device=input.device)
-        flags = self._bias_flags(causal, skip_hidden, (sb, sh, sq_), True)
-        with _device_of(input):
-            rc = lib.oslo_softmax_bias_dropout_fwd(
-                _ptr(input), _ptr(bias), _ptr(out), _ptr(stats), b, np_, sq, sk, sb, sh, sq_,
-                bcode, flags, float(scale_factor), float(p), int(seed), int(offset),
-                _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return [out, stats]
+        return self._calls.bias_dropout_forward(
+            input, bias, scale_factor, p, seed, offset, causal, skip_hidden
+        )
 
     def softmax_bias_dropout_backward(
         self, output_grads, input, bias, stats, scale_factor, p, seed, offset,
         causal=False, skip_hidden=None, inplace=False,
     ):
-        lib = self._lib
-        _check_input(output_grads, "output_grads")
-        _check_input(input, "input")
-        _check_input(stats, "stats")
-        if output_grads.dtype != input.dtype or output_grads.shape != input.shape:
-            raise RuntimeError("output_grads and input differ in dtype or shape")
-        bias, sb, sh, sq_, bcode = self._bias_operand(bias, input)
-        b, np_, sq, sk = input.shape
-        if stats.dtype != torch.float32 or stats.numel() != 2 * b * np_ * sq:
-            raise RuntimeError("stats must be float32 [rows, 2]")
-        flags = self._bias_flags(causal, skip_hidden, (sb, sh, sq_), False)
-        grad_input = output_grads if inplace else _softmax_out(output_grads, 2)
-        with _device_of(input):
-            rc = lib.oslo_softmax_bias_dropout_bwd(
-                _ptr(output_grads), _ptr(input), _ptr(bias), _ptr(stats), _ptr(grad_input),
-                b, np_, sq, sk, sb, sh, sq_, bcode, flags, float(scale_factor), float(p),
-                int(seed), int(offset), _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return grad_input
+        return self._calls.bias_dropout_backward(
+            output_grads, input, bias, stats, scale_factor, p, seed, offset, causal, skip_hidden,
+            inplace,
+        )
 
 
 # ---------------------------------------------------------------------------
 # bias-GeLU and bias-dropout-add (TorchScript in the reference,
 # oslo/torch/nn/modules/functional.py:23-50, 295-298; native here)
 # ---------------------------------------------------------------------------
-def _rows_cols(x, bias):
-    cols = x.shape[-1] if x.dim() > 0 else 1
-    if bias is not None:
-        if bias.dim() != 1 or bias.shape[0] != cols:
-            raise RuntimeError(
-                "bias of size %s does not match the last dimension of input of size %s"
-                % (list(bias.shape), list(x.shape))
-            )
-    rows = x.numel() // cols if cols > 0 else 0
-    return rows, cols
-
-
 class _FusedElementwiseKernel:
     def __init__(self, lib):
         self._lib = lib
+        self._calls = load_calls()
 
     def bias_gelu_forward(self, input, bias):
-        lib = self._lib
-        _check_input(input, "input")
-        if bias is not None:
-            _check_input(bias, "bias")
-            if bias.dtype != input.dtype:
-                raise RuntimeError("bias and input differ in dtype")
-        rows, cols = _rows_cols(input, bias)
-        out = torch.empty_like(input)
-        with _device_of(input):
-            rc = lib.oslo_bias_gelu_fwd(
-                _ptr(input), _ptr(bias), _ptr(out), rows, cols,
-                _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return out
+        return self._calls.gelu_forward(input, bias)
 
     def bias_gelu_backward(self, grad_output, input, bias, need_bias_grad=True):
-        lib = self._lib
-        _check_input(grad_output, "grad_output")
-        _check_input(input, "input")
-        if grad_output.dtype != input.dtype or grad_output.shape != input.shape:
-            raise RuntimeError("grad_output does not match input")
-        if bias is not None:
-            _check_input(bias, "bias")
-            if bias.dtype != input.dtype:
-                raise RuntimeError("bias and input differ in dtype")
-        rows, cols = _rows_cols(input, bias)
-        grad_input = torch.empty_like(input)
-        grad_bias = None
         lease = _NO_WORKSPACE
         if bias is not None and need_bias_grad:
-            grad_bias = torch.empty_like(bias)
-            lease = _workspace(lib, OSLO_OP_BIAS_GELU_BWD, rows, cols, input.device)
-        with _device_of(input), lease as ws:
-            rc = lib.oslo_bias_gelu_bwd(
-                _ptr(grad_output), _ptr(input), _ptr(bias), _ptr(grad_input),
-                _ptr(grad_bias), _ptr(ws.tensor), ws.nbytes, rows, cols,
-                _dtype_code(input, "input"), _stream(input),
+            lease = self._workspace(OSLO_OP_BIAS_GELU_BWD, input)
+        with lease as ws:
+            return self._calls.gelu_backward(
+                grad_output, input, bias, need_bias_grad, ws.tensor, ws.nbytes
             )
-            _check(rc, lib)
-        return grad_input, grad_bias
 
     def bias_dropout_add_forward(
         self, input, bias, residual, p, seed, offset, out=None, return_mask=False
     ):
-        lib = self._lib
-        _check_input(input, "input")
-        for name, t in (("bias", bias), ("residual", residual)):
-            if t is not None:
-                _check_input(t, name)
-                if t.dtype != input.dtype:
-                    raise RuntimeError("%s and input differ in dtype" % name)
-        if residual is not None and residual.shape != input.shape:
-            raise RuntimeError("residual does not match input")
-        rows, cols = _rows_cols(input, bias)
-        if out is None:
-            out = torch.empty_like(input)
-        mask = (
-            torch.empty(input.shape, dtype=torch.uint8, device=input.device)
-            if return_mask
-            else None
+        result = self._calls.dropout_add_forward(
+            input, bias, residual, p, seed, offset, out, return_mask
         )
-        with _device_of(input):
-            rc = lib.oslo_bias_dropout_add_fwd(
-                _ptr(input), _ptr(bias), _ptr(residual), _ptr(out), _ptr(mask),
-                rows, cols, float(p), int(seed), int(offset),
-                _dtype_code(input, "input"), _stream(input),
-            )
-            _check(rc, lib)
-        return (out, mask) if return_mask else out
+        return result if return_mask else result[0]
 
     def bias_dropout_add_backward(
         self, grad_output, p, seed, offset, need_input_grad=True, need_bias_grad=True
     ):
-        lib = self._lib
-        _check_input(grad_output, "grad_output")
-        cols = grad_output.shape[-1]
-        rows = grad_output.numel() // cols if cols > 0 else 0
-        grad_input = torch.empty_like(grad_output) if need_input_grad else None
-        grad_bias = None
         lease = _NO_WORKSPACE
         if need_bias_grad:
-            grad_bias = torch.empty(cols, dtype=grad_output.dtype, device=grad_output.device)
-            lease = _workspace(
-                lib, OSLO_OP_BIAS_DROPOUT_ADD_BWD, rows, cols, grad_output.device
+            lease = self._workspace(OSLO_OP_BIAS_DROPOUT_ADD_BWD, grad_output)
+        with lease as ws:
+            return self._calls.dropout_add_backward(
+                grad_output, p, seed, offset, need_input_grad, need_bias_grad,
+                ws.tensor, ws.nbytes,
             )
-        if grad_input is None and grad_bias is None:
-            return None, None
-        with _device_of(grad_output), lease as ws:
-            rc = lib.oslo_bias_dropout_add_bwd(
-                _ptr(grad_output), _ptr(grad_input), _ptr(grad_bias), _ptr(ws.tensor), ws.nbytes,
-                rows, cols, float(p), int(seed), int(offset),
-                _dtype_code(grad_output, "grad_output"), _stream(grad_output),
-            )
-            _check(rc, lib)
-        return grad_input, grad_bias
+
+    def _workspace(self, op, x):
+        if not x.is_cuda:
+            return _NO_WORKSPACE  # (the native call refuses it)
+        cols = x.shape[-1] if x.dim() > 0 else 1
+        return _workspace(self._lib, op, x.numel() // cols if cols > 0 else 0, cols, x.device)
 
     def philox_mask(self, n, p, seed, offset, device):
         lib = self._lib

@@ -12,6 +12,7 @@ from torch import Tensor  # noqa: F401  (named by the type comment of fused_bias
 from torch.nn import functional as F
 
 from oslo_amd.torch._C import (
+    device_rng,
     get_fused_elementwise_kernel,
     get_layernorm_kernel,
     get_softmax_kernel,
@@ -20,6 +21,17 @@ from oslo_amd.torch._C import (
 """
 Autograd Functions
 """
+
+
+class _NullContext:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NULL_CONTEXT = _NullContext()
 
 
 def _cast_if_autocast_enabled(*args):
@@ -219,9 +231,7 @@ def _next_philox_state(device):
 
 def _rng(seed):
     """Context for a kernel call: a tensor `seed` is the device-resident pair."""
-    from oslo_amd.torch._C import device_rng
-
-    return device_rng(seed if isinstance(seed, torch.Tensor) else None)
+    return device_rng(seed) if isinstance(seed, torch.Tensor) else _NULL_CONTEXT
 
 
 def _seed_arg(seed):
@@ -726,15 +736,7 @@ def _outside_autocast(x):
     """Context in which a Function runs on operands that were cast already."""
     if x.is_cuda and torch.is_autocast_enabled("cuda"):
         return torch.amp.autocast("cuda", enabled=False)
-    return _NullContext()
-
-
-class _NullContext:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
+    return _NULL_CONTEXT
 
 
 def _check_dropout_p(p):
@@ -820,11 +822,10 @@ def _bias_dropout_add_norm(rms, x, bias, residual, weight, norm_bias, normalized
         return (y, h) if return_sum else y
     p_eff = float(p) if training else 0.0
     seed, offset = _next_philox_state(x.device) if p_eff > 0.0 else (0, 0)
-    args = _cast_if_autocast_enabled(x, bias, residual, weight, norm_bias)
-    with torch.amp.autocast("cuda", enabled=False):
-        y, h = _FusedBiasDropoutAddNormFunction.apply(
-            *args, normalized_shape, eps, p_eff, seed, offset, bool(rms)
-        )
+    y, h = _apply_outside_autocast(
+        _FusedBiasDropoutAddNormFunction, x, bias, residual, weight, norm_bias,
+        normalized_shape, eps, p_eff, seed, offset, bool(rms),
+    )
     return (y, h) if return_sum else y
 
 
