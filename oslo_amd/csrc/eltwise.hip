@@ -503,7 +503,7 @@ static int generic_colsum_of_stored(const void *a, void *out, void *ws,
 
 static inline int eltwise_unroll(int dflt) {
   const int u = g_tune.eltwise_unroll;
-  return u == 1 || u == 2 || u == 4 || (u == 8 && dflt == 8) ? u : dflt;
+  return u == 1 || u == 2 || u == 4 ? u : dflt;
 }
 
 // Tile shape for `cols`: tx lanes wide (a power of two up to 256), ty = 256 /
@@ -543,14 +543,15 @@ static inline void eltwise_tile(int64_t cols, int E, int *tx, int *ty, int *tile
 // per operand in flight plus the prefetch of the next step, and the partial
 // rows stay below one percent of the tensor traffic.
 constexpr int kBwdTileMax = 128;
-constexpr int kBwdWorkgroupsPerCu = 3;
+constexpr int kBwdWorkgroupsPerCu = 3;  // the most a launch takes
 
-static int64_t colsum_parts_eltwise_e(int64_t rows, int64_t cols, int E) {
+static int64_t colsum_parts_eltwise_e(int64_t rows, int64_t cols, int E,
+                                      int per_cu = kBwdWorkgroupsPerCu) {
   int tx, ty, tiles;
   eltwise_tile(cols, E, &tx, &ty, &tiles, kBwdTileMax);
   int64_t parts = g_tune.eltwise_rowgroups > 0
                       ? g_tune.eltwise_rowgroups
-                      : ((int64_t)device_cu_count() * kBwdWorkgroupsPerCu) / tiles;
+                      : ((int64_t)device_cu_count() * per_cu) / tiles;
   const int64_t min_band =
       g_tune.eltwise_rowgroups > 0 ? ty : (16 > ty ? 16 : ty);
   const int64_t maxp = ceil_div(rows, min_band);
@@ -566,14 +567,15 @@ int64_t colsum_parts_eltwise(int64_t rows, int64_t cols) {
   return a > b ? a : b;
 }
 
-static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int unroll, int E) {
+static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int unroll, int E,
+                                       int per_cu = kBwdWorkgroupsPerCu) {
   EltGeom g;
   g.rows = rows;
   g.cols = cols;
   g.nchunks = (int)(cols / E);
   eltwise_tile(cols, E, &g.tx, &g.ty, &g.tiles, kBwdTileMax);
   const int64_t nsteps = ceil_div(rows, (int64_t)g.ty * unroll);
-  g.slots = colsum_parts_eltwise_e(rows, cols, E);
+  g.slots = colsum_parts_eltwise_e(rows, cols, E, per_cu);
   if (g.slots > nsteps) g.slots = nsteps;
   return g;
 }
@@ -676,10 +678,16 @@ static int run_bias_gelu_bwd(const void *gr, const void *x, const void *bias,
     if (rc != OSLO_OK || dbias == nullptr) return rc;
     return generic_colsum_of_stored<T>(dx, dbias, ws, ws_bytes, rows, cols, st);
   }
-  // eight chunks of each operand in flight per lane (16-bit types; measured
-  // 1-3 % faster than four), four for fp32
-  const int unroll = eltwise_unroll(sizeof(T) == 2 ? 8 : 4);
-  const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE);
+  // Chunks of each operand in flight per lane: eight for the 16-bit types
+  // (1-3 % faster than four), four for fp32.  16-bit tensors of less than 256 MB,
+  // which is what the last-level cache holds, take two and two workgroups per
+  // CU: a narrower window and more, shorter steps ([16384, 4096] bf16 77 -> 71 us,
+  // [12000, 5000] fp16 78 -> 68, [8803, 2880] bf16 39 -> 32, [3048, 4096] 20 -> 18,
+  // [358, 1536] 9.5 -> 7.7).  Larger tensors with rows of a power of two lose by
+  // it when they start on one 2 MiB phase ([16384, 16384] 267 -> 300 us).
+  const bool narrow = sizeof(T) == 2 && rows * cols * (int64_t)sizeof(T) < (256ll << 20);
+  const int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4);
+  const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE, narrow ? 2 : kBwdWorkgroupsPerCu);
   const int64_t parts = g.slots;
   const int64_t nblocks = parts * g.tiles;
   OSLO_REQUIRE(nblocks <= max_workgroups(256), "bias_gelu bwd: too many workgroups");
