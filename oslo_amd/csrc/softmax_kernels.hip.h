@@ -315,13 +315,15 @@ __device__ __forceinline__ float bias_at(const uint8_t *row, int i, bool f32) {
 }
 
 // ---------------------------------------------------------------------------
-// Ragged rows (RAG builds; bound: HBM, with dropout VALU): a row length that is no multiple of a chunk, or
-// operands off the 16-byte grid.  The chunks are counted from the first key of
-// the row and accessed where they lie; the last one ends with the row and
-// overlaps the chunk before it, so that every access is a whole vector inside
-// the row.  Its first dup_keys() keys are held twice: they count once in the
-// sums, and both lanes store the same bits.  (One wave per row with 2-byte
-// accesses before; bf16 causal [51, 1531, 1531]: forward 176 -> 67 us,
+// Ragged rows (RAG builds; bound: HBM, with dropout VALU): a row length that is
+// no multiple of a chunk, or operands off the 16-byte grid.  The chunks are
+// counted from the first key of the row and accessed where they lie; the last
+// one ends with the row and overlaps the chunk before it, so that every load is
+// a whole vector inside the row.  Its first dup_keys() keys are held twice.
+// They belong to the chunk before it: the last chunk leaves them out of the
+// sums and stores its own keys only (the two chunks may differ in whether they
+// were read at all, so they need not hold the same bits).  (One wave per row with
+// 2-byte accesses before; bf16 causal [51, 1531, 1531]: forward 176 -> 67 us,
 // backward 246 -> 89, with dropout 390 -> 79 and 305 -> 94; fp32 1003 keys
 // 94 -> 78 and 126 -> 96 us.)
 // ---------------------------------------------------------------------------
@@ -334,6 +336,17 @@ __device__ __forceinline__ int chunk_key(int c, int sk) {
 template <int E, bool RAG>
 __device__ __forceinline__ int dup_keys(int c, int sk) {
   return RAG ? c * E - chunk_key<E, RAG>(c, sk) : 0;
+}
+
+// Stores chunk c of a row, `o` being the keys from chunk_key() on: all of them,
+// or the keys of a ragged row's last chunk that are its own.
+template <typename T, int E, bool RAG>
+__device__ __forceinline__ void store_row_chunk(T *row, int c, int sk, const float *o) {
+  const int own = sk - c * E;
+  if (RAG && own < E)
+    store_last<T>(row + sk, io<T>::pack(o), own);
+  else
+    store_chunk<T, E, RAG>(row + (int64_t)c * E, o);
 }
 
 // Dropout of a ragged row: its chunks straddle the groups of eight elements of
@@ -732,7 +745,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
             }
           }
         }
-        store_chunk<T, E, RAG>(yr + chunk_key<E, RAG>(c, g.sk), o);
+        store_row_chunk<T, E, RAG>(yr, c, g.sk, o);
       }
     }
   }
@@ -947,7 +960,7 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
           for (int e = 0; e < E; ++e)
             o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
         }
-        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
+        store_row_chunk<T, E, RAG>(dxr, c, g.sk, o);
       }
     }
   }
@@ -1100,7 +1113,7 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
           for (int e = 0; e < E; ++e)
             o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
         }
-        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
+        store_row_chunk<T, E, RAG>(dxr, c, g.sk, o);
       }
     }
   }

@@ -86,3 +86,93 @@ def test_backward_in_place(device, sk):
     want = k.softmax_dropout_backward(g.to(device), x.to(device), stats, None, 0.5, 0.1, 9, 8)
     got = k.softmax_dropout_backward(g.to(device), x.to(device), stats, None, 0.5, 0.1, 9, 8, inplace=True)
     assert torch.equal(got, want)
+
+
+# lengths whose last chunk and the one before it lie in one lane group, in one
+# wave (same slot and different slots of it) and in two waves
+OVERLAPS = [(BF16, n) for n in (77, 381, 513, 1531, 2049, 4099)] + [(F16, 2051), (F32, 39), (F32, 1027)]
+
+
+def _overlap(dtype, sk):
+    """First key of the row's last chunk, first key that only it holds, and the
+    first key of the chunk before it."""
+    e = 4 if dtype == F32 else 8
+    own = (sk - 1) // e * e
+    return sk - e, own, own - e
+
+
+@pytest.mark.parametrize("dtype,sk", OVERLAPS)
+def test_a_key_held_twice_belongs_to_the_chunk_before(device, dtype, sk):
+    """The last two chunks of a row differ in being read: the chunk before the
+    last is hidden altogether (mask, absorbing term), so whatever gradient its
+    keys carry, they get zeros and the row does not see them."""
+    dup, own, before = _overlap(dtype, sk)
+    b, h, sq, scale, p = 2, 2, 9, 0.25, 0.1
+    x, g = randn((b, h, sq, sk), dtype, 1).to(device), randn((b, h, sq, sk), dtype, 2).to(device)
+    hidden = torch.zeros(b, 1, 1, sk, dtype=torch.bool, device=device)
+    hidden[..., before:own] = True
+    term = torch.zeros(b, 1, 1, sk, dtype=dtype, device=device).masked_fill_(hidden, float("-inf"))
+    bad = g.clone()
+    bad[..., dup:own] = float("nan")
+    k = _C.get_softmax_kernel()
+    y = k.fused_scaled_masked_softmax_forward(x, hidden, scale)
+    outs = []
+    for grad in (g, bad):
+        _, st = k.softmax_dropout_forward(x, hidden, scale, p, 3, 8)
+        _, st_term = k.softmax_bias_dropout_forward(x, term, scale, p, 3, 8)
+        outs.append((k.fused_scaled_masked_softmax_backward(grad, y, scale, hidden),
+                     k.softmax_bias_backward(grad, y, scale, term),
+                     k.softmax_dropout_backward(grad, x, st, hidden, scale, p, 3, 8),
+                     k.softmax_bias_dropout_backward(grad, x, term, st_term, scale, p, 3, 8)))
+    for i, (clean, dirty) in enumerate(zip(*outs)):
+        assert torch.equal(clean, dirty), "output %d" % i   # (false for a NaN)
+        assert (dirty[..., before:own] == 0).all(), "output %d" % i
+
+
+@pytest.mark.parametrize("dtype,sk", OVERLAPS)
+def test_the_sign_of_a_zero_held_twice(device, dtype, sk):
+    """The other way round: the chunk before the last is read for its first key,
+    the last one lies beyond the diagonal.  A hidden key of a chunk that is read
+    is scale * (0 * (g - s)), whose sign the gradient decides."""
+    dup, own, before = _overlap(dtype, sk)
+    scale, ab = 0.25, 64
+    # the first of sk - before queries sees `before + 1` keys; the others are not looked at
+    xq, gq = (torch.zeros(ab, sk - before, sk, dtype=dtype, device=device) for _ in range(2))
+    xq[:, 0], gq[:, 0] = (randn((ab, sk), dtype, seed).to(device) for seed in (1, 2))
+    g = gq[:, 0].double()
+    k = _C.get_softmax_kernel()
+    y = k.fused_scaled_upper_triang_masked_softmax_forward(xq, scale)
+    assert (y[:, 0, before + 1:] == 0).all() and (y[:, 0, before] > 0).all()
+    dx = k.fused_scaled_upper_triang_masked_softmax_backward(gq, y, scale)[:, 0].float()
+    margin = g - (y[:, 0].double() * g).sum(-1, keepdim=True)
+    first = max(dup, before + 1)
+    got, want = torch.signbit(dx[:, first:own]), margin[:, first:own] < 0
+    sure = margin[:, first:own].abs() > 1e-3   # (s is an fp32 sum of terms below 5)
+    assert (dx[:, first:own] == 0).all()
+    assert torch.equal(got[sure], want[sure])
+
+
+@pytest.mark.parametrize("dtype,sk", [(BF16, 2049), (BF16, 4099), (F32, 1027)])
+def test_backward_in_place_over_several_waves(device, dtype, sk):
+    """In place where the chunk that overlaps its neighbour is held by another
+    wave: every wave has read its chunks before one of them stores."""
+    b, h, sq, scale, p = 2, 3, 11, 0.25, 0.1
+    x, g = randn((b, h, sq, sk), dtype, 3).to(device), randn((b, h, sq, sk), dtype, 4).to(device)
+    hidden = (torch.arange(sk, device=device) % 5 == 1).expand(b, 1, 1, sk).contiguous()
+    hidden[1, ..., sk // 2:] = True
+    term = torch.zeros(b, 1, 1, sk, dtype=dtype, device=device).masked_fill_(hidden, float("-inf"))
+    k = _C.get_softmax_kernel()
+    for causal in (False, True):
+        y = k.fused_scaled_masked_softmax_forward(x, hidden, scale, causal=causal)
+        z = k.softmax_bias_forward(x, term, scale, causal=causal)
+        _, st = k.softmax_dropout_forward(x, hidden, scale, p, 3, 8, causal=causal)
+        _, st_term = k.softmax_bias_dropout_forward(x, term, scale, p, 3, 8, causal=causal)
+        for run in (lambda t, ip: k.fused_scaled_masked_softmax_backward(t, y, scale, hidden, ip, causal),
+                    lambda t, ip: k.softmax_bias_backward(t, z, scale, term, causal, inplace=ip),
+                    lambda t, ip: k.softmax_dropout_backward(t, x, st, hidden, scale, p, 3, 8, ip, causal),
+                    lambda t, ip: k.softmax_bias_dropout_backward(t, x, term, st_term, scale, p, 3, 8, causal,
+                                                                  inplace=ip)):
+            want = run(g.clone(), False)
+            buf = g.clone()
+            got = run(buf, True)
+            assert got.data_ptr() == buf.data_ptr() and torch.equal(got, want)
