@@ -170,34 +170,6 @@ __device__ __forceinline__ void store_chunk(T *p, const float *f) {
     st16_stream_at<ANY>(p + v * io<T>::EPV, io<T>::pack(f + v * io<T>::EPV));
 }
 
-// Stores the last `n` elements of a vector, 0 < n < EPV, so that they end at
-// `end`: one store for each power of two in n, nothing written in front of them.
-template <typename T> __device__ __forceinline__ void store_last(T *end, u32x4 r, int n) {
-  if constexpr (sizeof(T) == 4) {
-    uint32_t *p = reinterpret_cast<uint32_t *>(end);
-    if (n & 1) __builtin_nontemporal_store(r.w, p - 1);
-    if (n & 2) {
-      const u32x2 v = n & 1 ? u32x2{r.y, r.z} : u32x2{r.z, r.w};
-      __builtin_nontemporal_store(v, reinterpret_cast<u32x2_any *>(p - n));
-    }
-  } else {
-    uint16_t *p = reinterpret_cast<uint16_t *>(end);
-    const bool odd = n & 1;
-    if (odd) __builtin_nontemporal_store((uint16_t)(r.w >> 16), p - 1);
-    if (n & 2) {
-      const uint32_t v = odd ? __builtin_amdgcn_alignbit(r.w, r.z, 16) : r.w;
-      __builtin_nontemporal_store(v, reinterpret_cast<u32_any *>(p - (n & 3)));
-    }
-    if (n & 4) {
-      const bool two = n & 2;
-      const uint32_t a = two ? r.x : r.y, b = two ? r.y : r.z, c = two ? r.z : r.w;
-      const u32x2 v = odd ? u32x2{__builtin_amdgcn_alignbit(b, a, 16), __builtin_amdgcn_alignbit(c, b, 16)}
-                          : u32x2{b, c};
-      __builtin_nontemporal_store(v, reinterpret_cast<u32x2_any *>(p - n));
-    }
-  }
-}
-
 // Stores a chunk (p may be null: nothing is written) and replaces f by the
 // values as stored, taken from the very registers that were written.  Code
 // that accumulates "the tensor as stored" must go through this: rounding f a

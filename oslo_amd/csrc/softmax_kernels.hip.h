@@ -318,14 +318,18 @@ __device__ __forceinline__ float bias_at(const uint8_t *row, int i, bool f32) {
 // Ragged rows (RAG builds; bound: HBM, with dropout VALU): a row length that is
 // no multiple of a chunk, or operands off the 16-byte grid.  The chunks are
 // counted from the first key of the row and accessed where they lie; the last
-// one ends with the row and overlaps the chunk before it, so that every load is
-// a whole vector inside the row.  Its first dup_keys() keys are held twice.
-// They belong to the chunk before it: the last chunk leaves them out of the
-// sums and stores its own keys only (the two chunks may differ in whether they
-// were read at all, so they need not hold the same bits).  (One wave per row with
-// 2-byte accesses before; bf16 causal [51, 1531, 1531]: forward 176 -> 67 us,
-// backward 246 -> 89, with dropout 390 -> 79 and 305 -> 94; fp32 1003 keys
-// 94 -> 78 and 126 -> 96 us.)
+// one ends with the row and overlaps the chunk before it, so that every access
+// is a whole vector inside the row.  Its first dup_keys() keys are held twice:
+// they count once in the sums, and both lanes store the same bits.  One of the
+// two chunks may be read and the other not (hidden keys only), so a hidden key
+// of these two gets a value that depends on the row alone: zero in the forward
+// pass, also in a row of NaN, and hidden_grad() in the backward passes, which
+// take its gradient for zero.  (Storing such keys from one of the lanes only, as
+// one store for each power of two in their number or merged from the other lane,
+// costs 3 to 4 % from 1000 keys on and up to 37 % for short rows.)
+// (One wave per row with 2-byte accesses before; bf16 causal [51, 1531, 1531]:
+// forward 176 -> 67 us, backward 246 -> 89, with dropout 390 -> 79 and 305 -> 94;
+// fp32 1003 keys 94 -> 78 and 126 -> 96 us.)
 // ---------------------------------------------------------------------------
 template <int E, bool RAG>
 __device__ __forceinline__ int chunk_key(int c, int sk) {
@@ -338,15 +342,18 @@ __device__ __forceinline__ int dup_keys(int c, int sk) {
   return RAG ? c * E - chunk_key<E, RAG>(c, sk) : 0;
 }
 
-// Stores chunk c of a row, `o` being the keys from chunk_key() on: all of them,
-// or the keys of a ragged row's last chunk that are its own.
-template <typename T, int E, bool RAG>
-__device__ __forceinline__ void store_row_chunk(T *row, int c, int sk, const float *o) {
-  const int own = sk - c * E;
-  if (RAG && own < E)
-    store_last<T>(row + sk, io<T>::pack(o), own);
-  else
-    store_chunk<T, E, RAG>(row + (int64_t)c * E, o);
+// one of the two chunks that hold the keys of a ragged row held twice
+template <int E>
+__device__ __forceinline__ bool shares_keys(int c, int sk) { return c * E > sk - 2 * E; }
+// input gradient of a hidden key in a row whose sum is s: what scale * y * (g - s)
+// comes to for y = 0, g = 0 (a zero, or NaN with the rest of the row)
+__device__ __forceinline__ float hidden_grad(float scale, float s) { return scale * (0.f * (0.f - s)); }
+// float16 results of a ragged row: the float value converted as it is (in one
+// slot of a kernel the product could otherwise be fused into the conversion and
+// in another not, which differs on ties)
+template <typename T, bool RAG> __device__ __forceinline__ float one_rounding(float v) {
+  if constexpr (RAG && __is_same(T, _Float16)) return pinned(v);
+  return v;
 }
 
 // Dropout of a ragged row: its chunks straddle the groups of eight elements of
@@ -567,6 +574,13 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         float bf[E];
         unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
         xraw[j][k].unpack(v[j][k]);
+        if constexpr (RAG) {
+          // (an absorbing term is the sum, whether or not the chunk was read)
+          if (g.bias_skip) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[j][k][e] = bf[e] <= kBiasHidden ? 0.f : v[j][k][e];
+          }
+        }
         // (wave-uniform: no lane of the wave left the logits of this slot unread)
         const bool no_skip = __builtin_amdgcn_ballot_w64(bhid[j][k]) == 0;
         if (DROP && no_skip && all_visible[j][k]) {
@@ -672,6 +686,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     const float inv = empty || nokey[j] ? 0.f : row_recip(sm[j]);
     const float fill = empty ? g.inv_sk : 0.f;
     T *yr = y + row[j] * g.sk;
+    // (uniform over the wave: one of its rows is NaN)
+    const bool nan_row = __builtin_amdgcn_ballot_w64(sm[j] != sm[j]) != 0;
     if constexpr (DROP) {
       if (c0 == 0) {
         stats[2 * row[j]] = empty || nokey[j] ? 0.f : mx[j];
@@ -717,7 +733,18 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
           for (int e = 0; e < E; ++e) o[e] = fill;
         } else {
 #pragma unroll
-          for (int e = 0; e < E; ++e) o[e] = v[j][k][e] * inv + fill;
+          for (int e = 0; e < E; ++e) o[e] = one_rounding<T, RAG && !DROP>(v[j][k][e] * inv + fill);
+          if constexpr (RAG) {
+            // (with dropout the keep bits of hidden keys are off; a key under an
+            //  absorbing term is what a slot that was left unread takes it for)
+            if (nan_row && (!DROP || kBias)) {
+              const bool skipped = kBias && g.bias_skip;
+              const uint32_t hid = sm[j] != sm[j] ? mbits[j][k] : 0u;
+#pragma unroll
+              for (int e = 0; e < E; ++e)
+                o[e] = skipped && v[j][k][e] == 0.f ? 0.f : keep_or_zero(o[e], ~hid, e);
+            }
+          }
           // (the float value as it is: with a zero fill the product could
           //  otherwise be fused into the conversion to float16 in one build
           //  of the kernel and not in another, which differs on ties)
@@ -732,7 +759,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
             if constexpr (kPairDraw || RAG) {
               uint32_t keep;
               if constexpr (RAG)
-                keep = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk));
+                keep = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk)) &
+                       ~(empty ? 0u : mbits[j][k]);
               else
                 keep = paired ? keepk[k] : chunk_keep_bits<E>(row[j], g.sk, c, d);
 #pragma unroll
@@ -745,7 +773,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
             }
           }
         }
-        store_row_chunk<T, E, RAG>(yr, c, g.sk, o);
+        store_chunk<T, E, RAG>(yr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }
@@ -846,6 +874,12 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
           float bf[E];
           unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
           if (rmax[j] > kBiasHidden && bias_all_hidden<E>(bf)) mb = kAll;
+          if constexpr (RAG) {
+            if (rmax[j] > kBiasHidden && shares_keys<E>(c, g.sk)) {
+#pragma unroll
+              for (int e = 0; e < E; ++e) mb |= bf[e] <= kBiasHidden ? 1u << e : 0u;
+            }
+          }
         }
       }
       mbits[j][k] = mb;
@@ -896,7 +930,8 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
       uint32_t keep_bits = 0;
       int dup = 0;
       if constexpr (RAG) {
-        keep_bits = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk));
+        // (hidden keys take their gradient for zero)
+        keep_bits = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk)) & ~mbits[j][k];
         dup = dup_keys<E, RAG>(c, g.sk);
       } else {
         keep = chunk_keep_words<E>(row[j], g.sk, c, d);
@@ -954,13 +989,13 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
         float o[E];
         if (none_loaded[j][k]) {
 #pragma unroll
-          for (int e = 0; e < E; ++e) o[e] = 0.f;
+          for (int e = 0; e < E; ++e) o[e] = RAG ? hidden_grad(scale, s[j]) : 0.f;
         } else {
 #pragma unroll
           for (int e = 0; e < E; ++e)
-            o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
+            o[e] = one_rounding<T, RAG>(scale * (yv[j][k][e] * (gv[j][k][e] - s[j])));
         }
-        store_row_chunk<T, E, RAG>(dxr, c, g.sk, o);
+        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }
@@ -996,6 +1031,8 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
   MaskChunk<E, RAG> mraw[MODE == kModeMasked ? VPL : 1];
   u32x4 braw[kBias ? VPL : 1][kBias ? E / 4 : 1];
   RawChunk<T, E> yraw[RPW][VPL], graw[RPW][VPL];
+  constexpr bool kHides = RAG && MODE != kModeDense;
+  uint32_t hid[kHides ? VPL : 1];  // hidden keys of the chunks that share keys
 
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
@@ -1022,9 +1059,18 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
     if constexpr (MODE == kModeMasked || kBias) wait_loads();
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
+      const int c = c0 + k * cstride;
+      const bool shares = kHides && shares_keys<E>(c, g.sk);
+      if constexpr (kHides) hid[k] = 0;
       if constexpr (MODE == kModeMasked) {
-        const int i0 = chunk_key<E, RAG>(c0 + k * cstride, g.sk);
-        if (!skip[j][k]) skip[j][k] = (mraw[k].bits() | beyond_bits<E>(i0, visible)) == kAll;
+        const int i0 = chunk_key<E, RAG>(c, g.sk);
+        if (!skip[j][k]) {
+          const uint32_t bits = mraw[k].bits() | beyond_bits<E>(i0, visible);
+          skip[j][k] = bits == kAll;
+          if constexpr (kHides) hid[k] = shares && !skip[j][k] ? bits : 0u;
+        }
+      } else if constexpr (kHides) {
+        if (shares && !skip[j][k]) hid[k] = beyond_bits<E>(chunk_key<E, RAG>(c, g.sk), visible);
       }
       if constexpr (kBias) {
         // every additive term of the chunk absorbs its logit: the
@@ -1034,6 +1080,11 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
           float bf[E];
           unpack_bias_raw<T, E>(braw[k], g.bias_esize == 4, bf);
           skip[j][k] = bias_all_hidden<E>(bf);
+          if (shares) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) hid[kHides ? k : 0] |= bf[e] <= kBiasHidden ? 1u << e : 0u;
+          }
+          if (kHides && skip[j][k]) hid[kHides ? k : 0] = 0;
         }
       }
       if (!skip[j][k]) anyvis = 1.f;
@@ -1044,8 +1095,10 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
       if (g.wpr > 1) __syncthreads();
       if (anyvis == 0.f) {
 #pragma unroll
-        for (int k = 0; k < VPL; ++k)
+        for (int k = 0; k < VPL; ++k) {
           skip[j][k] = !(rvalid[j] && c0 + k * cstride < nchunks);
+          if constexpr (kHides) hid[k] = 0;
+        }
       }
     }
   }
@@ -1082,6 +1135,15 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
       if (none_loaded[j][k]) continue;
       yraw[j][k].unpack(yv[j][k]);
       graw[j][k].unpack(gv[j][k]);
+      if constexpr (kHides) {
+        if (__builtin_amdgcn_ballot_w64(hid[k] != 0u) != 0) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            yv[j][k][e] = keep_or_zero(yv[j][k][e], ~hid[k], e);
+            gv[j][k][e] = keep_or_zero(gv[j][k][e], ~hid[k], e);
+          }
+        }
+      }
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         if constexpr (RAG)
@@ -1107,13 +1169,13 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
         float o[E];
         if (none_loaded[j][k]) {
 #pragma unroll
-          for (int e = 0; e < E; ++e) o[e] = 0.f;
+          for (int e = 0; e < E; ++e) o[e] = RAG ? hidden_grad(scale, s[j]) : 0.f;
         } else {
 #pragma unroll
           for (int e = 0; e < E; ++e)
-            o[e] = scale * (yv[j][k][e] * (gv[j][k][e] - s[j]));
+            o[e] = one_rounding<T, RAG>(scale * (yv[j][k][e] * (gv[j][k][e] - s[j])));
         }
-        store_row_chunk<T, E, RAG>(dxr, c, g.sk, o);
+        store_chunk<T, E, RAG>(dxr + chunk_key<E, RAG>(c, g.sk), o);
       }
     }
   }

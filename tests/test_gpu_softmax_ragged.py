@@ -102,10 +102,11 @@ def _overlap(dtype, sk):
 
 
 @pytest.mark.parametrize("dtype,sk", OVERLAPS)
-def test_a_key_held_twice_belongs_to_the_chunk_before(device, dtype, sk):
+def test_hidden_keys_held_twice(device, dtype, sk):
     """The last two chunks of a row differ in being read: the chunk before the
-    last is hidden altogether (mask, absorbing term), so whatever gradient its
-    keys carry, they get zeros and the row does not see them."""
+    last is hidden altogether (mask, absorbing term).  Whatever gradient its keys
+    carry, also those that the last chunk holds and reads, they get zeros and the
+    row does not see them."""
     dup, own, before = _overlap(dtype, sk)
     b, h, sq, scale, p = 2, 2, 9, 0.25, 0.1
     x, g = randn((b, h, sq, sk), dtype, 1).to(device), randn((b, h, sq, sk), dtype, 2).to(device)
@@ -132,8 +133,8 @@ def test_a_key_held_twice_belongs_to_the_chunk_before(device, dtype, sk):
 @pytest.mark.parametrize("dtype,sk", OVERLAPS)
 def test_the_sign_of_a_zero_held_twice(device, dtype, sk):
     """The other way round: the chunk before the last is read for its first key,
-    the last one lies beyond the diagonal.  A hidden key of a chunk that is read
-    is scale * (0 * (g - s)), whose sign the gradient decides."""
+    the last one lies beyond the diagonal.  A hidden key that both hold gets the
+    same zero from either, scale * (0 * (0 - s))."""
     dup, own, before = _overlap(dtype, sk)
     scale, ab = 0.25, 64
     # the first of sk - before queries sees `before + 1` keys; the others are not looked at
@@ -144,12 +145,40 @@ def test_the_sign_of_a_zero_held_twice(device, dtype, sk):
     y = k.fused_scaled_upper_triang_masked_softmax_forward(xq, scale)
     assert (y[:, 0, before + 1:] == 0).all() and (y[:, 0, before] > 0).all()
     dx = k.fused_scaled_upper_triang_masked_softmax_backward(gq, y, scale)[:, 0].float()
-    margin = g - (y[:, 0].double() * g).sum(-1, keepdim=True)
+    s = (y[:, 0].double() * g).sum(-1, keepdim=True)
     first = max(dup, before + 1)
-    got, want = torch.signbit(dx[:, first:own]), margin[:, first:own] < 0
-    sure = margin[:, first:own].abs() > 1e-3   # (s is an fp32 sum of terms below 5)
     assert (dx[:, first:own] == 0).all()
-    assert torch.equal(got[sure], want[sure])
+    sure = (s.abs() > 1e-3).expand(-1, own - first)   # (an fp32 sum of terms below 5)
+    assert torch.equal(torch.signbit(dx[:, first:own])[sure], (s > 0).expand(-1, own - first)[sure])
+
+
+@pytest.mark.parametrize("dtype,sk", OVERLAPS)
+def test_hidden_keys_of_a_row_of_nan(device, dtype, sk):
+    """Forward: a NaN among the logits of a row leaves NaN at the keys that the
+    row sees and zeros at the others, however its chunks lie; with dropout a key
+    that is seen may be dropped."""
+    dup, own, before = _overlap(dtype, sk)
+    b, h, sq, scale, p = 2, 2, 3, 0.25, 0.1
+    x = randn((b, h, sq, sk), dtype, 1).to(device)
+    hidden = torch.zeros(b, 1, 1, sk, dtype=torch.bool, device=device)
+    hidden[..., dup:own] = True
+    hidden[1, ..., before:] = True
+    x[:, :, 1, 0] = float("nan")
+    k = _C.get_softmax_kernel()
+    y = k.fused_scaled_masked_softmax_forward(x, hidden, scale)
+    z, _ = k.softmax_dropout_forward(x, hidden, scale, p, 3, 8)
+    h4 = hidden.expand_as(x)
+    assert (y[h4] == 0).all() and (z[h4] == 0).all()
+    assert y[:, :, 1][~h4[:, :, 1]].isnan().all() and not y[:, :, 0].isnan().any()
+    seen = z[:, :, 1][~h4[:, :, 1]]
+    assert (seen.isnan() | (seen == 0)).all()
+    # causal: the row of the NaN sees `before + 1` keys
+    xq = torch.zeros(2, sk - before, sk, dtype=dtype, device=device)
+    xq[:, 0, 0] = float("nan")
+    y = k.fused_scaled_upper_triang_masked_softmax_forward(xq, scale)[:, 0]
+    z, _ = k.softmax_dropout_forward(xq, None, scale, p, 3, 8)
+    assert y[:, :before + 1].isnan().all()
+    assert (y[:, before + 1:] == 0).all() and (z[:, 0, before + 1:] == 0).all()
 
 
 @pytest.mark.parametrize("dtype,sk", [(BF16, 2049), (BF16, 4099), (F32, 1027)])
