@@ -1635,9 +1635,16 @@ static inline unsigned ragged_keep_lds(const SoftmaxPlan &pl) {
 // limit in the 16-bit forward, causal with a key mask 160 KB (314 against 342 us),
 // rows of several waves 160 and 96 KB (4096 keys backward 322 against 348 us),
 // ragged rows, two to a workgroup, 128 KB.
+// All of these are of rows that fill the lanes that hold them.  A wave with idle
+// lanes requests less, so more of them are kept: 16 waves of rows that fill five
+// lanes of eight, or half of them, is 20 to 30 % slower than no limit (additive
+// term, fp32 80 keys forward 178 -> 142 us; causal fp16 8 keys 768 -> 627, 72 keys
+// 198 -> 163, 288 keys 203 -> 165; key mask, fp32 608 keys backward 189 -> 172).
+// Additive terms with several rows to a wave, which waits for both operands: 96 KB
+// (bf16 392 keys 373 -> 327 us, fp16 352 keys 387 -> 362 at 900 MB).
 template <typename T, int MODE>
-static int softmax_waves_per_cu(const SoftmaxPlan &pl, bool backward, bool drop, bool causal,
-                                bool ragged) {
+static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bool drop,
+                                bool causal, bool ragged) {
   constexpr bool k16 = sizeof(T) == 2;
   int kb;
   if (backward) {
@@ -1647,6 +1654,7 @@ static int softmax_waves_per_cu(const SoftmaxPlan &pl, bool backward, bool drop,
     if (pl.wpr > 1 || (MODE == kModeMasked && causal)) kb = 160;
   } else {
     kb = MODE == kModeMasked ? 112 : 64;
+    if (MODE == kModeBias && pl.rpw > 1) kb = 96;
     if (drop) kb = 96;
     if (pl.wpr > 1 && kb < 96) kb = 96;
     if (drop && k16) return 0;
@@ -1658,7 +1666,9 @@ static int softmax_waves_per_cu(const SoftmaxPlan &pl, bool backward, bool drop,
   if (!backward && !drop && !ragged && waves > 28 &&
       !(MODE == kModeCausal && k16 && pl.lpr == kWave))
     waves = 28;
-  return waves;
+  if (ragged) return waves;  // (measured as they are)
+  const int64_t slots = (int64_t)pl.vpl * (pl.lpr == kWave ? kWave * pl.wpr : pl.lpr);
+  return (int)(waves * slots / ceil_div(sk, io<T>::EPV));
 }
 
 // LDS that a launch of `nblocks` workgroups reserves in order to keep at most
@@ -1818,7 +1828,7 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
   const unsigned occ = occupancy_lds(
-      softmax_waves_per_cu<T, MODE>(pl, false, drop, g.causal, ragged), threads, nblocks);
+      softmax_waves_per_cu<T, MODE>(pl, g.sk, false, drop, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_FWD(VPL, RPW, LPR_)                                  \
   if constexpr (VPL * RPW * E <= (MODE == kModeBias ? kBiasMaxElems : kFwdMaxElems)) { \
@@ -1902,7 +1912,7 @@ int launch_softmax_bwd(const void *dy, const void *y,
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
   const unsigned occ = occupancy_lds(
-      softmax_waves_per_cu<T, MODE>(pl, true, false, g.causal, ragged), threads, nblocks);
+      softmax_waves_per_cu<T, MODE>(pl, g.sk, true, false, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_BWD(VPL, RPW, LPR_)                        \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_))       \
@@ -1976,7 +1986,7 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
   const unsigned occ = occupancy_lds(
-      softmax_waves_per_cu<T, MODE>(pl, true, true, g.causal, ragged), threads, nblocks);
+      softmax_waves_per_cu<T, MODE>(pl, g.sk, true, true, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
 #define OSLO_SM_DBWD(VPL, RPW, LPR_)                                \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_) && (MODE != kModeBias || RPW <= 2)) \
