@@ -106,7 +106,8 @@ def test_hidden_keys_held_twice(device, dtype, sk):
     """The last two chunks of a row differ in being read: the chunk before the
     last is hidden altogether (mask, absorbing term).  Whatever gradient its keys
     carry, also those that the last chunk holds and reads, they get zeros and the
-    row does not see them."""
+    row does not see them.  (The plain backward of shorter rows does not look at
+    the mask: a gradient that is not finite then shows in both chunks.)"""
     dup, own, before = _overlap(dtype, sk)
     b, h, sq, scale, p = 2, 2, 9, 0.25, 0.1
     x, g = randn((b, h, sq, sk), dtype, 1).to(device), randn((b, h, sq, sk), dtype, 2).to(device)
@@ -121,8 +122,10 @@ def test_hidden_keys_held_twice(device, dtype, sk):
     for grad in (g, bad):
         _, st = k.softmax_dropout_forward(x, hidden, scale, p, 3, 8)
         _, st_term = k.softmax_bias_dropout_forward(x, term, scale, p, 3, 8)
-        outs.append((k.fused_scaled_masked_softmax_backward(grad, y, scale, hidden),
-                     k.softmax_bias_backward(grad, y, scale, term),
+        chunks = -(-sk // (4 if dtype == F32 else 8))
+        masked, biased = (grad if chunks > most else g for most in (48, 64 if dtype == F32 else 128))
+        outs.append((k.fused_scaled_masked_softmax_backward(masked, y, scale, hidden),
+                     k.softmax_bias_backward(biased, y, scale, term),
                      k.softmax_dropout_backward(grad, x, st, hidden, scale, p, 3, 8),
                      k.softmax_bias_dropout_backward(grad, x, term, st_term, scale, p, 3, 8)))
     for i, (clean, dirty) in enumerate(zip(*outs)):
@@ -205,3 +208,26 @@ def test_backward_in_place_over_several_waves(device, dtype, sk):
             buf = g.clone()
             got = run(buf, True)
             assert got.data_ptr() == buf.data_ptr() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype,chunks", [(BF16, 48), (BF16, 49), (BF16, 128), (BF16, 129), (F32, 48), (F32, 49),
+                                          (F32, 64), (F32, 65)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_plain_backward_with_and_without_a_look_at_the_mask(device, dtype, chunks, causal):
+    """Around the row lengths at which the plain backward starts to look at the
+    mask or at the additive term: padding, a row of which every key is hidden
+    (uniform under the mask, over all keys), per-query masks, absorbing terms."""
+    e = 4 if dtype == F32 else 8
+    sk = chunks * e - 3
+    check_causal_masked(device, 2, 2, 9, sk, dtype, 0.25, "holes")
+    check_masked(device, 2, 2, 9, sk, dtype, 0.25, "full")
+    b, h, sq, scale = 2, 2, 9, 0.25
+    x, g = randn((b, h, sq, sk), dtype, 1), randn((b, h, sq, sk), dtype, 2)
+    hidden = torch.arange(sk).expand(b, 1, 1, sk) >= torch.tensor([sk, sk // 2]).view(b, 1, 1, 1)
+    k = _C.get_softmax_kernel()
+    for fill in (-10000.0, float("-inf"), torch.finfo(dtype).min):
+        term = torch.zeros(b, 1, 1, sk, dtype=dtype).masked_fill_(hidden, fill)
+        y = k.softmax_bias_forward(x.to(device), term.to(device), scale, causal)
+        for skip in (None, True):
+            dx = k.softmax_bias_backward(g.to(device), y, scale, term.to(device), causal, skip)
+            check(dx, cf.softmax_bwd(f64(g), f64(y), scale), "additive %g" % fill, atol=1e-7)
