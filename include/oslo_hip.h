@@ -284,7 +284,9 @@ int oslo_softmax_causal_masked_dropout_bwd(const void *dout, const void *x,
  * a row whose terms are all -inf gives NaN, as torch.softmax does.
  * flags: OSLO_SOFTMAX_CAUSAL hides key j of query i when j > i + (sk - sq)
  * as well (exact zeros, also in a query row that the diagonal leaves without
- * any key when sq > sk; neither x nor M is read there);
+ * any key when sq > sk; neither x nor M is read there.  In a row that is NaN the
+ * keys beyond the diagonal are zeros if the row length is no multiple of 16
+ * bytes, else NaN or zero);
  * OSLO_SOFTMAX_SKIP_HIDDEN reads M first and leaves the logits of a 16-byte
  * chunk unread when every term of it is at or below the lowest finite
  * bfloat16 (-3.39e38; the lowest float and -inf are), where the float sum is

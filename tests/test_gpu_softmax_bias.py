@@ -444,3 +444,28 @@ def test_row_order_of_a_term_shared_by_the_batch(device, b, np_, sq, sk, dtype, 
     for other in outs[1:]:
         for a, c in zip(outs[0], other):
             assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("sk", [3, 7, 77, 301, 1531, 2049, 33001])
+def test_diagonal_of_a_row_of_nan(device, dtype, sk):
+    """Left-padded causal attention with a -inf term: the queries in the padding
+    see keys under -inf only, and their rows are NaN up to the diagonal (with
+    dropout, NaN or dropped) and, at lengths that are no multiple of a vector,
+    exact zeros beyond it."""
+    b, h, sq, scale, p = 2, 2, min(sk, 5), 0.25, 0.1
+    pad = sk - sq + 2                  # the first two queries lie in the padding
+    x = randn((b, h, sq, sk), dtype, seed=1).to(device)
+    term = torch.zeros(b, 1, 1, sk, dtype=dtype, device=device)
+    term[..., :pad] = float("-inf")
+    k = _C.get_softmax_kernel()
+    beyond = torch.arange(sk, device=device) > torch.arange(sq, device=device).view(-1, 1) + (sk - sq)
+    beyond = beyond.expand(b, h, sq, sk)
+    nan_row = (torch.arange(sq, device=device).view(-1, 1) + (sk - sq) < pad).expand(b, h, sq, sk)
+    y = k.softmax_bias_forward(x, term, scale, causal=True)
+    z, _ = k.softmax_bias_dropout_forward(x, term, scale, p, 3, 8, causal=True)
+    for t in (y, z):
+        assert (t[beyond] == 0).all() and not t[~nan_row].isnan().any()
+    assert y[nan_row & ~beyond].isnan().all()
+    seen = z[nan_row & ~beyond]
+    assert (seen.isnan() | (seen == 0)).all()
