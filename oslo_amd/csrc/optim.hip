@@ -42,6 +42,7 @@ struct AdamArgs {
   float beta1, beta2, eps, lr, decay;
   Recip rbc1, rbc2;
   int mode;
+  int scaled;  // eps beyond 2^-96 ... 2^90: see quotient()
 };
 static_assert(sizeof(AdamTable) + sizeof(AdamArgs) <= 4096, "kernel arguments");
 
@@ -73,24 +74,36 @@ __device__ __forceinline__ float root(float x) {
 }
 
 // a / b, one Newton step on a * v_rcp_f32(b): q + (a - b q) / b, with the
-// special values (zero, infinity, NaN) of the exact quotient.
-__device__ __forceinline__ float quotient(float a, float b) {
+// special values (zero, infinity, NaN) of the exact quotient.  A quotient that
+// overflows stays infinite (its residual enters the step as the largest float).
+// The divisors that v_rcp_f32 does not take, subnormal ones and those whose
+// reciprocal is subnormal, are scaled with the dividend; only an eps of that size
+// leads to one (SCALED, a branch of the whole vector: in every step it would cost
+// 16-bit tensors of 2 M parameters 5 %).
+template <bool SCALED> __device__ __forceinline__ float quotient(float a, float b) {
+  if constexpr (SCALED) {
+    const float k = fabsf(b) < 0x1p-96f ? 0x1p64f : fabsf(b) > 0x1p96f ? 0x1p-64f : 1.f;
+    a *= k;
+    b *= k;
+  }
   const float r = __builtin_amdgcn_rcpf(b);
   const float q = a * r;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-b, q, a), r, q), b, a);
+  const float rest = __builtin_amdgcn_fmed3f(fmaf(-b, q, a), -__FLT_MAX__, __FLT_MAX__);
+  return __builtin_amdgcn_div_fixupf(fmaf(rest, r, q), b, a);
 }
 
 // The update of multi_tensor_adam.cu:78-96, term for term.  Its three
 // divisions and the square root as the language defines them are some 145
 // instructions an element: bf16 spent 83 % of its time in them.  The two by
 // constants are products here, the other two take one Newton step.
+template <bool SCALED>
 __device__ __forceinline__ void adam_update(float g, float &p, float &m,
                                             float &v, const AdamArgs &a) {
   if (a.mode == 0) g = g + a.decay * p;
   m = a.beta1 * m + (1.f - a.beta1) * g;
   v = a.beta2 * v + (1.f - a.beta2) * g * g;
   const float denom = root(times(v, a.rbc2)) + a.eps;
-  float update = quotient(times(m, a.rbc1), denom);
+  float update = quotient<SCALED>(times(m, a.rbc1), denom);
   if (a.mode != 0) update = update + a.decay * p;
   p = p - a.lr * update;
 }
@@ -133,8 +146,13 @@ __global__ __launch_bounds__(kAdamThreads) void multi_tensor_adam_kernel(
 #pragma unroll
     for (int u = 0; u < kAdamUnroll; ++u) {
       const int64_t i = start + ((int64_t)u * kAdamThreads + threadIdx.x) * E;
+      if (a.scaled) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) adam_update(rg[u][e], rp[u][e], rm[u][e], rv[u][e], a);
+        for (int e = 0; e < E; ++e) adam_update<true>(rg[u][e], rp[u][e], rm[u][e], rv[u][e], a);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) adam_update<false>(rg[u][e], rp[u][e], rm[u][e], rv[u][e], a);
+      }
       store_chunk<T, E>(p + i, rp[u]);
       store_chunk<T, E>(m + i, rm[u]);
       store_chunk<T, E>(v + i, rv[u]);
@@ -148,7 +166,10 @@ __global__ __launch_bounds__(kAdamThreads) void multi_tensor_adam_kernel(
     float pp = io<T>::from_scalar(p[i]);
     float mm = io<T>::from_scalar(m[i]);
     float vv = io<T>::from_scalar(v[i]);
-    adam_update(gg, pp, mm, vv, a);
+    if (a.scaled)
+      adam_update<true>(gg, pp, mm, vv, a);
+    else
+      adam_update<false>(gg, pp, mm, vv, a);
     p[i] = io<T>::to_scalar(pp);
     m[i] = io<T>::to_scalar(mm);
     v[i] = io<T>::to_scalar(vv);
@@ -232,6 +253,7 @@ int oslo_multi_tensor_adam(const void *const *g, void *const *p, void *const *m,
   a.lr = lr;
   a.decay = weight_decay;
   a.mode = mode;
+  a.scaled = eps != 0.f && !(eps >= 0x1p-96f && eps <= 0x1p90f);
   // multi_tensor_adam.cu:120-125: 1 - beta^step, evaluated by std::pow on the
   // float betas (which promotes to double) and stored as float
   float bc1 = 1.0f, bc2 = 1.0f;

@@ -45,6 +45,28 @@ def test_special_values(device):
         assert p[3] == -inf and p[4].isnan() and p[6].isnan() and p[7] < 0.0
 
 
+def test_quotients_at_the_ends_of_the_range(device):
+    """update = m / (sqrt(v) + eps) where it overflows (loaded moments; it is
+    infinite, not NaN), and with divisors that have no normal reciprocal."""
+    inf = float("inf")
+    cases = [(1e35, 0.0, 1e-8), (-3e38, 1e-30, 0.0), (3e38, 0.25, 0.5), (-3.4e38, 0.2, 0.5), (1e-10, 0.0, 1e-40),
+             (1.0, 0.0, 1e-45), (-1e-44, 0.0, 1e-44), (0.0, 0.0, 1e-40), (1e38, 0.0, 2e38), (-3e38, 0.0, 3.3e38),
+             (1e-38, 0.0, 1e38), (1e-30, 1e-45, 0.0), (1e30, 3e38, 0.0), (inf, 0.0, 1e-40), (2e38, 0.0, 0.5)]
+    for m, v, eps in cases:
+        host = [torch.tensor([t], dtype=F32) for t in (0.0, 0.0, m, v)]
+        lists = [[t.to(device)] for t in host]
+        _C.get_adam_kernel().multi_tensor_adam(0, None, lists, 1.0, 1.0, 1.0, eps, 1, 1, 0, 0.0)
+        got = float(lists[1][0])
+        denom = np.float32(np.float32(np.sqrt(f64(host[3])[0])) + np.float32(eps))
+        with np.errstate(over="ignore"):
+            want = -float(np.float32(f64(host[2])[0] / np.float64(denom)))
+        if np.isinf(want):
+            assert got == want, (m, v, eps, got)
+        else:
+            # (a subnormal quotient is rounded once more)
+            assert abs(got - want) <= 4e-7 * abs(want) + 1.5e-45, (m, v, eps, got, want)
+
+
 @pytest.mark.parametrize("dtype", [F32, torch.bfloat16])
 @pytest.mark.parametrize("count", [1, 2, 87, 88, 89, 177])
 def test_tensor_table(device, dtype, count):
