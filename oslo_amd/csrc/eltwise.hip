@@ -501,9 +501,10 @@ static int generic_colsum_of_stored(const void *a, void *out, void *ws,
   return check_launch("colsum_generic_kernel");
 }
 
-static inline int eltwise_unroll(int dflt) {
+// (`eight`: the kernel has a build with eight chunks in flight)
+static inline int eltwise_unroll(int dflt, bool eight = false) {
   const int u = g_tune.eltwise_unroll;
-  return u == 1 || u == 2 || u == 4 ? u : dflt;
+  return u == 1 || u == 2 || u == 4 || (u == 8 && eight) ? u : dflt;
 }
 
 // Tile shape for `cols`: tx lanes wide (a power of two up to 256), ty = 256 /
@@ -686,7 +687,7 @@ static int run_bias_gelu_bwd(const void *gr, const void *x, const void *bias,
   // [358, 1536] 9.5 -> 7.7).  Larger tensors with rows of a power of two lose by
   // it when they start on one 2 MiB phase ([16384, 16384] 267 -> 300 us).
   const bool narrow = sizeof(T) == 2 && rows * cols * (int64_t)sizeof(T) < (256ll << 20);
-  const int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4);
+  const int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4, sizeof(T) == 2);
   const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE, narrow ? 2 : kBwdWorkgroupsPerCu);
   const int64_t parts = g.slots;
   const int64_t nblocks = parts * g.tiles;

@@ -38,3 +38,27 @@ def test_both_launch_shapes(device, dtype, rows):
     total = dx.double().sum(0)
     bound = 8 * 2 ** -24 * rows ** 0.5 * dx.double().square().sum(0).sqrt() + torch.finfo(dtype).eps * total.abs()
     assert ((db.double() - total).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("chunks", [2, 8])
+def test_the_override_reaches_the_build(device, dtype, chunks):
+    """eltwise_unroll below the 256 MB: a workgroup of four rows of lanes takes
+    4 * chunks rows a step, and a small problem has one partial row per step."""
+    rows, cols = 64, 512
+    x, g = (randn((rows, cols), dtype, i).to(device) for i in (1, 2))
+    bias = torch.zeros(cols, dtype=dtype, device=device)
+    dx, db = torch.empty_like(x), torch.empty_like(bias)
+    lib = _C.load_library()
+    _C.tune("eltwise_unroll", chunks)
+    try:
+        nbytes = lib.oslo_workspace_bytes(_C.OSLO_OP_BIAS_GELU_BWD, rows, cols)
+        ws = torch.full((nbytes // 4,), float("nan"), device=device)
+        assert lib.oslo_bias_gelu_bwd(g.data_ptr(), x.data_ptr(), bias.data_ptr(), dx.data_ptr(), db.data_ptr(),
+                                      ws.data_ptr(), nbytes, rows, cols, 1 if dtype == torch.float16 else 2,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+    finally:
+        _C.tune("eltwise_unroll", 0)
+    torch.cuda.synchronize()
+    written = int((~ws.isnan()).sum())
+    assert written == min(rows // 16, rows // (4 * chunks)) * cols
