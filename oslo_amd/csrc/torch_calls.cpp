@@ -9,13 +9,14 @@
 // took 9-11 us of a norm's 14.6 us a call, of which the launch is about 3.
 //
 // The GIL is held while the arguments are read and released from the first
-// allocation to the launch, so that a launch that blocks (a full queue) does
-// not stop other Python threads.
+// allocation to the launch (but for the lease of a workspace between the two),
+// so that a launch that blocks (a full queue) does not stop other Python threads.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -72,6 +73,11 @@ struct Args {
     const int64_t v = PyLong_AsLongLong(next());
     if (v == -1 && PyErr_Occurred()) throw python_error();
     return v;
+  }
+  // a callable, null for None
+  PyObject *callable() {
+    PyObject *o = next();
+    return o == Py_None ? nullptr : o;
   }
   // any integer, modulo 2^64
   uint64_t word() {
@@ -189,6 +195,57 @@ struct OnDevice {
       : guard(t.device()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
 };
 
+// A backward workspace: the lease that `get` (n1, n2, device) hands out, held
+// from here to the end of the scope.  It is taken behind the checks, so that a
+// refused call leaves the cache as it is, on the operand's device, whose capture
+// decides about the cache, and behind the outputs.  Constructed and destroyed
+// with the GIL held.
+struct Workspace {
+  PyObject *lease = nullptr;
+  Tensor tensor;
+  int64_t nbytes = 0;
+
+  Workspace(PyObject *get, int64_t n1, int64_t n2, const Tensor &like) {
+    if (get == nullptr) return;
+    PyObject *device = THPDevice_New(like.device());
+    if (device != nullptr) lease = PyObject_CallFunction(get, "LLN", (long long)n1, (long long)n2, device);
+    if (lease == nullptr) throw python_error();
+    try {
+      PyObject *entered = PyObject_CallMethod(lease, "__enter__", nullptr);
+      if (entered == nullptr) throw python_error();
+      Py_DECREF(entered);
+    } catch (...) {
+      Py_DECREF(lease);
+      throw;
+    }
+    PyObject *t = PyObject_GetAttrString(lease, "tensor");
+    PyObject *n = t != nullptr ? PyObject_GetAttrString(lease, "nbytes") : nullptr;
+    if (n != nullptr) {
+      if (THPVariable_Check(t)) tensor = THPVariable_Unpack(t);
+      nbytes = PyLong_AsLongLong(n);
+    }
+    Py_XDECREF(t);
+    Py_XDECREF(n);
+    if (PyErr_Occurred()) {
+      release();
+      throw python_error();
+    }
+  }
+  Workspace(const Workspace &) = delete;
+  ~Workspace() { release(); }
+
+  void release() {
+    if (lease == nullptr) return;
+    PyObject *type, *value, *trace;  // (an error on its way out stays)
+    PyErr_Fetch(&type, &value, &trace);
+    PyObject *r = PyObject_CallMethod(lease, "__exit__", "OOO", Py_None, Py_None, Py_None);
+    if (r == nullptr) PyErr_WriteUnraisable(lease);
+    Py_XDECREF(r);
+    Py_CLEAR(lease);
+    PyErr_Restore(type, value, trace);
+  }
+};
+
 // An output of the softmax: from 64 MiB on it starts k * (1 MiB + 4 KiB) past
 // a 2 MiB boundary (empty_staggered of the Python module says why).
 Tensor softmax_out(const Tensor &like, int k) {
@@ -243,7 +300,7 @@ PyObject *norm_forward(Args &g) {
   return rms ? wrap_all({out, inv}, true) : wrap_all({out, mean, inv}, true);
 }
 
-// (rms, dout, mean, invvar, input, normalized_shape, gamma, beta, workspace, nbytes)
+// (rms, dout, mean, invvar, input, normalized_shape, gamma, beta, workspace)
 // -> (grad_input, grad_gamma, grad_beta)
 PyObject *norm_backward(Args &g) {
   const bool rms = g.flag();
@@ -252,8 +309,8 @@ PyObject *norm_backward(Args &g) {
   const Tensor &inv = g.tensor();
   const Tensor &x = g.tensor();
   const auto shape = g.sizes();
-  const Tensor gamma = g.optional(), beta = g.optional(), ws = g.optional();
-  const int64_t nbytes = g.integer();
+  const Tensor gamma = g.optional(), beta = g.optional();
+  PyObject *const get = g.callable();
   check_input(dy, "dout");
   check_input(inv, "invvar");
   check_input(x, "input");
@@ -279,18 +336,22 @@ PyObject *norm_backward(Args &g) {
                 " but dout has dtype ", dtype_name(dy.scalar_type()));
   }
   Tensor dx, dg, db;
+  const OnDevice on(x);
   {
     NoGil nogil;
-    const OnDevice on(x);
     dx = at::empty(x.sizes(), x.options());
     if (gamma.defined()) {
       dg = at::empty_like(gamma);
       if (!rms) db = at::empty_like(beta.defined() ? beta : gamma);
     }
-    check_rc(rms ? oslo_rms_bwd(ptr(dy), ptr(x), ptr(inv), ptr(gamma), ptr(dx), ptr(dg), ptr(ws), nbytes, n1,
-                                n2, din, dcode, on.stream)
+  }
+  const Workspace ws(get, n1, n2, x);
+  {
+    NoGil nogil;
+    check_rc(rms ? oslo_rms_bwd(ptr(dy), ptr(x), ptr(inv), ptr(gamma), ptr(dx), ptr(dg), ptr(ws.tensor), ws.nbytes,
+                                n1, n2, din, dcode, on.stream)
                  : oslo_ln_bwd(ptr(dy), ptr(x), ptr(mean), ptr(inv), ptr(gamma), ptr(dx), ptr(dg), ptr(db),
-                               ptr(ws), nbytes, n1, n2, din, dcode, on.stream));
+                               ptr(ws.tensor), ws.nbytes, n1, n2, din, dcode, on.stream));
   }
   return wrap_all({dx, dg, db}, false);
 }
@@ -337,7 +398,7 @@ PyObject *residual_norm_forward(Args &g) {
 }
 
 // (rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma, p, seed, offset,
-//  need_bias_grad, workspace, nbytes)
+//  need_bias_grad, workspace)
 // -> (grad_residual, grad_input, grad_gamma, grad_beta, grad_bias)
 PyObject *residual_norm_backward(Args &g) {
   const bool rms = g.flag();
@@ -351,8 +412,7 @@ PyObject *residual_norm_backward(Args &g) {
   const double p = g.real();
   const uint64_t seed = g.word(), offset = g.word();
   const bool want_bias = g.flag();
-  const Tensor ws = g.optional();
-  const int64_t nbytes = g.integer();
+  PyObject *const get = g.callable();
   check_input(dy, "dout");
   check_input(h, "h");
   check_input(inv, "invvar");
@@ -382,9 +442,9 @@ PyObject *residual_norm_backward(Args &g) {
                 " but h has dtype ", dtype_name(h.scalar_type()));
   }
   Tensor dres, dx, dg, db, dbias;
+  const OnDevice on(h);
   {
     NoGil nogil;
-    const OnDevice on(h);
     dres = at::empty(h.sizes(), h.options());
     if (p > 0.0) dx = at::empty(h.sizes(), h.options());
     if (gamma.defined()) {
@@ -392,9 +452,14 @@ PyObject *residual_norm_backward(Args &g) {
       if (!rms) db = at::empty_like(gamma);
     }
     if (want_bias) dbias = at::empty(shape, h.options());
+  }
+  const Workspace ws(get, n1, n2, h);
+  {
+    NoGil nogil;
     check_rc(oslo_bias_dropout_add_norm_bwd(ptr(dy), ptr(extra), ptr(h), rms ? nullptr : (const float *)ptr(mean), (const float *)ptr(inv),
-                                            ptr(gamma), ptr(dres), ptr(dx), ptr(dg), ptr(db), ptr(dbias), ptr(ws),
-                                            nbytes, n1, n2, (float)p, seed, offset, rms, code, on.stream));
+                                            ptr(gamma), ptr(dres), ptr(dx), ptr(dg), ptr(db), ptr(dbias),
+                                            ptr(ws.tensor), ws.nbytes, n1, n2, (float)p, seed, offset, rms, code,
+                                            on.stream));
   }
   return wrap_all({dres, dx.defined() ? dx : dres, dg, db, dbias}, false);
 }
@@ -787,14 +852,13 @@ PyObject *gelu_forward(Args &g) {
   return wrap(out);
 }
 
-// (grad_output, input, bias, need_bias_grad, workspace, nbytes) -> (grad_input, grad_bias)
+// (grad_output, input, bias, need_bias_grad, workspace) -> (grad_input, grad_bias)
 PyObject *gelu_backward(Args &g) {
   const Tensor &dy = g.tensor();
   const Tensor &x = g.tensor();
   const Tensor bias = g.optional();
   const bool want_bias = g.flag();
-  const Tensor ws = g.optional();
-  const int64_t nbytes = g.integer();
+  PyObject *const get = g.callable();
   check_input(dy, "grad_output");
   check_input(x, "input");
   TORCH_CHECK(dy.scalar_type() == x.scalar_type() && dy.sizes() == x.sizes(), "grad_output does not match input");
@@ -803,13 +867,17 @@ PyObject *gelu_backward(Args &g) {
   rows_and_cols(x, bias, rows, cols);
   const int code = dtype_code(x, "input");
   Tensor dx, db;
+  const OnDevice on(x);
   {
     NoGil nogil;
-    const OnDevice on(x);
     dx = at::empty(x.sizes(), x.options());
     if (bias.defined() && want_bias) db = at::empty_like(bias);
-    check_rc(oslo_bias_gelu_bwd(ptr(dy), ptr(x), ptr(bias), ptr(dx), ptr(db), ptr(ws), nbytes, rows, cols, code,
-                                on.stream));
+  }
+  const Workspace ws(get, rows, cols, x);
+  {
+    NoGil nogil;
+    check_rc(oslo_bias_gelu_bwd(ptr(dy), ptr(x), ptr(bias), ptr(dx), ptr(db), ptr(ws.tensor), ws.nbytes, rows, cols,
+                                code, on.stream));
   }
   return wrap_all({dx, db}, false);
 }
@@ -844,27 +912,30 @@ PyObject *dropout_add_forward(Args &g) {
   return wrap_all({out, mask}, false);
 }
 
-// (grad_output, p, seed, offset, need_input_grad, need_bias_grad, workspace, nbytes)
+// (grad_output, p, seed, offset, need_input_grad, need_bias_grad, workspace)
 // -> (grad_input, grad_bias)
 PyObject *dropout_add_backward(Args &g) {
   const Tensor &dy = g.tensor();
   const float p = (float)g.real();
   const uint64_t seed = g.word(), offset = g.word();
   const bool want_input = g.flag(), want_bias = g.flag();
-  const Tensor ws = g.optional();
-  const int64_t nbytes = g.integer();
+  PyObject *const get = g.callable();
   check_input(dy, "grad_output");
   int64_t rows, cols;
   rows_and_cols(dy, Tensor(), rows, cols);
   Tensor dx, db;
   if (want_input || want_bias) {
     const int code = dtype_code(dy, "grad_output");
-    NoGil nogil;
     const OnDevice on(dy);
-    if (want_input) dx = at::empty(dy.sizes(), dy.options());
-    if (want_bias) db = at::empty({cols}, dy.options());
-    check_rc(oslo_bias_dropout_add_bwd(ptr(dy), ptr(dx), ptr(db), ptr(ws), nbytes, rows, cols, p, seed, offset, code,
-                                       on.stream));
+    {
+      NoGil nogil;
+      if (want_input) dx = at::empty(dy.sizes(), dy.options());
+      if (want_bias) db = at::empty({cols}, dy.options());
+    }
+    const Workspace ws(get, rows, cols, dy);
+    NoGil nogil;
+    check_rc(oslo_bias_dropout_add_bwd(ptr(dy), ptr(dx), ptr(db), ptr(ws.tensor), ws.nbytes, rows, cols, p, seed,
+                                       offset, code, on.stream));
   }
   return wrap_all({dx, db}, false);
 }

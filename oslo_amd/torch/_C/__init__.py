@@ -434,12 +434,10 @@ def _workspace(lib, op, n1, n2, device):
     return _ws_cache.lease(index, stream, op, nbytes)
 
 
-def _norm_workspace(lib, op, input, normalized_shape):
-    """Lease for a norm backward; the native call refuses what is not on the GPU."""
-    if not input.is_cuda:
-        return _NO_WORKSPACE
-    n1, n2 = _compute_n1_n2(input, normalized_shape)
-    return _workspace(lib, op, n1, n2, input.device)
+def _leases(lib, op):
+    """What a native backward calls for its workspace, once it has checked its
+    operands: ``(n1, n2, device)`` -> lease."""
+    return lambda n1, n2, device: _workspace(lib, op, n1, n2, device)
 
 
 class device_rng:
@@ -479,42 +477,14 @@ def tune(key, value):
 # ---------------------------------------------------------------------------
 # LayerNorm / RMSNorm
 # ---------------------------------------------------------------------------
-def _compute_n1_n2(input, normalized_shape):
-    # check_args / compute_n1_n2 of FusedLayerNormBinder.cpp:19-36, 59-93
-    if len(normalized_shape) == 1 and input.dim() >= 1 and input.shape[-1] == normalized_shape[0]:
-        n2 = int(normalized_shape[0])  # the common case, without building tuples
-        return (input.numel() // n2 if n2 > 0 else 0), n2
-    normalized_shape = tuple(int(s) for s in normalized_shape)
-    if len(normalized_shape) < 1:
-        raise RuntimeError(
-            "Expected normalized_shape to be at least 1-dimensional, i.e., "
-            "containing at least one element, but got normalized_shape=%s"
-            % (list(normalized_shape),)
-        )
-    nd = len(normalized_shape)
-    if input.dim() < nd or tuple(input.shape[input.dim() - nd:]) != normalized_shape:
-        raise RuntimeError(
-            "Given normalized_shape=%s, expected input with shape [*, %s], but got "
-            "input of size%s"
-            % (
-                list(normalized_shape),
-                ", ".join(str(s) for s in normalized_shape),
-                list(input.shape),
-            )
-        )
-    n2 = 1
-    for s in normalized_shape:
-        n2 *= s
-    n1 = input.numel() // n2 if n2 > 0 else 0
-    return n1, n2
-
-
 class _LayerNormKernel:
     """The ten functions of the reference's ``oslo_fused_layer_norm`` module."""
 
     def __init__(self, lib):
         self._lib = lib
         self._calls = load_calls()
+        self._leases = [_leases(lib, op) for op in
+                        (OSLO_OP_LN_BWD, OSLO_OP_RMS_BWD, OSLO_OP_BIAS_DROPOUT_ADD_NORM_BWD)]
 
     # -- forward ----------------------------------------------------------
     def layer_norm_forward(self, input, normalized_shape, eps):
@@ -537,15 +507,10 @@ class _LayerNormKernel:
 
     # -- backward ---------------------------------------------------------
     def _backward(self, rms, dout, mean, invvar, input, normalized_shape, gamma, beta):
-        lease = _NO_WORKSPACE
-        if gamma is not None:
-            op = OSLO_OP_RMS_BWD if rms else OSLO_OP_LN_BWD
-            lease = _norm_workspace(self._lib, op, input, normalized_shape)
-        with lease as ws:
-            return self._calls.norm_backward(
-                rms, dout, mean, invvar, input, normalized_shape, gamma, beta,
-                ws.tensor, ws.nbytes,
-            )
+        return self._calls.norm_backward(
+            rms, dout, mean, invvar, input, normalized_shape, gamma, beta,
+            None if gamma is None else self._leases[1 if rms else 0],
+        )
 
     def layer_norm_backward(self, dout, mean, invvar, input, normalized_shape, eps):
         return self._backward(False, dout, mean, invvar, input, normalized_shape, None, None)[0]
@@ -589,16 +554,10 @@ class _LayerNormKernel:
     ):
         """Returns ``(grad_residual, grad_input, grad_gamma, grad_beta, grad_bias)``;
         ``grad_input`` is ``grad_residual`` itself when ``p == 0``."""
-        lease = _NO_WORKSPACE
-        if gamma is not None or need_bias_grad:
-            lease = _norm_workspace(
-                self._lib, OSLO_OP_BIAS_DROPOUT_ADD_NORM_BWD, h, normalized_shape
-            )
-        with lease as ws:
-            return self._calls.residual_norm_backward(
-                rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma, p, seed, offset,
-                need_bias_grad, ws.tensor, ws.nbytes,
-            )
+        return self._calls.residual_norm_backward(
+            rms, dout, dh_extra, h, mean, invvar, normalized_shape, gamma, p, seed, offset,
+            need_bias_grad, self._leases[2] if gamma is not None or need_bias_grad else None,
+        )
 
 
 # ---------------------------------------------------------------------------
@@ -762,18 +721,17 @@ class _FusedElementwiseKernel:
     def __init__(self, lib):
         self._lib = lib
         self._calls = load_calls()
+        self._gelu_leases = _leases(lib, OSLO_OP_BIAS_GELU_BWD)
+        self._dropout_leases = _leases(lib, OSLO_OP_BIAS_DROPOUT_ADD_BWD)
 
     def bias_gelu_forward(self, input, bias):
         return self._calls.gelu_forward(input, bias)
 
     def bias_gelu_backward(self, grad_output, input, bias, need_bias_grad=True):
-        lease = _NO_WORKSPACE
-        if bias is not None and need_bias_grad:
-            lease = self._workspace(OSLO_OP_BIAS_GELU_BWD, input)
-        with lease as ws:
-            return self._calls.gelu_backward(
-                grad_output, input, bias, need_bias_grad, ws.tensor, ws.nbytes
-            )
+        return self._calls.gelu_backward(
+            grad_output, input, bias, need_bias_grad,
+            self._gelu_leases if bias is not None and need_bias_grad else None,
+        )
 
     def bias_dropout_add_forward(
         self, input, bias, residual, p, seed, offset, out=None, return_mask=False
@@ -786,20 +744,10 @@ class _FusedElementwiseKernel:
     def bias_dropout_add_backward(
         self, grad_output, p, seed, offset, need_input_grad=True, need_bias_grad=True
     ):
-        lease = _NO_WORKSPACE
-        if need_bias_grad:
-            lease = self._workspace(OSLO_OP_BIAS_DROPOUT_ADD_BWD, grad_output)
-        with lease as ws:
-            return self._calls.dropout_add_backward(
-                grad_output, p, seed, offset, need_input_grad, need_bias_grad,
-                ws.tensor, ws.nbytes,
-            )
-
-    def _workspace(self, op, x):
-        if not x.is_cuda:
-            return _NO_WORKSPACE  # (the native call refuses it)
-        cols = x.shape[-1] if x.dim() > 0 else 1
-        return _workspace(self._lib, op, x.numel() // cols if cols > 0 else 0, cols, x.device)
+        return self._calls.dropout_add_backward(
+            grad_output, p, seed, offset, need_input_grad, need_bias_grad,
+            self._dropout_leases if need_bias_grad else None,
+        )
 
     def philox_mask(self, n, p, seed, offset, device):
         lib = self._lib

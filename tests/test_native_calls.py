@@ -50,6 +50,50 @@ def test_other_arguments_are_refused():
         calls.norm_forward(False, X, 8, None, None, 1e-5, False)
 
 
+def _backwards(device, n1, n2, other):
+    """The four backwards that take a workspace, on [n1, n2] with an incoming
+    gradient of `other` columns."""
+    ln, _, el = _C.get_layernorm_kernel(), None, _C.get_fused_elementwise_kernel()
+    x, g = torch.randn(n1, n2, device=device), torch.randn(n1, other, device=device)
+    w, stat = torch.ones(n2, device=device), torch.ones(n1, device=device)
+    return [lambda: ln.layer_norm_backward_affine(g, stat, stat, x, (n2,), w, w, 1e-5),
+            lambda: ln.rms_norm_backward_affine(g, stat, x, (n2,), w, 1e-5),
+            lambda: ln.bias_dropout_add_norm_backward(False, g, None, x, stat, stat, (n2,), w, 0.1, 1, 0),
+            lambda: el.bias_gelu_backward(g, x, w)]
+
+
+def _cached():
+    return {key: slot.tensor for key, slot in _C._ws_cache.slots.items()}
+
+
+@pytest.mark.gpu
+def test_a_refused_backward_leaves_the_workspaces_alone(device):
+    before = _cached()
+    for call in _backwards(device, 2048, 8192, 8):   # (larger than what other tests leave there)
+        with pytest.raises(RuntimeError):
+            call()
+    after = _cached()
+    assert after.keys() == before.keys() and all(after[k] is before[k] for k in after)
+
+
+@pytest.mark.gpu
+def test_a_failed_allocation_of_a_workspace(device, monkeypatch):
+    """The error comes through as it is, and the slot is free for the next call."""
+    def fail(nbytes, index):
+        raise MemoryError("no workspace")
+
+    with torch.cuda.stream(torch.cuda.Stream()):      # (a stream without cached workspaces)
+        calls = _backwards(device, 64, 128, 128)
+        with monkeypatch.context() as m:
+            m.setattr(_C._ws_cache, "allocate", fail)
+            for call in calls:
+                with pytest.raises(MemoryError, match="no workspace"):
+                    call()
+        for call in calls:
+            assert all(torch.isfinite(t).all() for t in call())
+    torch.cuda.synchronize()
+
+
 @pytest.mark.gpu
 def test_large_softmax_outputs_are_staggered(device):
     sm = _C.get_softmax_kernel()
