@@ -64,7 +64,8 @@ int oslo_wave_reduce_selftest(float *out4, void *stream);
  * the default, with eight lanes per slice and 32 columns per workgroup, or
  * 256 with four lanes per slice and 16 columns), "softmax_waves_per_cu" (waves
  * of a softmax launch kept on a compute unit, 1..32; by default from the bytes
- * that a wave requests);
+ * that a wave requests; 32, and values that leave fewer than three workgroups,
+ * do not limit the launch);
  * value 0 restores the default.  Other values must be ones the launch code
  * has a kernel build and a valid workgroup shape for, else
  * OSLO_ERR_INVALID_ARGUMENT: chunks per lane (*_vpl: 1, 2, 4, forward also 8,

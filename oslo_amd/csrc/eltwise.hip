@@ -680,12 +680,17 @@ static int run_bias_gelu_bwd(const void *gr, const void *x, const void *bias,
     return generic_colsum_of_stored<T>(dx, dbias, ws, ws_bytes, rows, cols, st);
   }
   // Chunks of each operand in flight per lane: eight for the 16-bit types
-  // (1-3 % faster than four), four for fp32.  16-bit tensors of less than 256 MB,
-  // which is what the last-level cache holds, take two and two workgroups per
-  // CU: a narrower window and more, shorter steps ([16384, 4096] bf16 77 -> 71 us,
-  // [12000, 5000] fp16 78 -> 68, [8803, 2880] bf16 39 -> 32, [3048, 4096] 20 -> 18,
-  // [358, 1536] 9.5 -> 7.7).  Larger tensors with rows of a power of two lose by
-  // it when they start on one 2 MiB phase ([16384, 16384] 267 -> 300 us).
+  // (1-3 % faster than four), four for fp32.  16-bit tensors of less than 256 MB
+  // take two and two workgroups per CU, a narrower window and more, shorter
+  // steps: faster at each of nineteen shapes from 31 MB up to the line, rows of
+  // powers of two among them, with the operands on four combinations of 2 MiB
+  // phases ([8191, 16384] bf16 132-136 us against 137-141, [16300, 8192] 131-136
+  // against 138-141, [2047, 65536] 140-143 against 147-149, [12000, 5000] 67
+  // against 75, [8803, 2880] 32 against 39).  The line is a matter of caution:
+  // above it a loop of this kernel alone gains as well ([16384, 16384] 272 ->
+  // 261 us, [8192, 24576] 219 -> 201), but forward and backward of [16384, 16384]
+  // in turn took 458 us with the narrow window against 433, the backward 300
+  // when x, the gradient and dx started on one phase, and the cause is not known.
   const bool narrow = sizeof(T) == 2 && rows * cols * (int64_t)sizeof(T) < (256ll << 20);
   const int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4, sizeof(T) == 2);
   const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE, narrow ? 2 : kBwdWorkgroupsPerCu);

@@ -10,9 +10,15 @@ from oslo_amd.torch import _C
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("waves", [1, 12, 28, 32])
-@pytest.mark.parametrize("sk,dtype", [(2048, torch.bfloat16), (1531, torch.float16), (260, torch.float32),
-                                      (4100, torch.bfloat16)])
+# (values that leave at least three workgroups of 1, 2, 1 and 6 waves on a compute
+#  unit: below that a launch is not limited)
+CASES = [(sk, dtype, waves)
+         for sk, dtype, values in [(2048, torch.bfloat16, (3, 12, 20, 28)), (1531, torch.float16, (6, 12, 20, 28)),
+                                   (260, torch.float32, (3, 12, 20, 28)), (4100, torch.bfloat16, (18, 24, 31))]
+         for waves in values]
+
+
+@pytest.mark.parametrize("sk,dtype,waves", CASES)
 def test_waves_per_compute_unit_keep_the_bits(device, sk, dtype, waves):
     k = _C.get_softmax_kernel()
     x, g = randn((2, 37, sk), dtype, 1).to(device), randn((2, 37, sk), dtype, 2).to(device)
