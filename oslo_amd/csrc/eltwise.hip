@@ -682,9 +682,9 @@ static int run_bias_gelu_bwd(const void *gr, const void *x, const void *bias,
   // Chunks of each operand in flight per lane: eight for the 16-bit types
   // (1-3 % faster than four), four for fp32.  16-bit tensors of less than 256 MB
   // take two and two workgroups per CU, a narrower window and more, shorter
-  // steps: faster at each of nineteen shapes from 31 MB up to the line, rows of
-  // powers of two among them, with the operands on four combinations of 2 MiB
-  // phases ([8191, 16384] bf16 132-136 us against 137-141, [16300, 8192] 131-136
+  // steps: up to 15 % faster and slower at none of nineteen shapes from 31 MB up
+  // to the line, rows of powers of two among them, with the operands on four
+  // combinations of 2 MiB phases ([8191, 16384] bf16 132-136 us against 137-141, [16300, 8192] 131-136
   // against 138-141, [2047, 65536] 140-143 against 147-149, [12000, 5000] 67
   // against 75, [8803, 2880] 32 against 39).  The line is a matter of caution:
   // above it a loop of this kernel alone gains as well ([16384, 16384] 272 ->

@@ -12,6 +12,10 @@ from oracle import closed_form as cf
 from oracle import philox
 from oslo_amd.torch import _C
 
+from test_gpu_norm import test_layer_norm as check_layer_norm
+from test_gpu_norm import test_rms_norm as check_rms_norm
+from test_gpu_residual_norm import test_fused_vs_oracle as check_fused
+
 pytestmark = pytest.mark.gpu
 
 F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
@@ -45,3 +49,22 @@ def test_slots(device, n1, n2, dtype, fused):
     tensors = 2 if fused else 1
     for i, (g, w) in enumerate(zip(got, want)):
         check(g, w, "output %d" % i, atol=2e-6 if i < tensors else atol, max_ulp=1 if i < tensors else 2)
+
+
+@pytest.mark.parametrize("prefetch", [1, 2])
+@pytest.mark.parametrize("tin,tout", [(F32, F32), (F16, F16), (BF16, BF16), (F32, F16), (F32, BF16)])
+def test_sixteen_slots_of_sixteen_elements_per_lane(device, tin, tout, prefetch):
+    """Rows that one wave holds with 16 elements a lane, the last ones idle, and
+    enough of them that a workgroup keeps its sixteen slots."""
+    n1, n2 = 15 * 256 + 10, 800
+    _C.tune("norm_bwd_vpl", 4)
+    _C.tune("norm_bwd_prefetch", prefetch)
+    try:
+        check_layer_norm(device, n1, n2, tin, tout, True)
+        check_rms_norm(device, n1, n2, tin, tout, True)
+        if tin == tout:
+            check_fused(device, n1, n2, tin, 0.1, False)
+            check_fused(device, n1, n2, tin, 0.1, True)
+    finally:
+        _C.tune("norm_bwd_vpl", 0)
+        _C.tune("norm_bwd_prefetch", 0)
