@@ -823,9 +823,9 @@ def module_table(L, dev, iters, kernel_rows):
         t = time_launches(torch, fn, iters, nsets)
         gbps = nbytes / (t[0] * 1e-3) / 1e9
         # the same eager calls enqueued behind a few ms of other GPU work, so that the
-        # host runs ahead: a call costs the host 90-130 us of Python per forward +
-        # backward (autograd.Function, ctypes), more than the shorter kernels run, and
-        # a loop of nothing but such calls measures Python, not the GPU
+        # host runs ahead: a call costs the host time in Python per forward +
+        # backward (autograd.Function), which can be more than the shorter kernels run, and
+        # a loop of nothing but such calls then measures Python, not the GPU
         tq = time_queued(torch, fn, nsets, blocker)
         qgbps = nbytes / (tq * 1e-3) / 1e9
         rows.append({
@@ -1374,7 +1374,7 @@ def main():
                     "events on the launch stream, rotating inputs, gradients cleared to None before each call); MB = "
                     "algorithmic bytes of the pair; c_abi_GBps = the same pair through the raw C ABI on pre-allocated "
                     "buffers (kernel table); ratio_to_c_abi = GBps / c_abi_GBps; us / GBps = a loop of nothing but "
-                    "these calls (bound by the 90-130 us of Python per call where the kernels are shorter); queued_* "
+                    "these calls (bound by the Python of a call where the kernels are shorter); queued_* "
                     "= the same eager calls enqueued behind ~5 ms of other GPU work, so that the host runs ahead of "
                     "the GPU as it does in a training step (events on the stream bracket the calls' GPU time)",
             "rows": module_table(L, dev, max(20, args.table_iters // 2), rows),
