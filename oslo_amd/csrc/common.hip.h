@@ -13,6 +13,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
@@ -219,9 +220,18 @@ template <typename A, typename B> struct chunk_elems {
 
 // ---------------------------------------------------------------------------
 // wave64 reductions.  Four DPP steps make every row of 16 lanes uniform
-// (quad swaps, then the half-row and row mirrors); the four row values are
-// then read through v_readlane and combined in a fixed order, so every lane
-// ends with the same, deterministic result.  All 64 lanes must be active.
+// (quad swaps, then the half-row and row mirrors); two more carry row 0 into
+// row 1 and row 2 into row 3, then the sum of the lower half into the upper
+// one, whose last lane is read back: every lane ends with the same,
+// deterministic result, (r0 + r1) + (r2 + r3).  All 64 lanes must be active.
+//
+// Bound: instruction issue (these run twice per softmax or norm row).  Written
+// as assembly, one instruction a step: the compiler keeps four for a maximum
+// (it quietens both operands first) and combines the rows through four
+// v_readlane.  The wait states are those of a DPP read after a vector write
+// (two) and of v_readlane (one); the first step waits five, since the compiler
+// does not see what reads the operand there and may have written it with a dot
+// product (three) or a transcendental.
 // ---------------------------------------------------------------------------
 template <int CTRL> __device__ __forceinline__ float dpp_mov(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(
@@ -237,25 +247,59 @@ __device__ __forceinline__ float readlane(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+#define OSLO_DPP_STEP(OP, CTRL, ROWS) \
+  "v_" OP "_f32_dpp %0, %0, %0 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\ts_nop 1\n\t"
+#define OSLO_DPP_8(OP)                                \
+  "s_nop 4\n\t"                                       \
+  OSLO_DPP_STEP(OP, "quad_perm:[1,0,3,2]", "0xf")     \
+  OSLO_DPP_STEP(OP, "quad_perm:[2,3,0,1]", "0xf")     \
+  OSLO_DPP_STEP(OP, "row_half_mirror", "0xf")
+#define OSLO_DPP_16(OP) OSLO_DPP_8(OP) OSLO_DPP_STEP(OP, "row_mirror", "0xf")
+#define OSLO_DPP_64(OP)                               \
+  OSLO_DPP_16(OP)                                     \
+  OSLO_DPP_STEP(OP, "row_bcast:15", "0xa")            \
+  OSLO_DPP_STEP(OP, "row_bcast:31", "0xc")
+
+// apply: one operation; group<N>: over each run of N consecutive lanes (8 or
+// 16), in place; wave: over all lanes, the result in lane 63
 struct OpSum {
   static __device__ __forceinline__ float apply(float a, float b) {
     return a + b;
   }
+  template <int N> static __device__ __forceinline__ float group(float v) {
+    if constexpr (N == 8)
+      asm(OSLO_DPP_8("add") : "+v"(v));
+    else
+      asm(OSLO_DPP_16("add") : "+v"(v));
+    return v;
+  }
+  static __device__ __forceinline__ float wave(float v) {
+    asm(OSLO_DPP_64("add") : "+v"(v));
+    return v;
+  }
 };
 struct OpMax {
+  // (one instruction; NaN as fmaxf takes it: the other operand)
   static __device__ __forceinline__ float apply(float a, float b) {
-    return fmaxf(a, b);
+    float r;
+    asm("s_nop 2\n\tv_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
+  template <int N> static __device__ __forceinline__ float group(float v) {
+    if constexpr (N == 8)
+      asm(OSLO_DPP_8("max") : "+v"(v));
+    else
+      asm(OSLO_DPP_16("max") : "+v"(v));
+    return v;
+  }
+  static __device__ __forceinline__ float wave(float v) {
+    asm(OSLO_DPP_64("max") : "+v"(v));
+    return v;
   }
 };
 
 template <typename Op> __device__ __forceinline__ float wave_allreduce(float v) {
-  v = Op::apply(v, dpp_mov<kDppQuadSwap1>(v));
-  v = Op::apply(v, dpp_mov<kDppQuadSwap2>(v));
-  v = Op::apply(v, dpp_mov<kDppRowHalfMirror>(v));
-  v = Op::apply(v, dpp_mov<kDppRowMirror>(v));
-  float r0 = readlane(v, 0), r1 = readlane(v, 16);
-  float r2 = readlane(v, 32), r3 = readlane(v, 48);
-  return Op::apply(Op::apply(r0, r1), Op::apply(r2, r3));
+  return readlane(Op::wave(v), 63);
 }
 __device__ __forceinline__ float wave_sum(float v) {
   return wave_allreduce<OpSum>(v);
@@ -356,11 +400,7 @@ __device__ __forceinline__ float rsqrt_refined(float a) {
 // waves that share a row: lane l < wpr reads wave l's value from LDS, the
 // other lanes pass the identity.
 template <typename Op> __device__ __forceinline__ float row16_allreduce(float v) {
-  v = Op::apply(v, dpp_mov<kDppQuadSwap1>(v));
-  v = Op::apply(v, dpp_mov<kDppQuadSwap2>(v));
-  v = Op::apply(v, dpp_mov<kDppRowHalfMirror>(v));
-  v = Op::apply(v, dpp_mov<kDppRowMirror>(v));
-  return readlane(v, 0);
+  return readlane(Op::template group<16>(v), 0);
 }
 
 // A product / difference that is rounded on its own and never fused with a
@@ -387,6 +427,10 @@ __device__ __forceinline__ float pinned(float v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+__device__ __forceinline__ uint32_t pinned(uint32_t v) {
+  asm("" : "+v"(v));
+  return v;
+}
 
 // Reduction within each group of LPR (8, 16 or 32) consecutive lanes; every
 // lane of a group receives its group's result (each step is symmetric, so the
@@ -394,11 +438,13 @@ __device__ __forceinline__ float pinned(float v) {
 template <typename Op, int LPR>
 __device__ __forceinline__ float group_allreduce(float v) {
   static_assert(LPR == 8 || LPR == 16 || LPR == 32, "group size");
-  v = Op::apply(v, dpp_mov<kDppQuadSwap1>(v));
-  v = Op::apply(v, dpp_mov<kDppQuadSwap2>(v));
-  v = Op::apply(v, dpp_mov<kDppRowHalfMirror>(v));
-  if constexpr (LPR >= 16) v = Op::apply(v, dpp_mov<kDppRowMirror>(v));
-  if constexpr (LPR >= 32) v = Op::apply(v, __shfl_xor(v, 16));
+  v = Op::template group<(LPR < 16 ? 8 : 16)>(v);
+  if constexpr (LPR == 32) {
+    // the other row of 16 lanes of the pair, without a trip through the LDS
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                                    false, false);
+    v = Op::apply(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
   return v;
 }
 
@@ -473,14 +519,37 @@ dropout_keep_bits(uint64_t group, uint64_t seed, uint64_t offset,
       philox4x32_10((uint32_t)offset, (uint32_t)(offset >> 32),
                     (uint32_t)group, (uint32_t)(group >> 32), (uint32_t)seed,
                     (uint32_t)(seed >> 32));
+#if defined(__HIP_DEVICE_COMPILE__)
+  // Two 16-bit fields at a time: field -sat (threshold - 1) is not zero exactly
+  // for the fields that reach the threshold, and a minimum with 1 makes it the
+  // decision: 14 instructions for the eight, 24 one by one.  (A threshold of 0
+  // keeps everything and is not representable; it is taken apart, uniformly.)
+  const uint32_t t1 = threshold - (threshold != 0u ? 1u : 0u);
+  const u16x2 limit = __builtin_bit_cast(u16x2, t1 | (t1 << 16));
+  // (hidden from the optimiser, as the differences below are, which would turn
+  //  the pair into two compares)
+  uint32_t ones = 0x10001u;
+  asm("" : "+s"(ones));
+  const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+  uint32_t f[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t d = pinned(__builtin_bit_cast(
+        uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, w[i]), limit)));
+    f[i] = __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, d), __builtin_bit_cast(u16x2, ones)));
+  }
+  const uint32_t x = (f[0] | (f[1] << 2)) | ((f[2] << 4) | (f[3] << 6));
+  return ((x | (x >> 15)) & 0xffu) | (threshold == 0 ? 0xffu : 0u);
+#else
   const uint32_t w[4] = {r.x, r.y, r.z, r.w};
   uint32_t bits = 0;
-#pragma unroll
   for (int i = 0; i < 4; ++i) {
     bits |= ((w[i] & 0xffffu) >= threshold ? 1u : 0u) << (2 * i);
     bits |= ((w[i] >> 16) >= threshold ? 1u : 0u) << (2 * i + 1);
   }
   return bits;
+#endif
 }
 
 // Dropout parameters of one call.  Element i of the flattened tensor belongs

@@ -208,8 +208,9 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70
 template <int E>
 __device__ __forceinline__ uint32_t beyond_bits(int i0, int visible) {
   constexpr uint32_t kAllBits = (1u << E) - 1u;
-  const int left = visible - i0;  // keys of the chunk below the diagonal
-  return left >= E ? 0u : (left <= 0 ? kAllBits : kAllBits & ~((1u << left) - 1u));
+  // keys of the chunk below the diagonal, 0 .. E
+  const int left = min(max(visible - i0, 0), E);
+  return kAllBits & (kAllBits << left);
 }
 
 // Row bookkeeping shared by forward and backward.  Rows are numbered so that
@@ -385,11 +386,40 @@ __device__ __forceinline__ uint32_t row_keep_bits(const uint8_t *kb, int64_t row
   typedef uint16_t u16_any __attribute__((aligned(1)));
   return (uint32_t)*reinterpret_cast<const u16_any *>(kb + (at >> 3)) >> (at & 7u);
 }
-// v where bit e of the keep bits is set, else +0: two instructions
-__device__ __forceinline__ float keep_or_zero(float v, uint32_t keep, int e) {
-  return __uint_as_float(__float_as_uint(v) &
-                         (uint32_t)__builtin_amdgcn_sbfe((int)keep, e, 1));
+// All ones where bit e of `bits` is set, else zero.  (Hidden from the optimiser,
+// which would make the two instructions that use it a test, a compare and a
+// select, with two wait states between the last two.)
+__device__ __forceinline__ uint32_t bit_mask(uint32_t bits, int e) {
+  return pinned((uint32_t)__builtin_amdgcn_sbfe((int)bits, e, 1));
 }
+// v where bit e of the keep bits is set, else +0
+__device__ __forceinline__ float keep_or_zero(float v, uint32_t keep, int e) {
+  return __uint_as_float(__float_as_uint(v) & bit_mask(keep, e));
+}
+// -inf where bit e of the hidden keys' bits is set, else v
+__device__ __forceinline__ float hide(float v, uint32_t hidden, int e) {
+  const uint32_t m = bit_mask(hidden, e);
+  return __uint_as_float((m & 0xff800000u) | (~m & __float_as_uint(v)));
+}
+// s plus the E values of chunk c, without those of the keys held twice; only
+// the slot of the row's last chunk has such keys (wave-uniform test)
+template <int E, bool RAG>
+__device__ __forceinline__ float add_chunk(float s, const float *v, int c, int sk) {
+  if constexpr (RAG) {
+    const int dup = dup_keys<E, RAG>(c, sk);
+    // (lanes beyond the row hold nothing that counts)
+    if (__builtin_amdgcn_ballot_w64(dup != 0) != 0) {
+      const uint32_t once = ~((1u << (dup < E ? dup : E)) - 1u);
+#pragma unroll
+      for (int e = 0; e < E; ++e) s += keep_or_zero(v[e], once, e);
+      return s;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) s += v[e];
+  return s;
+}
+
 // bytes of keep bits per lane group of a row: one for each chunk it can hold,
 // one for the group that the row's first key shifts past them, one that is
 // read but never used
@@ -565,6 +595,10 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
       if (none_visible[j][k]) continue;
+      // (the values of a slot are formed first and the hidden ones replaced in a
+      //  wave-uniform branch of its own: with the arithmetic in both branches the
+      //  compiler evaluates it twice)
+      xraw[j][k].unpack(v[j][k]);
       if constexpr (MODE == kModeBias) {
         // the sum scale * x + term as one fused multiply-add, kept in the
         // natural domain: a large negative term (-10000) then costs the logit
@@ -573,7 +607,6 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         //  the logits they cost a wave per SIMD)
         float bf[E];
         unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
-        xraw[j][k].unpack(v[j][k]);
         if constexpr (RAG) {
           // (an absorbing term is the sum, whether or not the chunk was read)
           if (g.bias_skip) {
@@ -581,49 +614,23 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
             for (int e = 0; e < E; ++e) v[j][k][e] = bf[e] <= kBiasHidden ? 0.f : v[j][k][e];
           }
         }
-        // (wave-uniform: no lane of the wave left the logits of this slot unread)
-        const bool no_skip = __builtin_amdgcn_ballot_w64(bhid[j][k]) == 0;
-        if (DROP && no_skip && all_visible[j][k]) {
-          // (the common slot as a branch of its own, two instructions a key, in
-          //  the kernels with dropout, which are bound by instruction issue:
-          //  204 -> 186 us at [16, 16, 1024, 1024] fp16; the kernels without
-          //  dropout are bound by memory there and measure 2 % slower with
-          //  the branch, 163 -> 167 us)
-#pragma unroll
-          for (int e = 0; e < E; ++e) {
-            const float t = __builtin_fmaf(v[j][k][e], scale, bf[e]);
-            v[j][k][e] = t;
-            m = fmaxf(m, t);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < E; ++e) {
-            float t = bhid[j][k] ? bf[e] : __builtin_fmaf(v[j][k][e], scale, bf[e]);
-            t = (mbits[j][k] >> e) & 1u ? ninf : t;
-            v[j][k][e] = t;
-            m = fmaxf(m, t);
-          }
-        }
-        continue;
-      }
-      xraw[j][k].unpack(v[j][k]);
-      if (all_visible[j][k]) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-          // (rounded product, never fused into the later subtraction: the
-          //  backward pass of the dropout variant recomputes it bit for bit)
-          const float t = mul_rn(v[j][k][e], c2);
-          v[j][k][e] = t;
-          m = fmaxf(m, t);
+          const float t = __builtin_fmaf(v[j][k][e], scale, bf[e]);
+          v[j][k][e] = bhid[j][k] ? bf[e] : t;  // (a slot that was left unread)
         }
       } else {
+        // (rounded product, never fused into the later subtraction: the
+        //  backward pass of the dropout variant recomputes it bit for bit)
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const float t = (mbits[j][k] >> e) & 1u ? ninf : mul_rn(v[j][k][e], c2);
-          v[j][k][e] = t;
-          m = fmaxf(m, t);
-        }
+        for (int e = 0; e < E; ++e) v[j][k][e] = mul_rn(v[j][k][e], c2);
       }
+      if (!all_visible[j][k]) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[j][k][e] = hide(v[j][k][e], mbits[j][k], e);
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) m = fmaxf(m, v[j][k][e]);
     }
     mx[j] = m;
   }
@@ -657,13 +664,9 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
       for (int e = 0; e < E; ++e) {
         float d = sub_rn(v[j][k][e], off);
         if constexpr (kBias) d = mul_rn(d, kLog2e);
-        const float p = __builtin_amdgcn_exp2f(d);
-        v[j][k][e] = p;  // exp2(-inf) == 0 for masked keys
-        if constexpr (RAG)
-          s += e < dup_keys<E, RAG>(c0 + k * cstride, g.sk) ? 0.f : p;
-        else
-          s += p;
+        v[j][k][e] = __builtin_amdgcn_exp2f(d);  // exp2(-inf) == 0 for masked keys
       }
+      s = add_chunk<E, RAG>(s, v[j][k], c0 + k * cstride, g.sk);
     }
     sm[j] = s;
   }
@@ -683,8 +686,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     // a row without any visible key: uniform distribution, as softmax of a
     // constant fill value gives
     const bool empty = mx[j] == ninf && !kBias;
-    const float inv = empty || nokey[j] ? 0.f : row_recip(sm[j]);
-    const float fill = empty ? g.inv_sk : 0.f;
+    float inv = empty || nokey[j] ? 0.f : row_recip(sm[j]);
+    float fill = empty ? g.inv_sk : 0.f;
     T *yr = y + row[j] * g.sk;
     // (uniform over the wave: one of its rows is NaN)
     const bool nan_row = __builtin_amdgcn_ballot_w64(sm[j] != sm[j]) != 0;
@@ -693,6 +696,9 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
         stats[2 * row[j]] = empty || nokey[j] ? 0.f : mx[j];
         stats[2 * row[j] + 1] = empty ? -fill : inv;
       }
+      // (the factor of the kept probabilities, once a row)
+      inv *= d.scale;
+      fill *= d.scale;
     }
     // A 4-element chunk is half a dropout group, and the lanes 2i and 2i + 1
     // hold the two halves: instead of evaluating every group twice, the even
@@ -728,10 +734,20 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
       const int c = c0 + k * cstride;
       if (c < nchunks) {
         float o[E];
-        if (none_visible[j][k]) {
+        // (wave-uniform; exact zeros need no draw)
+        if (none_visible[j][k] && !(DROP && empty)) {
 #pragma unroll
           for (int e = 0; e < E; ++e) o[e] = fill;
-        } else {
+          store_chunk<T, E, RAG>(yr + chunk_key<E, RAG>(c, g.sk), o);
+          continue;
+        }
+        if constexpr (DROP) {
+          if (none_visible[j][k]) {  // a row without a visible key: uniform, drawn
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[j][k][e] = 0.f;
+          }
+        }
+        {
 #pragma unroll
           for (int e = 0; e < E; ++e) o[e] = one_rounding<T, RAG && !DROP>(v[j][k][e] * inv + fill);
           if constexpr (RAG) {
@@ -754,23 +770,19 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
           }
         }
         if constexpr (DROP) {
-          // exact zeros need no draw (wave-uniform test)
-          if (!none_visible[j][k] || empty) {
-            if constexpr (kPairDraw || RAG) {
-              uint32_t keep;
-              if constexpr (RAG)
-                keep = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk)) &
-                       ~(empty ? 0u : mbits[j][k]);
-              else
-                keep = paired ? keepk[k] : chunk_keep_bits<E>(row[j], g.sk, c, d);
+          if constexpr (kPairDraw || RAG) {
+            uint32_t keep;
+            if constexpr (RAG)
+              keep = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk)) &
+                     ~(empty ? 0u : mbits[j][k]);
+            else
+              keep = paired ? keepk[k] : chunk_keep_bits<E>(row[j], g.sk, c, d);
 #pragma unroll
-              for (int e = 0; e < E; ++e) o[e] = keep_or_zero(o[e] * d.scale, keep, e);
-            } else {
-              const KeepWords<E> keep = chunk_keep_words<E>(row[j], g.sk, c, d);
+            for (int e = 0; e < E; ++e) o[e] = keep_or_zero(o[e], keep, e);
+          } else {
+            const KeepWords<E> keep = chunk_keep_words<E>(row[j], g.sk, c, d);
 #pragma unroll
-              for (int e = 0; e < E; ++e)
-                o[e] = keep.kept(e) ? o[e] * d.scale : 0.f;
-            }
+            for (int e = 0; e < E; ++e) o[e] = keep.kept(e) ? o[e] : 0.f;
           }
         }
         store_chunk<T, E, RAG>(yr + chunk_key<E, RAG>(c, g.sk), o);
@@ -928,15 +940,14 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
       const int c = c0 + k * cstride;
       KeepWords<E> keep;
       uint32_t keep_bits = 0;
-      int dup = 0;
       if constexpr (RAG) {
         // (hidden keys take their gradient for zero)
         keep_bits = row_keep_bits(kb, row[j], g.sk, chunk_key<E, RAG>(c, g.sk)) & ~mbits[j][k];
-        dup = dup_keys<E, RAG>(c, g.sk);
       } else {
         keep = chunk_keep_words<E>(row[j], g.sk, c, d);
       }
       float bf[kBias ? E : 1];
+      float pd[E];
       if constexpr (kBias) unpack_bias_raw<T, E>(braw[j][k], bias_f32, bf);
       xraw[j][k].unpack(yv[j][k]);
       graw[j][k].unpack(gv[j][k]);
@@ -958,7 +969,7 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
           p = __builtin_amdgcn_exp2f(sub_rn(mul_rn(yv[j][k][e], c2), rmax[j])) * rinv[j];
         }
         if (empty) p = -rinv[j];
-        if ((mbits[j][k] >> e) & 1u) p = 0.f;
+        p = keep_or_zero(p, ~mbits[j][k], e);
         float dp;
         if constexpr (RAG)
           dp = keep_or_zero(mul_rn(gv[j][k][e], d.scale), keep_bits, e);
@@ -967,10 +978,11 @@ __global__ __launch_bounds__(1024) void softmax_dropout_bwd_kernel(
         yv[j][k][e] = p;
         gv[j][k][e] = dp;
         if constexpr (RAG)
-          a += e < dup ? 0.f : p * dp;
+          pd[e] = p * dp;
         else
           a += p * dp;
       }
+      if constexpr (RAG) a = add_chunk<E, RAG>(a, pd, c, g.sk);
     }
     s[j] = a;
   }
@@ -1148,12 +1160,14 @@ __global__ __launch_bounds__(1024) void softmax_bwd_kernel(
           }
         }
       }
+      if constexpr (RAG) {
+        float yg[E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        if constexpr (RAG)
-          a += e < dup_keys<E, RAG>(c0 + k * cstride, g.sk) ? 0.f : yv[j][k][e] * gv[j][k][e];
-        else
-          a += yv[j][k][e] * gv[j][k][e];
+        for (int e = 0; e < E; ++e) yg[e] = yv[j][k][e] * gv[j][k][e];
+        a = add_chunk<E, RAG>(a, yg, c0 + k * cstride, g.sk);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) a += yv[j][k][e] * gv[j][k][e];
       }
     }
     s[j] = a;
@@ -1244,15 +1258,16 @@ __global__ __launch_bounds__(256) void softmax_fwd_generic_kernel(
     s = block_reduce_256(s, sh, false);
     const float inv = empty ? 0.f : row_recip(s);
     const float fill = empty ? g.inv_sk : 0.f;
+    const float factor = DROP ? inv * d.scale : inv, rest = DROP ? fill * d.scale : fill;
     for (int i = threadIdx.x; i < g.sk; i += 256) {
       float p = 0.f;
       if (!is_hidden(i)) p = __builtin_amdgcn_exp2f(expo(i, m));
-      float o = p * inv + fill;
+      float o = p * factor + rest;
       // (a key beyond the diagonal is an exact zero in a NaN row, too)
       if (kBias && is_hidden(i)) o = 0.f;
       if constexpr (kBias) o = pinned(o);
       if constexpr (DROP)
-        o = keep_element(row * g.sk + i, d) ? o * d.scale : 0.f;
+        o = keep_element(row * g.sk + i, d) ? o : 0.f;
       yr[i] = io<T>::to_scalar(o);
     }
     if constexpr (DROP) {
@@ -1381,11 +1396,11 @@ __global__ __launch_bounds__(256) void softmax_fwd_tiny_kernel(
     if (!in_row) continue;
     const float inv = empty ? 0.f : row_recip(s);
     const float fill = empty ? g.inv_sk : 0.f;
-    float o = p * inv + fill;
+    float o = DROP ? p * (inv * d.scale) + fill * d.scale : p * inv + fill;
     // (a key beyond the diagonal is an exact zero in a NaN row, too)
     if (kBias && i >= visible) o = 0.f;
     if constexpr (kBias) o = pinned(o);
-    if constexpr (DROP) o = keep_element(row * g.sk + i, d) ? o * d.scale : 0.f;
+    if constexpr (DROP) o = keep_element(row * g.sk + i, d) ? o : 0.f;
     y[row * g.sk + i] = io<T>::to_scalar(o);
     if constexpr (DROP) {
       if (i == 0) {
