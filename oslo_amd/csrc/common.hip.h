@@ -353,8 +353,7 @@ __device__ __forceinline__ Welford wave_welford(Welford v) {
   return chan_merge(chan_merge(r[0], r[1]), chan_merge(r[2], r[3]));
 }
 
-// The same all-reduce when every lane holds the same number of values
-// (`per_lane`): the merge of two equal-sized sets needs no division and is
+// The same when every set holds the same number of values: the merge of two equal-sized sets needs no division and is
 // symmetric, mean = (ma + mb) / 2, M2 = M2a + M2b + (mb - ma)^2 * n / 2.
 __device__ __forceinline__ void merge_equal(float &mean, float &m2, float omean,
                                             float om2, float n_each) {
@@ -363,25 +362,32 @@ __device__ __forceinline__ void merge_equal(float &mean, float &m2, float omean,
   m2 = (m2 + om2) + d * d * (0.5f * n_each);
 }
 
+// Over a whole wave: the six steps of the reductions above, six instructions
+// each with no wait state between them (74 instructions through merge_equal and
+// v_readlane, 38 here); the result is that of lane 63.
+#define OSLO_WELFORD_STEP(CTRL, ROWS, C)                                          \
+  "v_sub_f32_dpp %2, %0, %0 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"         \
+  "v_add_f32_dpp %0, %0, %0 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"         \
+  "v_add_f32_dpp %1, %1, %1 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"         \
+  "v_mul_f32 %0, 0.5, %0\n\tv_mul_f32 %2, %2, %2\n\tv_fmac_f32 %1, " C ", %2\n\t"
 __device__ __forceinline__ Welford wave_welford_equal(float mean, float m2,
                                                       float per_lane) {
-  merge_equal(mean, m2, dpp_mov<kDppQuadSwap1>(mean),
-              dpp_mov<kDppQuadSwap1>(m2), per_lane);
-  merge_equal(mean, m2, dpp_mov<kDppQuadSwap2>(mean),
-              dpp_mov<kDppQuadSwap2>(m2), 2.f * per_lane);
-  merge_equal(mean, m2, dpp_mov<kDppRowHalfMirror>(mean),
-              dpp_mov<kDppRowHalfMirror>(m2), 4.f * per_lane);
-  merge_equal(mean, m2, dpp_mov<kDppRowMirror>(mean),
-              dpp_mov<kDppRowMirror>(m2), 8.f * per_lane);
-  float ma = readlane(mean, 0), qa = readlane(m2, 0);
-  float mb = readlane(mean, 32), qb = readlane(m2, 32);
-  merge_equal(ma, qa, readlane(mean, 16), readlane(m2, 16), 16.f * per_lane);
-  merge_equal(mb, qb, readlane(mean, 48), readlane(m2, 48), 16.f * per_lane);
-  merge_equal(ma, qa, mb, qb, 32.f * per_lane);
+  const float c = 0.5f * per_lane;
+  float d;
+  asm("s_nop 4\n\t"
+      OSLO_WELFORD_STEP("quad_perm:[1,0,3,2]", "0xf", "%3")
+      OSLO_WELFORD_STEP("quad_perm:[2,3,0,1]", "0xf", "%4")
+      OSLO_WELFORD_STEP("row_half_mirror", "0xf", "%5")
+      OSLO_WELFORD_STEP("row_mirror", "0xf", "%6")
+      OSLO_WELFORD_STEP("row_bcast:15", "0xa", "%7")
+      OSLO_WELFORD_STEP("row_bcast:31", "0xc", "%8")
+      "s_nop 1"
+      : "+v"(mean), "+v"(m2), "=&v"(d)
+      : "s"(c), "s"(2.f * c), "s"(4.f * c), "s"(8.f * c), "s"(16.f * c), "s"(32.f * c));
   Welford w;
   w.n = 64.f * per_lane;
-  w.mean = ma;
-  w.m2 = qa;
+  w.mean = readlane(mean, 63);
+  w.m2 = readlane(m2, 63);
   return w;
 }
 
@@ -550,6 +556,17 @@ dropout_keep_bits(uint64_t group, uint64_t seed, uint64_t offset,
   }
   return bits;
 #endif
+}
+
+// All ones where bit e of `bits` is set, else zero.  (Hidden from the optimiser,
+// which would make the two instructions that use it a test, a compare and a
+// select, with two wait states between the last two.)
+__device__ __forceinline__ uint32_t bit_mask(uint32_t bits, int e) {
+  return pinned((uint32_t)__builtin_amdgcn_sbfe((int)bits, e, 1));
+}
+// v where bit e of the keep bits is set, else +0
+__device__ __forceinline__ float keep_or_zero(float v, uint32_t keep, int e) {
+  return __uint_as_float(__float_as_uint(v) & bit_mask(keep, e));
 }
 
 // Dropout parameters of one call.  Element i of the flattened tensor belongs

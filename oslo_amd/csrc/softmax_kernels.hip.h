@@ -399,16 +399,6 @@ __device__ __forceinline__ uint32_t row_keep_bits(const uint8_t *kb, int64_t row
   typedef uint16_t u16_any __attribute__((aligned(1)));
   return (uint32_t)*reinterpret_cast<const u16_any *>(kb + (at >> 3)) >> (at & 7u);
 }
-// All ones where bit e of `bits` is set, else zero.  (Hidden from the optimiser,
-// which would make the two instructions that use it a test, a compare and a
-// select, with two wait states between the last two.)
-__device__ __forceinline__ uint32_t bit_mask(uint32_t bits, int e) {
-  return pinned((uint32_t)__builtin_amdgcn_sbfe((int)bits, e, 1));
-}
-// v where bit e of the keep bits is set, else +0
-__device__ __forceinline__ float keep_or_zero(float v, uint32_t keep, int e) {
-  return __uint_as_float(__float_as_uint(v) & bit_mask(keep, e));
-}
 // -inf where bit e of the hidden keys' bits is set, else v
 __device__ __forceinline__ float hide(float v, uint32_t hidden, int e) {
   const uint32_t m = bit_mask(hidden, e);
