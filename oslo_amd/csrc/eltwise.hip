@@ -121,7 +121,14 @@ __global__ __launch_bounds__(256) void bias_gelu_fwd_kernel(
 }
 
 // Folds the per-lane column sums of the ty rows of the workgroup and writes
-// the partial row of this slot.  sh is [ty][kE][tx] floats (at most 8 KB).
+// the partial row of this slot.  Bound: the latency of the LDS reads, at the end
+// of every workgroup.  Each thread adds kE values whatever the shape of the tile:
+// by the first row of lanes alone, tiles of 16 lanes added 128 values in each
+// (whole backward, finalize included, bf16 [59, 448] 9.5 -> 5.3 us, [512, 768] 8.1
+// -> 5.9, [27294, 704] 28.3 -> 24.3).  sh is [ty][kE][tx] floats, with eight
+// columns of padding from 32 lanes on, so that the lanes that read kE values of
+// neighbouring chunks meet 64 different banks.
+template <int kE> constexpr int kFoldFloats = 320 * kE;  // 64 rows of 32 + 8 columns at most
 template <int kE>
 __device__ __forceinline__ void write_col_partials(const float *acc, float *sh,
                                                    float *__restrict__ part,
@@ -129,18 +136,18 @@ __device__ __forceinline__ void write_col_partials(const float *acc, float *sh,
                                                    const EltPos &ps) {
   const int cx = threadIdx.x % g.tx;
   const int ry = threadIdx.x / g.tx;
+  const int stride = g.tx >= 32 ? g.tx + 8 : g.tx;
 #pragma unroll
-  for (int e = 0; e < kE; ++e) sh[(ry * kE + e) * g.tx + cx] = acc[e];
+  for (int e = 0; e < kE; ++e) sh[(ry * kE + e) * stride + cx] = acc[e];
   __syncthreads();
-  if (ry == 0 && ps.cc < g.nchunks) {
-    float o[kE];
-#pragma unroll
-    for (int e = 0; e < kE; ++e) {
-      float s = sh[e * g.tx + cx];
-      for (int q = 1; q < g.ty; ++q) s += sh[(q * kE + e) * g.tx + cx];
-      o[e] = s;
-    }
-    store_chunk<float, kE>(part + ps.slot * g.cols + (int64_t)ps.cc * kE, o);
+  const int64_t tile0 = (int64_t)(ps.cc - cx) * kE;  // first column of the tile
+  for (int i = threadIdx.x; i < kE * g.tx; i += 256) {
+    const int e = i & (kE - 1), c = i / kE;
+    const int64_t col = tile0 + i;
+    if (col >= g.cols) break;
+    float s = sh[e * stride + c];
+    for (int q = 1; q < g.ty; ++q) s += sh[(q * kE + e) * stride + c];
+    part[ps.slot * g.cols + col] = s;
   }
 }
 
@@ -150,7 +157,7 @@ __global__ __launch_bounds__(256) void bias_gelu_bwd_kernel(
     const T *__restrict__ bias, T *__restrict__ dx, float *__restrict__ part,
     EltGeom g) {
   constexpr int kE = io<T>::EPV;
-  __shared__ float sh[256 * kE];
+  __shared__ float sh[kFoldFloats<kE>];
   const EltPos ps = elt_pos(g);
   float b[kE], acc[kE];
 #pragma unroll
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(256) void bias_dropout_add_fwd_kernel(
 #pragma unroll
         for (int e = 0; e < kE; ++e) {
           float t = HAS_BIAS ? v[u][e] + b[e] : v[u][e];
-          if constexpr (DROP) t = (keep >> e) & 1u ? t * d.scale : 0.f;
+          if constexpr (DROP) t = keep_or_zero(t * d.scale, keep, e);
           o[e] = HAS_RES ? t + rv[u][e] : t;
         }
         store_chunk<T, kE>(out + r * g.cols + coff, o);
@@ -267,7 +274,7 @@ __global__ __launch_bounds__(256) void bias_dropout_add_bwd_kernel(
     EltGeom g, DropArgs d) {
   constexpr int kE = io<T>::EPV;
   d = resolve_drop(d);
-  __shared__ float sh[256 * kE];
+  __shared__ float sh[kFoldFloats<kE>];
   const EltPos ps = elt_pos(g);
   float acc[kE];
 #pragma unroll
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(256) void bias_dropout_add_bwd_kernel(
 #pragma unroll
           for (int e = 0; e < kE; ++e) {
             float t = gv[u][e];
-            if constexpr (DROP) t = (keep >> e) & 1u ? t * d.scale : 0.f;
+            if constexpr (DROP) t = keep_or_zero(t * d.scale, keep, e);
             o[e] = t;
           }
           store_chunk_readback<T, kE>(dx != nullptr ? dx + r * g.cols + coff : nullptr, o);
@@ -546,16 +553,24 @@ static inline void eltwise_tile(int64_t cols, int E, int *tx, int *ty, int *tile
 constexpr int kBwdTileMax = 128;
 constexpr int kBwdWorkgroupsPerCu = 3;  // the most a launch takes
 
-static int64_t colsum_parts_eltwise_e(int64_t rows, int64_t cols, int E,
+// Partial rows of a launch: slots of at least 16 rows, and with few rows finer
+// ones as long as they are no more than 128, which the finalize launch adds up in
+// one step (384 instead of 55 at [867, 2048]: 7.5 -> 8.5 us).
+constexpr int64_t kFineParts = 128;
+
+static int64_t colsum_parts_eltwise_e(int64_t rows, int64_t cols, int E, bool fine = true,
                                       int per_cu = kBwdWorkgroupsPerCu) {
   int tx, ty, tiles;
   eltwise_tile(cols, E, &tx, &ty, &tiles, kBwdTileMax);
   int64_t parts = g_tune.eltwise_rowgroups > 0
                       ? g_tune.eltwise_rowgroups
                       : ((int64_t)device_cu_count() * per_cu) / tiles;
-  const int64_t min_band =
-      g_tune.eltwise_rowgroups > 0 ? ty : (16 > ty ? 16 : ty);
-  const int64_t maxp = ceil_div(rows, min_band);
+  const int64_t min_band = g_tune.eltwise_rowgroups > 0 || ty > 16 ? ty : 16;
+  int64_t maxp = ceil_div(rows, min_band);
+  if (fine && g_tune.eltwise_unroll == 0 && maxp < kFineParts) {
+    const int64_t steps = ceil_div(rows, (int64_t)ty);
+    maxp = steps < kFineParts ? steps : kFineParts;
+  }
   if (parts > maxp) parts = maxp;
   if (parts < 1) parts = 1;
   return parts;
@@ -568,17 +583,36 @@ int64_t colsum_parts_eltwise(int64_t rows, int64_t cols) {
   return a > b ? a : b;
 }
 
-static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int unroll, int E,
+// The geometry of a backward, and the chunks per lane and operand in flight:
+// `unroll`, or fewer where the rows do not make a step of that height for every
+// workgroup of the launch.  Few rows then spread over more workgroups: such a
+// launch is bound by what one lane does in a row, each chunk with its draw.
+// (bf16 [269, 2048], finalize included: bias-GeLU 9.0 -> 7.1 us, bias-dropout-add
+// 8.2 -> 6.9; fp32 [108, 768] 5.9 -> 5.3 and 6.5 -> 5.5.)
+static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int *unroll, int E,
                                        int per_cu = kBwdWorkgroupsPerCu) {
   EltGeom g;
   g.rows = rows;
   g.cols = cols;
   g.nchunks = (int)(cols / E);
   eltwise_tile(cols, E, &g.tx, &g.ty, &g.tiles, kBwdTileMax);
-  const int64_t nsteps = ceil_div(rows, (int64_t)g.ty * unroll);
-  g.slots = colsum_parts_eltwise_e(rows, cols, E, per_cu);
-  if (g.slots > nsteps) g.slots = nsteps;
+  const int64_t most = colsum_parts_eltwise_e(rows, cols, E, true, per_cu);
+  if (g_tune.eltwise_unroll == 0)
+    while (*unroll > 1 && ceil_div(rows, (int64_t)g.ty * *unroll) < most) *unroll /= 2;
+  const int64_t nsteps = ceil_div(rows, (int64_t)g.ty * *unroll);
+  g.slots = most < nsteps ? most : nsteps;
   return g;
+}
+
+// Bytes of partial rows of a launch.  A workspace that holds those of slots of at
+// least 16 rows, but not all of the finer ones, is used as far as it goes: any
+// number of slots covers the rows.
+static inline int64_t fit_workspace(EltGeom *g, int E, int per_cu, const void *ws, int64_t ws_bytes) {
+  const int64_t row = g->cols * (int64_t)sizeof(float);
+  const int64_t coarse = colsum_parts_eltwise_e(g->rows, g->cols, E, false, per_cu);
+  if (ws != nullptr && ws_bytes < g->slots * row && coarse < g->slots && ws_bytes >= coarse * row)
+    g->slots = ws_bytes / row;
+  return g->slots * row;
 }
 
 static inline EltGeom eltwise_geom_fwd(int64_t rows, int64_t cols, int unroll, int E) {
@@ -692,21 +726,22 @@ static int run_bias_gelu_bwd(const void *gr, const void *x, const void *bias,
   // in turn took 458 us with the narrow window against 433, the backward 300
   // when x, the gradient and dx started on one phase, and the cause is not known.
   const bool narrow = sizeof(T) == 2 && rows * cols * (int64_t)sizeof(T) < (256ll << 20);
-  const int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4, sizeof(T) == 2);
-  const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE, narrow ? 2 : kBwdWorkgroupsPerCu);
-  const int64_t parts = g.slots;
-  const int64_t nblocks = parts * g.tiles;
-  OSLO_REQUIRE(nblocks <= max_workgroups(256), "bias_gelu bwd: too many workgroups");
-  const dim3 grid((unsigned)nblocks);
+  int unroll = eltwise_unroll(narrow ? 2 : sizeof(T) == 2 ? 8 : 4, sizeof(T) == 2);
+  const int per_cu = narrow ? 2 : kBwdWorkgroupsPerCu;
+  EltGeom g = eltwise_geom_bwd(rows, cols, &unroll, kE, per_cu);
   float *part = nullptr;
   if (dbias != nullptr) {
-    const int64_t need = parts * cols * (int64_t)sizeof(float);
+    const int64_t need = fit_workspace(&g, kE, per_cu, ws, ws_bytes);
     if (ws == nullptr || ws_bytes < need)
       return fail(OSLO_ERR_WORKSPACE,
                   "bias_gelu bwd: workspace of %lld bytes needed, %lld given",
                   (long long)need, (long long)ws_bytes);
     part = (float *)ws;
   }
+  const int64_t parts = g.slots;
+  const int64_t nblocks = parts * g.tiles;
+  OSLO_REQUIRE(nblocks <= max_workgroups(256), "bias_gelu bwd: too many workgroups");
+  const dim3 grid((unsigned)nblocks);
   OSLO_ELT_U8(unroll, {
     // (eight steps in flight are built for the 16-bit types, whose default it is)
     if constexpr (U < 8 || sizeof(T) == 2) {
@@ -804,15 +839,11 @@ static int run_bda_bwd(const void *gr, void *dx, void *dbias, void *ws,
     if (rc != OSLO_OK || dbias == nullptr) return rc;
     return generic_colsum_of_stored<T>(dx, dbias, ws, ws_bytes, rows, cols, st);
   }
-  const int unroll = eltwise_unroll(4);
-  const EltGeom g = eltwise_geom_bwd(rows, cols, unroll, kE);
-  const int64_t parts = g.slots;
-  const int64_t nblocks = parts * g.tiles;
-  OSLO_REQUIRE(nblocks <= max_workgroups(256), "bias_dropout_add bwd: too many workgroups");
-  const dim3 grid((unsigned)nblocks);
+  int unroll = eltwise_unroll(4);
+  EltGeom g = eltwise_geom_bwd(rows, cols, &unroll, kE);
   float *part = nullptr;
   if (dbias != nullptr) {
-    const int64_t need = parts * cols * (int64_t)sizeof(float);
+    const int64_t need = fit_workspace(&g, kE, kBwdWorkgroupsPerCu, ws, ws_bytes);
     if (ws == nullptr || ws_bytes < need)
       return fail(OSLO_ERR_WORKSPACE,
                   "bias_dropout_add bwd: workspace of %lld bytes needed, %lld "
@@ -820,6 +851,10 @@ static int run_bda_bwd(const void *gr, void *dx, void *dbias, void *ws,
                   (long long)need, (long long)ws_bytes);
     part = (float *)ws;
   }
+  const int64_t parts = g.slots;
+  const int64_t nblocks = parts * g.tiles;
+  OSLO_REQUIRE(nblocks <= max_workgroups(256), "bias_dropout_add bwd: too many workgroups");
+  const dim3 grid((unsigned)nblocks);
   OSLO_ELT_U(unroll, {
     if (drop)
       bias_dropout_add_bwd_kernel<T, U, true><<<grid, 256, 0, st>>>(

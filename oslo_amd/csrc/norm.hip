@@ -1380,12 +1380,12 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
   // waves: the workgroups (one per CU) move in steps of P * rpb rows
   // ([3048, 1024] bf16, 8 slots, two steps, 74 % of their rows -> 4 slots, three
   // full steps: 11.5 -> 10.0 us, fused with dropout 15.4 -> 13.4; [1790, 4096]
-  // 18.2 -> 16.3 and 26.6 -> 23.0).  16-bit rows of eight waves take one slot at
-  // any batch: two rows then do not wait at one barrier ([16384, 4096] fused with
-  // dropout 119 -> 113.5 us; the plain backward, which has to add in the same
-  // order, 70.1 / 70.2).
+  // 18.2 -> 16.3 and 26.6 -> 23.0).  (One slot for 16-bit rows of eight waves at any
+  // batch gains 3 % in the fused backward of [16384, 4096], whose two rows then do
+  // not wait at one barrier, and costs the plain one, which has to add in the same
+  // order, 2 %.)
+  const int coarse_rpb = sp.rpb;
   if (upr == 0 && g_tune.norm_bwd_waves == 0) {
-    if (E == 8 && sp.wpr == 8) sp.rpb = 1;
     auto busy = [&](int rpb) {
       const int64_t step = colsum_parts_norm(n1, n2) * rpb;
       return (double)n1 / (double)(ceil_div(n1, step) * step);
@@ -1412,7 +1412,13 @@ static int launch_norm_bwd(const void *dy, const void *x, const float *mean,
   }
   const int narr = NARR + (fev.want_dbias ? 1 : 0);
   if (want_params) {
-    const int64_t need = (int64_t)narr * P * n2 * (int64_t)sizeof(float);
+    const int64_t row = (int64_t)narr * n2 * (int64_t)sizeof(float);
+    // (a workspace that holds the partial rows of the wider slots, but not all of
+    //  these, is used as far as it goes: any number of workgroups covers the rows)
+    const int64_t coarse = ceil_div(n1, (int64_t)coarse_rpb * (lpr < kWave ? kWave / lpr : 1));
+    if (ws != nullptr && ws_bytes < P * row && coarse < P && ws_bytes >= coarse * row)
+      P = ws_bytes / row;
+    const int64_t need = P * row;
     if (ws == nullptr || ws_bytes < need)
       return fail(OSLO_ERR_WORKSPACE,
                   "norm bwd: workspace of %lld bytes needed, %lld given",
