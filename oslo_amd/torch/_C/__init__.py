@@ -474,17 +474,37 @@ def tune(key, value):
     _ws_bytes_cache.clear()  # workspace sizes depend on the launch shapes
 
 
-# ---------------------------------------------------------------------------
-# LayerNorm / RMSNorm
-# ---------------------------------------------------------------------------
-class _LayerNormKernel:
-    """The ten functions of the reference's ``oslo_fused_layer_norm`` module."""
+class _Kernel:
+    """What the kernel objects of the layer ops share."""
 
     def __init__(self, lib):
         self._lib = lib
         self._calls = load_calls()
+        self._attributes = None
+
+    def replaced(self):
+        """Whether a method was replaced on this object (not on its class)."""
+        if len(self.__dict__) == self._attributes:
+            return False
+        # (a method that was put back is an attribute of the object still)
+        return any(getattr(v, "__func__", None) is not getattr(type(self), name)
+                   for name, v in self.__dict__.items() if hasattr(type(self), name))
+
+    def _built(self):
+        self._attributes = len(self.__dict__)
+
+
+# ---------------------------------------------------------------------------
+# LayerNorm / RMSNorm
+# ---------------------------------------------------------------------------
+class _LayerNormKernel(_Kernel):
+    """The ten functions of the reference's ``oslo_fused_layer_norm`` module."""
+
+    def __init__(self, lib):
+        super().__init__(lib)
         self._leases = [_leases(lib, op) for op in
                         (OSLO_OP_LN_BWD, OSLO_OP_RMS_BWD, OSLO_OP_BIAS_DROPOUT_ADD_NORM_BWD)]
+        self._built()
 
     # -- forward ----------------------------------------------------------
     def layer_norm_forward(self, input, normalized_shape, eps):
@@ -592,7 +612,7 @@ def empty_staggered(shape, dtype, device, k):
     return base[off:off + nbytes].view(dtype).view(tuple(shape))
 
 
-class _SoftmaxKernel:
+class _SoftmaxKernel(_Kernel):
     """The five functions of ``FusedScaleMaskSoftmaxBinder.cpp:111-127``.
 
     The reference admits fp16 / bf16 only (``:42-44, 84-86``); fp32 is accepted
@@ -602,8 +622,8 @@ class _SoftmaxKernel:
     """
 
     def __init__(self, lib):
-        self._lib = lib
-        self._calls = load_calls()
+        super().__init__(lib)
+        self._built()
 
     def fused_scaled_masked_softmax_forward(self, input, mask, scale_factor, causal=False):
         """``causal=True`` (not in the reference's shim) hides the keys beyond
@@ -717,12 +737,12 @@ class _SoftmaxKernel:
 # bias-GeLU and bias-dropout-add (TorchScript in the reference,
 # oslo/torch/nn/modules/functional.py:23-50, 295-298; native here)
 # ---------------------------------------------------------------------------
-class _FusedElementwiseKernel:
+class _FusedElementwiseKernel(_Kernel):
     def __init__(self, lib):
-        self._lib = lib
-        self._calls = load_calls()
+        super().__init__(lib)
         self._gelu_leases = _leases(lib, OSLO_OP_BIAS_GELU_BWD)
         self._dropout_leases = _leases(lib, OSLO_OP_BIAS_DROPOUT_ADD_BWD)
+        self._built()
 
     def bias_gelu_forward(self, input, bias):
         return self._calls.gelu_forward(input, bias)

@@ -20,7 +20,25 @@ from oslo_amd.torch._C import (
 
 """
 Autograd Functions
+
+The same Functions exist in native code (``csrc/torch_calls.cpp``, methods
+``ag_*``) and eager calls on GPU tensors go there: a Python Function costs 3 us
+forward and about 25 us in a backward pass, which is what bounded a small layer
+(340 us of host time for 130 us of kernels).  The ones below run what the native
+ones do not take: CPU tensors, calls under ``torch.jit`` tracing (which records a
+Python Function as such, and of a native one nothing), dropout under stream
+capture (whose state is a tensor) and dropout in place.
 """
+
+
+def _native(kernel, input):
+    """The native side of a kernel object where the call on ``input`` may take
+    its Functions, else None.  (The Python Functions call the methods of the
+    kernel object, which a caller may have replaced on it to watch or change
+    them; then they run.)"""
+    if input.is_cuda and not kernel.replaced() and torch._C._get_tracing_state() is None:
+        return kernel._calls
+    return None
 
 
 class _NullContext:
@@ -49,14 +67,14 @@ def _cast_if_autocast_enabled(*args):
 
 
 def _apply_outside_autocast(function, *args):
-    """``function.apply`` on operands cast to the autocast dtype with autocast
+    """``function`` on operands cast to the autocast dtype with autocast
     switched off (functional.py:249-284 of the reference); without an active
     autocast region neither step does anything and both are skipped."""
     if not torch.is_autocast_enabled("cuda"):
-        return function.apply(*args)
+        return function(*args)
     args = _cast_if_autocast_enabled(*args)
     with torch.amp.autocast("cuda", enabled=False):
-        return function.apply(*args)
+        return function(*args)
 
 
 def _gelu_fwd_torch(x):
@@ -676,30 +694,72 @@ User Functions
 """
 
 
+def _layer_norm_affine(input, weight, bias, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(False, False, input, weight, bias, normalized_shape, eps)
+    return _FusedLayerNormAffineFunction.apply(input, weight, bias, normalized_shape, eps)
+
+
+def _layer_norm(input, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(False, False, input, None, None, normalized_shape, eps)
+    return _FusedLayerNormFunction.apply(input, normalized_shape, eps)
+
+
+def _mixed_layer_norm_affine(input, weight, bias, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(False, True, input, weight, bias, normalized_shape, eps)
+    return _FusedLayerNormAffineMixedDtypesFunction.apply(input, weight, bias, normalized_shape, eps)
+
+
+def _rms_norm_affine(input, weight, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(True, False, input, weight, None, normalized_shape, eps)
+    return _FusedRMSNormAffineFunction.apply(input, weight, normalized_shape, eps)
+
+
+def _rms_norm(input, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(True, False, input, None, None, normalized_shape, eps)
+    return _FusedRMSNormFunction.apply(input, normalized_shape, eps)
+
+
+def _mixed_rms_norm_affine(input, weight, normalized_shape, eps):
+    calls = _native(get_layernorm_kernel(), input)
+    if calls is not None:
+        return calls.ag_norm(True, True, input, weight, None, normalized_shape, eps)
+    return _FusedRMSNormAffineMixedDtypesFunction.apply(input, weight, normalized_shape, eps)
+
+
 def fused_layer_norm_affine(input, weight, bias, normalized_shape, eps=1e-6):
-    return _apply_outside_autocast(_FusedLayerNormAffineFunction, input, weight, bias, normalized_shape, eps)
+    return _apply_outside_autocast(_layer_norm_affine, input, weight, bias, normalized_shape, eps)
 
 
 def fused_layer_norm(input, normalized_shape, eps=1e-6):
-    return _apply_outside_autocast(_FusedLayerNormFunction, input, normalized_shape, eps)
+    return _apply_outside_autocast(_layer_norm, input, normalized_shape, eps)
 
 
 def mixed_dtype_fused_layer_norm_affine(
     input, weight, bias, normalized_shape, eps=1e-6
 ):
-    return _apply_outside_autocast(_FusedLayerNormAffineMixedDtypesFunction, input, weight, bias, normalized_shape, eps)
+    return _apply_outside_autocast(_mixed_layer_norm_affine, input, weight, bias, normalized_shape, eps)
 
 
 def fused_rms_norm_affine(input, weight, normalized_shape, eps=1e-6):
-    return _apply_outside_autocast(_FusedRMSNormAffineFunction, input, weight, normalized_shape, eps)
+    return _apply_outside_autocast(_rms_norm_affine, input, weight, normalized_shape, eps)
 
 
 def fused_rms_norm(input, normalized_shape, eps=1e-6):
-    return _apply_outside_autocast(_FusedRMSNormFunction, input, normalized_shape, eps)
+    return _apply_outside_autocast(_rms_norm, input, normalized_shape, eps)
 
 
 def mixed_dtype_fused_rms_norm_affine(input, weight, normalized_shape, eps=1e-6):
-    return _apply_outside_autocast(_FusedRMSNormAffineMixedDtypesFunction, input, weight, normalized_shape, eps)
+    return _apply_outside_autocast(_mixed_rms_norm_affine, input, weight, normalized_shape, eps)
 
 
 _KERNEL_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
@@ -763,6 +823,9 @@ def fused_bias_gelu(x, bias):
     with _outside_autocast(x):
         if not fits:
             return _gelu_fwd_torch(x + bias)
+        calls = _native(get_fused_elementwise_kernel(), x)
+        if bias is not None and calls is not None:
+            return calls.ag_bias_gelu(x, bias)
         return _FusedBiasGeLUFunction.apply(x, bias)
 
 
@@ -795,9 +858,11 @@ def fused_bias_dropout_add(x, bias, residual, p, training, inplace=False):
             return y if residual is None else y + residual
         p_eff = float(p) if training else 0.0
         seed, offset = _next_philox_state(x.device) if p_eff > 0.0 else (0, 0)
-        return _FusedBiasDropoutAddFunction.apply(
-            x, bias, residual, p_eff, seed, offset, bool(inplace) and x is x_in
-        )
+        inplace = bool(inplace) and x is x_in
+        calls = _native(get_fused_elementwise_kernel(), x)
+        if calls is not None and not inplace and not isinstance(seed, torch.Tensor):
+            return calls.ag_dropout_add(x, bias, residual, p_eff, seed, offset)
+        return _FusedBiasDropoutAddFunction.apply(x, bias, residual, p_eff, seed, offset, inplace)
 
 
 def _bias_dropout_add_norm(rms, x, bias, residual, weight, norm_bias, normalized_shape,
@@ -823,10 +888,21 @@ def _bias_dropout_add_norm(rms, x, bias, residual, weight, norm_bias, normalized
     p_eff = float(p) if training else 0.0
     seed, offset = _next_philox_state(x.device) if p_eff > 0.0 else (0, 0)
     y, h = _apply_outside_autocast(
-        _FusedBiasDropoutAddNormFunction, x, bias, residual, weight, norm_bias,
+        _residual_norm, x, bias, residual, weight, norm_bias,
         normalized_shape, eps, p_eff, seed, offset, bool(rms),
     )
     return (y, h) if return_sum else y
+
+
+def _residual_norm(x, bias, residual, weight, norm_bias, normalized_shape, eps, p, seed, offset, rms):
+    calls = _native(get_layernorm_kernel(), x)
+    # (parts of this backward are those of the element-wise kernels)
+    if (calls is not None and not isinstance(seed, torch.Tensor)
+            and not get_fused_elementwise_kernel().replaced()):
+        return calls.ag_residual_norm(
+            rms, x, bias, residual, weight, norm_bias, normalized_shape, eps, p, seed, offset)
+    return _FusedBiasDropoutAddNormFunction.apply(
+        x, bias, residual, weight, norm_bias, normalized_shape, eps, p, seed, offset, rms)
 
 
 def fused_bias_dropout_add_layer_norm(x, bias, residual, weight, norm_bias,
@@ -853,13 +929,27 @@ def fused_bias_dropout_add_rms_norm(x, bias, residual, weight, normalized_shape,
 
 def scaled_upper_triang_masked_softmax(input, scale=1.0):
     """softmax(scale * input) under a causal mask; input is [attn_batches, sq, sk]."""
+    calls = _native(get_softmax_kernel(), input)
+    if calls is not None:
+        return calls.ag_causal(input, scale)
     return _ScaledUpperTriangMaskedSoftmax.apply(input, scale)
 
 
 def scaled_masked_softmax(input, mask, scale=1.0, causal=False):
     """softmax(scale * input) with `mask` (True = masked out); input is [b, np, sq, sk].
     With ``causal=True`` key j of query i is hidden when j > i + (sk - sq) as well."""
+    calls = _native(get_softmax_kernel(), input)
+    if calls is not None:
+        return calls.ag_masked(input, mask, scale, causal)
     return _ScaledMaskedSoftmax.apply(input, mask, scale, causal)
+
+
+def _masked_softmax_dropout(input, mask, scale, p, causal):
+    seed, offset = _next_philox_state(input.device)
+    calls = _native(get_softmax_kernel(), input)
+    if calls is not None and not isinstance(seed, torch.Tensor):
+        return calls.ag_dropout(input, mask, scale, p, seed, offset, causal)
+    return _ScaledMaskedSoftmaxDropout.apply(input, mask, scale, p, seed, offset, causal)
 
 
 def scaled_upper_triang_masked_softmax_dropout(input, scale=1.0, p=0.0, training=True):
@@ -867,9 +957,8 @@ def scaled_upper_triang_masked_softmax_dropout(input, scale=1.0, p=0.0, training
     _check_dropout_p(p)
     p_eff = float(p) if training else 0.0
     if p_eff == 0.0:
-        return _ScaledUpperTriangMaskedSoftmax.apply(input, scale)
-    seed, offset = _next_philox_state(input.device)
-    return _ScaledMaskedSoftmaxDropout.apply(input, None, scale, p_eff, seed, offset)
+        return scaled_upper_triang_masked_softmax(input, scale)
+    return _masked_softmax_dropout(input, None, scale, p_eff, False)
 
 
 def scaled_masked_softmax_dropout(input, mask, scale=1.0, p=0.0, training=True, causal=False):
@@ -878,9 +967,8 @@ def scaled_masked_softmax_dropout(input, mask, scale=1.0, p=0.0, training=True, 
     _check_dropout_p(p)
     p_eff = float(p) if training else 0.0
     if p_eff == 0.0:
-        return _ScaledMaskedSoftmax.apply(input, mask, scale, causal)
-    seed, offset = _next_philox_state(input.device)
-    return _ScaledMaskedSoftmaxDropout.apply(input, mask, scale, p_eff, seed, offset, causal)
+        return scaled_masked_softmax(input, mask, scale, causal)
+    return _masked_softmax_dropout(input, mask, scale, p_eff, causal)
 
 
 def scaled_bias_softmax(input, bias, scale=1.0, causal=False):
@@ -890,6 +978,9 @@ def scaled_bias_softmax(input, bias, scale=1.0, causal=False):
     finite value or -inf; a position bias [1, np, sq, sk]).  With
     ``causal=True`` key j of query i is hidden when j > i + (sk - sq) as well.
     `bias` may require a gradient."""
+    calls = _native(get_softmax_kernel(), input)
+    if calls is not None:
+        return calls.ag_term(input, bias, scale, causal)
     return _ScaledBiasSoftmax.apply(input, bias, scale, causal)
 
 
@@ -898,6 +989,9 @@ def scaled_bias_softmax_dropout(input, bias, scale=1.0, p=0.0, training=True, ca
     _check_dropout_p(p)
     p_eff = float(p) if training else 0.0
     if p_eff == 0.0:
-        return _ScaledBiasSoftmax.apply(input, bias, scale, causal)
+        return scaled_bias_softmax(input, bias, scale, causal)
     seed, offset = _next_philox_state(input.device)
+    calls = _native(get_softmax_kernel(), input)
+    if calls is not None and not isinstance(seed, torch.Tensor):
+        return calls.ag_term_dropout(input, bias, scale, p_eff, seed, offset, causal)
     return _ScaledBiasSoftmaxDropout.apply(input, bias, scale, p_eff, seed, offset, causal)
