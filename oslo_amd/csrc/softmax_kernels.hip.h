@@ -1569,21 +1569,51 @@ static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
 }
 
 // Ragged rows: at least one chunk, at most 64 bytes of an operand per lane and
-// sixteen waves.  Rows of up to 8 and 16 chunks take as many lanes; up to 96
-// chunks a row can be held by 8, 16 or 32 lanes with three chunks each, which
-// idles fewer lanes but reads the row in pieces of 128, 256 or 512 bytes at odd
-// addresses (one line more per piece than aligned), or by one chunk per lane
-// of 32 lanes or a wave, in one piece.  `min_x3` is the smallest lane group
-// that takes three chunks: 8 where the arithmetic is what costs, i.e. with
-// dropout (bf16 180 keys, additive term: forward 118 against 190 us) and in
-// the plain forward, which adds in the order of the forward with dropout (381
-// keys: 91 against 103 us; 180 keys: 119 against 127, causal 140 against 106);
-// none in the plain backward (381 keys: 128 against 102 us; 700: 99 against 88).
+// sixteen waves.  Rows of up to 96 chunks are held by 8, 16 or 32 lanes with one
+// to three chunks each.  More chunks in fewer lanes share the reductions, the
+// cut of the row's ends and, with dropout, the Philox rounds among more rows of a
+// wave; against it stand the pieces that a row is read in, of 128, 256 or 512
+// bytes at odd addresses (one line more per piece than aligned), and lanes
+// without keys.  us at 300 MB: forward with dropout, plain forward, backward with
+// dropout, under the diagonal unless said; first as the line below it would hold
+// the rows (one chunk per lane, or what is named):
+//   two of 8 lanes    bf16 67 keys 257, 167, 267 / 149, 120, 175; 95: 179, 123, 193
+//                     / 126, 117, 172; 125, one chunk: 146, 100, 159 / 135, 142,
+//                     176; fp32 33: 215, 144, 218 / 129, 116, 161; 47, one chunk:
+//                     151, 108, 164 / 128, 126, 159; a term shared by the batch,
+//                     bf16 79, one chunk: 228, 175, 262 / 237, 206, 300
+//   two of 16 lanes   bf16 201 keys 172, 121, 184 / 107, 100, 136; 253: 140, 99, 153
+//                     / 98, 97, 135; fp32 111: 131, 97, 142 / 102, 94, 129; 127, one
+//                     chunk: 117, 90, 130 / 102, 101, 128, with a term 125: 133,
+//                     103, 150 / 118, 114, 164; a term shared by the batch, bf16 223,
+//                     one chunk: 11 % faster, 12 and 15 % slower than two
+//   ... from three of 8, bf16 133 keys 162, 126, 184 / 135, 101, 153; fp32 79: 166,
+//                     121, 161 / 103, 99, 137; but 16 bits, three of 8: key mask 157
+//                     keys 160, 157, 206 / 179, 130, 202, term 133: 179, 159, 248 /
+//                     213, 146, 253
+//   three of 16       bf16 261 keys against two of 32: 108, 98, 137 / 131, 97, 148;
+//                     fp32 131: 109, 96, 132 / 114, 90, 134; 171, two of 32: 97, 94,
+//                     127 / 95, 86, 121; key mask 173: 111, 108, 146 / 119, 104, 140
+//   two of 32         bf16 389 keys 167, 121, 176 / 109, 86, 125; 507: 130, 98, 143
+//                     / 89, 84, 115; fp32 195: 154, 109, 146 / 89, 85, 117; 253:
+//                     121, 91, 118 / 86, 84, 111
+//   three of 32       bf16 517 keys against two of a wave: 90, 91, 120 / 128, 95, 140
+// Plain and dropout forward of a row hold it alike, so that they add in one order.
+// The plain backward has neither Philox rounds nor a row to cut twice, and takes
+// two chunks only where one leaves nearly half of the lanes idle: bf16 133 keys
+// 161 -> 140, 261: 161 -> 121, 341: 127 -> 118, but 181: 131 -> 140, 443: 110 -> 116;
+// fp32 67: 146 -> 139, 131: 146 -> 120, 171: 121 -> 116, but 189: 114 -> 116.
 // Two rows (of waves or sets of lane groups) to a workgroup: the line that two
 // rows share is then written through one L2 (bf16 1003 keys: causal backward
 // 102 -> 88 us, dense 156 -> 130 us; four measure the same, and slower beyond
 // 2048 keys).
-static SoftmaxPlan plan_softmax_ragged(int64_t sk, int E, int min_x3) {
+enum RaggedPass { kRaggedFwd, kRaggedDropBwd, kRaggedBwd };
+template <typename T, int MODE>
+static SoftmaxPlan plan_softmax_ragged(int64_t sk, RaggedPass pass, bool shared_term = false) {
+  constexpr int E = io<T>::EPV;
+  constexpr bool k16 = sizeof(T) == 2;
+  constexpr bool term = MODE == kModeBias, masked = MODE == kModeMasked;
+  const bool fwd = pass == kRaggedFwd, plain = pass == kRaggedBwd;
   SoftmaxPlan p{0, 1, 1, 1, kWave, false};
   if (sk < E) return p;
   const int64_t nchunks = ceil_div(sk, E);
@@ -1591,28 +1621,49 @@ static SoftmaxPlan plan_softmax_ragged(int64_t sk, int E, int min_x3) {
   if (wpr > 16) return p;
   p.ok = true;
   p.wpr = (int)wpr;
-  p.vpl = 1;
+  const auto group = [&](int chunks, int lanes) {
+    p.vpl = chunks;
+    p.lpr = lanes;
+  };
+  // (16-bit rows behind a mask or with a term: up to where three of 8 lanes
+  //  remain the better)
+  const bool shared = term && shared_term;
+  const int three8 = !k16 || plain ? 0 : fwd ? (term || masked ? 20 : 0) : (term ? 18 : 0);
   if (nchunks <= 8) {
-    p.lpr = 8;
+    group(1, 8);
+  } else if (nchunks <= (shared ? (k16 ? 9 : 8) : k16 ? 12 : 10) && !plain) {
+    group(2, 8);
   } else if (nchunks <= 16) {
-    p.lpr = 16;
-  } else if (nchunks <= 24 && min_x3 <= 8) {
-    p.lpr = 8;
-    p.vpl = 3;
+    group(1, 16);
+  } else if (nchunks <= three8) {
+    group(3, 8);
+  } else if (nchunks <= (plain ? 18 : shared ? 24 : k16 ? 32 : 28)) {
+    group(2, 16);
   } else if (nchunks <= 32) {
-    p.lpr = 32;
-  } else if (nchunks <= 48 && min_x3 <= 16) {
-    p.lpr = 16;
-    p.vpl = 3;
-  } else if (nchunks > 64 && nchunks <= 96 && min_x3 <= 32) {
-    p.lpr = 32;
-    p.vpl = 3;
+    group(1, 32);
+  } else if (nchunks <= (k16 || masked ? 48 : 40) && !plain) {
+    group(3, 16);
+  } else if (nchunks <= (plain ? 44 : 64)) {
+    group(2, 32);
+  } else if (nchunks > 64 && nchunks <= 96 && !plain) {
+    group(3, 32);
   } else {
-    p.vpl = (int)ceil_div(nchunks, kWave * wpr);
+    group((int)ceil_div(nchunks, kWave * wpr), kWave);
   }
   p.rpb = g_tune.softmax_rows_per_block > 0 ? g_tune.softmax_rows_per_block : 2;
   while (p.rpb * p.wpr > 16) --p.rpb;
   return p;
+}
+// ... and the builds that it can come out with
+template <typename T, int MODE>
+constexpr bool ragged_plan_reaches(int vpl, int lpr, RaggedPass pass) {
+  constexpr bool k16 = sizeof(T) == 2, term = MODE == kModeBias, masked = MODE == kModeMasked;
+  const bool plain = pass == kRaggedBwd;
+  if (lpr == kWave) return vpl > 1 || plain;
+  if (vpl == 3 && lpr == 8) return k16 && (term || (masked && pass == kRaggedFwd)) && !plain;
+  if (vpl == 3) return !plain;
+  if (vpl == 2) return !plain || lpr != 8;
+  return lpr != 32 || plain || !k16 || term;
 }
 #define OSLO_SM_RAGGED_CASES(LAUNCH)       \
   if (pl.lpr == 8 && pl.vpl == 1) {        \
@@ -1621,6 +1672,12 @@ static SoftmaxPlan plan_softmax_ragged(int64_t sk, int E, int min_x3) {
     LAUNCH(1, 16);                         \
   } else if (pl.lpr == 32 && pl.vpl == 1) { \
     LAUNCH(1, 32);                         \
+  } else if (pl.lpr == 8 && pl.vpl == 2) { \
+    LAUNCH(2, 8);                          \
+  } else if (pl.lpr == 16 && pl.vpl == 2) { \
+    LAUNCH(2, 16);                         \
+  } else if (pl.lpr == 32 && pl.vpl == 2) { \
+    LAUNCH(2, 32);                         \
   } else if (pl.lpr == 8) {                \
     LAUNCH(3, 8);                          \
   } else if (pl.lpr == 16) {               \
@@ -1662,11 +1719,22 @@ static inline unsigned ragged_keep_lds(const SoftmaxPlan &pl) {
 // lanes of eight, or half of them, is 20 to 30 % slower than no limit (additive
 // term, fp32 80 keys forward 178 -> 142 us; causal fp16 8 keys 768 -> 627, 72 keys
 // 198 -> 163, 288 keys 203 -> 165; key mask, fp32 608 keys backward 189 -> 172).
+// So it is in the forward of ragged rows in lane groups, where a limit pays for
+// groups that are nearly full: three chunks with dropout under the diagonal (20
+// waves of full groups, 24 of 32 lanes in 16 bits: bf16 379 keys 108 -> 94 us, 765:
+// 91 -> 87, fp32 383: 88 -> 82), two without it (24, of 8 lanes 18: bf16 95 keys
+// 132 -> 117, 253: 99 -> 96, fp32 111: 99 -> 94; not behind a key mask, 95 keys 133
+// -> 144).  Behind a key mask three chunks in 8 or 16 lanes take 24 to 28 waves
+// (bf16 133 keys 160 -> 146, with dropout 167 -> 152; 305: 124 -> 111, fp32 173: 112
+// -> 108), but not 16 lanes in 16 bits with dropout (373 keys: 111, with 24 waves
+// 118).  A term that the batch shares is served by the L2s if fewer rows are under
+// way: 16 waves with dropout (bf16 133 keys 278 -> 249, 345: 191 -> 179, fp32 153:
+// 179 -> 156).
 // Additive terms with several rows to a wave, which waits for both operands: 96 KB
 // (bf16 392 keys 373 -> 327 us, fp16 352 keys 387 -> 362 at 900 MB).
 template <typename T, int MODE>
 static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bool drop,
-                                bool causal, bool ragged) {
+                                bool causal, bool ragged, bool shared_term = false) {
   constexpr bool k16 = sizeof(T) == 2;
   int kb;
   if (backward) {
@@ -1679,6 +1747,16 @@ static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bo
     if (MODE == kModeBias && pl.rpw > 1) kb = 96;
     if (drop) kb = 96;
     if (pl.wpr > 1 && kb < 96) kb = 96;
+    if (ragged && pl.vpl == 3 && pl.lpr < kWave && drop && MODE == kModeCausal)
+      return (int)((k16 && pl.lpr == 32 ? 24 : 20) * (int64_t)pl.vpl * pl.lpr /
+                   ceil_div(sk, io<T>::EPV));
+    if (ragged && pl.vpl == 3 && pl.lpr < 32) {
+      if (MODE == kModeMasked && !drop) return k16 && !causal ? 24 : 28;
+      if (MODE == kModeMasked && (!k16 || pl.lpr == 8)) return k16 && causal ? 28 : 24;
+      if (MODE == kModeBias && drop && shared_term) return 16;
+    }
+    if (ragged && pl.vpl == 2 && pl.lpr < kWave && !drop && MODE != kModeMasked)
+      return (int)((pl.lpr == 8 ? 18 : 24) * (int64_t)pl.vpl * pl.lpr / ceil_div(sk, io<T>::EPV));
     if (drop && k16) return 0;
   }
   int waves = kb / (pl.vpl * pl.rpw * (backward ? 2 : 1));  // (1 KB per chunk slot and operand)
@@ -1816,7 +1894,7 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
                        (reinterpret_cast<uintptr_t>(mask) % E) == 0) &&
                       (MODE != kModeBias || bias_vec_ok(g, mask));
   const bool ragged = !vec_ok;
-  if (ragged) pl = plan_softmax_ragged(g.sk, E, 8);
+  if (ragged) pl = plan_softmax_ragged<T, MODE>(g.sk, kRaggedFwd, g.batch_inner != 0);
   if (ragged && g.sk < E) {
     const dim3 grid = tiny_grid(g.rows);
     if (drop)
@@ -1850,7 +1928,8 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   const int64_t nblocks =
       ceil_div(g.rows, (int64_t)pl.rpb * pl.rpw * (kWave / pl.lpr));
   const unsigned occ = occupancy_lds(
-      softmax_waves_per_cu<T, MODE>(pl, g.sk, false, drop, g.causal, ragged), threads, nblocks);
+      softmax_waves_per_cu<T, MODE>(pl, g.sk, false, drop, g.causal, ragged, g.batch_inner != 0),
+      threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
   if (ragged) g.die_end = nblocks & ~(int64_t)63;
 #define OSLO_SM_FWD(VPL, RPW, LPR_)                                  \
@@ -1866,7 +1945,7 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   } else                                                             \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax fwd: no kernel for %d x %d chunks per lane", VPL, RPW)
 #define OSLO_SM_FWD_RAGGED(VPL, LPR_)                                \
-  do {                                                               \
+  if constexpr (ragged_plan_reaches<T, MODE>(VPL, LPR_, kRaggedFwd)) {    \
     if (drop)                                                        \
       softmax_fwd_kernel<T, VPL, 1, MODE, true, LPR_, true>          \
           <<<dim3((unsigned)grid), threads, keep_lds > occ ? keep_lds : occ, st>>>( \
@@ -1875,7 +1954,8 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
       softmax_fwd_kernel<T, VPL, 1, MODE, false, LPR_, true>         \
           <<<dim3((unsigned)grid), threads, occ, st>>>(                \
               (const T *)x, mask, (T *)y, nullptr, g, scale, d);     \
-  } while (0)
+  } else                                                             \
+    return fail(OSLO_ERR_UNSUPPORTED, "softmax fwd: no kernel for %d chunks in %d lanes", VPL, LPR_)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
   int64_t launch_blocks = nblocks;
   if (MODE == kModeBias && g.batch_inner && g_tune.softmax_bias_order == 3 &&
@@ -1942,7 +2022,7 @@ int launch_softmax_bwd(const void *dy, const void *y,
       return launch_softmax_bwd<T, kModeDense>(dy, y, nullptr, dx, g, scale, st);
     }
   }
-  if (ragged) pl = plan_softmax_ragged(g.sk, E, kWave);
+  if (ragged) pl = plan_softmax_ragged<T, MODE>(g.sk, kRaggedBwd);
   if (ragged && g.sk < E) {
     softmax_bwd_tiny_kernel<T><<<tiny_grid(g.rows), 256, 0, st>>>(
         (const T *)dy, (const T *)y, (T *)dx, g.rows, g.sk, scale);
@@ -1975,7 +2055,7 @@ int launch_softmax_bwd(const void *dy, const void *y,
   else                                                     \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
 #define OSLO_SM_BWD_RAGGED(VPL, LPR_)                      \
-  if constexpr ((VPL == 1 || LPR_ == kWave) &&             \
+  if constexpr (ragged_plan_reaches<T, MODE>(VPL, LPR_, kRaggedBwd) && \
                 ragged_bwd_plan_reaches<T, MODE>(VPL, LPR_)) \
     softmax_bwd_kernel<T, VPL, 1, MODE, LPR_, true>        \
         <<<dim3((unsigned)grid), threads, occ, st>>>(        \
@@ -2015,7 +2095,7 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
                        (reinterpret_cast<uintptr_t>(mask) % E) == 0) &&
                       (MODE != kModeBias || bias_vec_ok(g, mask));
   const bool ragged = !vec_ok;
-  if (ragged) pl = plan_softmax_ragged(g.sk, E, 8);
+  if (ragged) pl = plan_softmax_ragged<T, MODE>(g.sk, kRaggedDropBwd, g.batch_inner != 0);
   if (ragged && g.sk < E) {
     softmax_dropout_bwd_tiny_kernel<T, MODE><<<tiny_grid(g.rows), 256, 0, st>>>(
         (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d);
@@ -2052,9 +2132,12 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
   else                                                              \
     return fail(OSLO_ERR_UNSUPPORTED, "softmax dropout bwd: no kernel for %d x %d chunks per lane", VPL, RPW)
 #define OSLO_SM_DBWD_RAGGED(VPL, LPR_)                              \
-  softmax_dropout_bwd_kernel<T, VPL, 1, MODE, LPR_, true>           \
-      <<<dim3((unsigned)grid), threads, keep_lds > occ ? keep_lds : occ, st>>>( \
-          (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d)
+  if constexpr (ragged_plan_reaches<T, MODE>(VPL, LPR_, kRaggedDropBwd))     \
+    softmax_dropout_bwd_kernel<T, VPL, 1, MODE, LPR_, true>         \
+        <<<dim3((unsigned)grid), threads, keep_lds > occ ? keep_lds : occ, st>>>( \
+            (const T *)dy, (const T *)x, stats, mask, (T *)dx, g, scale, d); \
+  else                                                              \
+    return fail(OSLO_ERR_UNSUPPORTED, "softmax dropout bwd: no kernel for %d chunks in %d lanes", VPL, LPR_)
   // (rows of a term shared by the batch: one die per run of consecutive blocks)
   int64_t launch_blocks = nblocks;
   if (MODE == kModeBias && g.batch_inner && g_tune.softmax_bias_order == 3 &&
