@@ -1492,10 +1492,16 @@ struct SoftmaxPlan {
   bool ok;
 };
 
+// Rows that do not fill two chunks per lane of 8, 16 or 32 lanes and take them
+// all the same: the most chunks for each, and the fewest altogether.
+struct TwoChunks {
+  int most8, most16, most32, from;
+};
+
 // max_elems: elements of one operand a lane may hold (register budget).
 static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
                                 int default_rpw, int one_chunk_rpw,
-                                bool two_chunk_groups = false) {
+                                const TwoChunks *two = nullptr) {
   SoftmaxPlan p{0, 1, 1, 1, kWave, false};
   if (sk % E != 0) return p;
   const int64_t nchunks = sk / E;
@@ -1527,11 +1533,14 @@ static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
     }
   }
   // forward: rows of exactly 2 x 8 / 16 / 32 chunks (128, 256, 512 16-bit
-  // keys) as two chunks per lane in a lane group
-  if (two_chunk_groups && nchunks % 2 == 0 && g_tune.softmax_lanes_per_row != kWave &&
+  // keys) as two chunks per lane in a lane group, and rows that leave nearly
+  // half of the lanes without keys otherwise, or half of the second chunks then
+  if (two != nullptr && g_tune.softmax_lanes_per_row != kWave &&
       g_tune.softmax_lanes_per_row != 1) {
-    const int64_t q = nchunks / 2;
-    if (q == 8 || q == 16 || q == 32) {
+    const int64_t q = nchunks <= 8 ? 0 : nchunks <= 16 ? 8 : nchunks <= 32 ? 16 : nchunks <= 64 ? 32 : 0;
+    const bool part = g_tune.softmax_lanes_per_row == 0 && nchunks >= two->from &&
+                      nchunks <= (q == 8 ? two->most8 : q == 16 ? two->most16 : two->most32);
+    if (q != 0 && (nchunks == 2 * q || part)) {
       // one row set per wave without a mask tensor, two with one (measured)
       int want = g_tune.softmax_rows_per_wave > 0 ? g_tune.softmax_rows_per_wave : default_rpw;
       p.vpl = 2;
@@ -1885,7 +1894,19 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   //  with an additive term one measures faster, 186 against 232 us at
   //  [16,16,1024,1024] fp16, whether or not the loads wait for the term)
   const int default_rpw = MODE == kModeMasked ? 2 : 1;
-  SoftmaxPlan pl = plan_softmax(g.sk, E, cap, default_rpw, 4, true);
+  // (two chunks per lane against one in twice the lanes, us at 300 MB, forward with
+  //  dropout and plain forward.  16 bits, 72 keys: causal 167, 114 / 120, 109, key mask
+  //  166, 117 / 121, 117, term 185, 136 / 161, 129, but 80: 134, 98 / 116, 116; 136:
+  //  167, 112 / 110, 100, 180, 128 / 113, 110, 199, 145 / 167, 120; 160: 139, 101 / 99,
+  //  93, 156, 114 / 106, 101, but 176: 128, 100 / 98, 99, 145, 104 / 111, 111; 264: 153,
+  //  102 / 113, 95, 179, 131 / 115, 100, 189, 139 / 174, 124; 352: 120, 97 / 94, 81, 137,
+  //  101 / 104, 92, but 392: 107, 96 / 92, 94, 124, 96 / 104, 103.  fp32 68: 143, 94 / 104,
+  //  95, 148, 102 / 112, 112; 132: 127, 91 / 103, 94; 144: 115, 89 / 96, 85, 141, 99 / 98,
+  //  93; 176: 98, 83 / 83, 82.  Longer rows gain behind a key mask with the diagonal,
+  //  504 bf16 keys 106, 86 / 88, 83, but add in the order of the key mask alone)
+  constexpr bool k16 = sizeof(T) == 2;
+  constexpr TwoChunks two = {k16 ? 9 : 8, k16 ? 20 : 16, 44, k16 ? 9 : 34};
+  SoftmaxPlan pl = plan_softmax(g.sk, E, cap, default_rpw, 4, &two);
   if (!pl.ok && cap < kFwdMaxElems && MODE != kModeBias)
     pl = plan_softmax(g.sk, E, kFwdMaxElems, default_rpw, 4);
   if (MODE == kModeBias && pl.ok && pl.vpl * pl.rpw * E > kBiasMaxElems) pl.ok = false;

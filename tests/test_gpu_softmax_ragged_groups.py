@@ -1,6 +1,7 @@
-"""Ragged softmax rows of two and three chunks per lane in lane groups: lengths
-on both sides of every change of the group that depends on the type, the mask or
-the pass, through the checks (and tolerances) of the other ragged rows."""
+"""Softmax rows of two and three chunks per lane in lane groups: lengths on both
+sides of every change of the group that depends on the type, the mask or the
+pass, ragged and whole chunks, through the checks (and tolerances) of the other
+ragged rows."""
 import pytest
 import torch
 
@@ -21,6 +22,12 @@ LENGTHS = [(d, n * e + r) for d, e in ((BF16, 8), (F16, 8), (F32, 4)) for n in E
 @pytest.mark.parametrize("dtype,sk", LENGTHS)
 def test_lengths(device, dtype, sk):
     check_length(device, dtype, sk)
+
+
+@pytest.mark.parametrize("chunks", [9, 10, 16, 17, 20, 21, 33, 34, 44, 45, 49, 63])
+@pytest.mark.parametrize("dtype", [BF16, F16, F32])
+def test_whole_chunks(device, dtype, chunks):
+    check_length(device, dtype, chunks * (4 if dtype == F32 else 8))
 
 
 @pytest.mark.parametrize("dtype,sk", [c for c in LENGTHS if c[0] != F16])
