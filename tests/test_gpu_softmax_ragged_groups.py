@@ -5,6 +5,13 @@ ragged rows."""
 import pytest
 import torch
 
+from test_gpu_softmax import test_masked as check_masked
+from test_gpu_softmax_bias import test_bias_softmax as check_bias
+from test_gpu_softmax_bias import test_bias_softmax_dropout as check_bias_dropout
+from test_gpu_softmax_causal_masked import test_causal_masked as check_causal_masked
+from test_gpu_softmax_dropout import test_causal_dropout as check_causal_dropout
+from test_gpu_softmax_dropout import test_masked_dropout as check_masked_dropout
+from test_gpu_softmax import test_causal as check_causal
 from test_gpu_softmax_ragged import BF16, F16, F32
 from test_gpu_softmax_ragged import test_hidden_keys_held_twice as check_held_twice
 from test_gpu_softmax_ragged import test_lengths as check_length
@@ -53,3 +60,26 @@ def test_rounds_of_workgroups(device, dtype, sk):
     assert torch.equal(stats.view(b, per, 2), first.view(1, per, 2).expand(b, per, 2))
     dd = k.softmax_dropout_backward(xs, xs, stats, None, 0.5, 0.0, 5, 8)
     assert torch.equal(dd, dd[:1].expand_as(dd))
+
+
+@pytest.mark.parametrize("dtype,sk", [(d, n) for d in (BF16, F16) for n in (71, 199, 257)] + [(F32, n) for n in (35, 99, 129)])
+def test_a_term_shared_by_the_batch(device, dtype, sk):
+    """... keeps other groups."""
+    check_bias(device, 3, 2, 9, sk, dtype, 0.25, "t5", False)
+    check_bias_dropout(device, 3, 2, 9, sk, dtype, 0.25, "t5", False, 0.1)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_two_row_sets_of_one_chunk(device, dtype):
+    """25 whole chunks, one per lane of 32, and two row sets to a wave."""
+    _C.tune("softmax_rows_per_wave", 2)
+    try:
+        check_causal(device, 2, 7, 200, dtype, 0.25)
+        check_causal_dropout(device, 2, 7, 200, dtype, 0.25, 0.1)
+        check_masked(device, 2, 2, 7, 200, dtype, 0.25, "padding")
+        check_masked_dropout(device, 2, 2, 7, 200, dtype, 0.25, "full", 0.1)
+        check_bias(device, 2, 2, 7, 200, dtype, 0.25, "t5", False)
+        check_bias_dropout(device, 2, 2, 7, 200, dtype, 0.25, "perq", True, 0.1)
+        check_causal_masked(device, 2, 2, 7, 200, dtype, 0.25, "holes")
+    finally:
+        _C.tune("softmax_rows_per_wave", 0)
