@@ -637,9 +637,13 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     }
     mx[j] = m;
   }
+  if constexpr (RPW == 4 && LPR < kWave) {
+    group_allreduce4<OpMax, LPR>(mx);
+  } else {
 #pragma unroll
-  for (int j = 0; j < RPW; ++j)
-    mx[j] = row_reduce_max<LPR>(mx[j], red[0], wave, first, g.wpr, lane);
+    for (int j = 0; j < RPW; ++j)
+      mx[j] = row_reduce_max<LPR>(mx[j], red[0], wave, first, g.wpr, lane);
+  }
   // (one barrier separates the two LDS areas; RPW > 1 implies wpr == 1,
   //  where LDS is not used at all)
 
@@ -673,9 +677,13 @@ __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
     }
     sm[j] = s;
   }
+  if constexpr (RPW == 4 && LPR < kWave) {
+    group_allreduce4<OpSum, LPR>(sm);
+  } else {
 #pragma unroll
-  for (int j = 0; j < RPW; ++j)
-    sm[j] = row_reduce_sum<LPR>(sm[j], red[1], wave, first, g.wpr, lane);
+    for (int j = 0; j < RPW; ++j)
+      sm[j] = row_reduce_sum<LPR>(sm[j], red[1], wave, first, g.wpr, lane);
+  }
   if constexpr (RAG && DROP) {
     // a row without a visible key is uniform: all of it is drawn
     if (rvalid[0] && mx[0] == ninf && !kBias)
