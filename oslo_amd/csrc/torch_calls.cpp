@@ -1066,11 +1066,14 @@ Shape dropout_words(const Dropout &d) { return {word_of(d.p), (int64_t)d.seed, (
 Dropout dropout_of(const Shape &w, size_t at = 0) { return {real_of(w[at]), (uint64_t)w[at + 1], (uint64_t)w[at + 2]}; }
 
 // LayerNorm and RMSNorm, with or without parameters, of one or of mixed dtypes.
+// Without a weight it is the norm without parameters, in the input's dtype,
+// whatever the bias, which gets no gradient then.
 struct NormFunction : Function<NormFunction> {
   static Tensor forward(AutogradContext *ctx, const Tensor &input, const OptTensor &weight, const OptTensor &bias,
                         bool rms, bool mixed, const Shape &shape, double eps) {
-    const Tensor x = input.contiguous(), w = contiguous(weight), b = contiguous(bias);
-    const NormOut r = norm_fwd(rms, x, shape, w, b, eps, mixed);
+    TORCH_CHECK(rms || !given(weight) || given(bias), "LayerNorm with a weight needs a bias");
+    const Tensor x = input.contiguous(), w = contiguous(weight), b = w.defined() ? contiguous(bias) : Tensor();
+    const NormOut r = norm_fwd(rms, x, shape, w, b, eps, mixed && w.defined());
     ctx->save_for_backward({x, w, b, r.mean, r.inv});
     Shape words{rms};
     words.insert(words.end(), shape.begin(), shape.end());

@@ -141,6 +141,32 @@ def test_native_and_python_functions_agree(device, name, dtype, layout):
         assert (node is not None) == bool(mask) and (node is None or "CppFunction" in type(node).__name__)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("name", ["layer_norm_affine", "mixed_layer_norm", "rms_norm_affine", "mixed_rms_norm"])
+def test_a_norm_without_a_weight(device, name, bias, dtype):
+    """The norm without parameters, in the input's dtype; a bias is not looked at."""
+    _, native, python = OPS[name]
+    if bias and "rms" in name:
+        pytest.skip("RMSNorm has no bias")
+    operands = norm_operands(dtype, device, w=BF16)[::2] if bias else norm_operands(dtype, device)[:1]
+    rest = () if "rms" in name or bias else (None,)
+    for mask in range(1 << len(operands)):
+        got = [evaluate(lambda x, *b, s, f=f: f(x, None, *b, *rest, s), operands, mask, "contiguous", device)
+               for f in (native, python)]
+        assert all(equal(a, b) for k in (0, 1) for a, b in zip(got[0][k], got[1][k])), mask
+        assert got[0][0][0].dtype == dtype and (got[0][2] is None) == (got[1][2] is None)
+
+
+def test_a_layer_norm_with_a_weight_needs_a_bias(device):
+    x, w, _ = norm_operands(F32, device, w=F32)
+    for call in (F.fused_layer_norm_affine, F.mixed_dtype_fused_layer_norm_affine):
+        before = torch.cuda.memory_stats(device)["allocation.all.allocated"]
+        with pytest.raises(RuntimeError, match="needs a bias"):
+            call(x, w, None, (48,))
+        assert torch.cuda.memory_stats(device)["allocation.all.allocated"] == before
+
+
 def test_only_the_sum_of_a_residual_norm_is_used(device):
     """No gradient arrives at the normalised output: the norm's parameters get none."""
     make, native, python = OPS["residual_layer_norm_0.3"]
