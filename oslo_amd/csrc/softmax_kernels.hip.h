@@ -1672,6 +1672,17 @@ static SoftmaxPlan plan_softmax_ragged(int64_t sk, RaggedPass pass, bool shared_
   while (p.rpb * p.wpr > 16) --p.rpb;
   return p;
 }
+// The blocks of ragged rows that are dealt out by die (work_block): all groups of
+// 64.  Not those of rows of whole waves that add a term shared by the batch: the
+// blocks of the same rows of its entries are 16 apart there and meet on one die in
+// launch order, whose L2 serves the term to all but the first (fp32 forward at
+// 300 MB, by die / in launch order: 1111 keys 106 / 87 us, 1777: 183 / 148, bf16
+// 1777: 130 / 118).  In lane groups the rows of one run fill two to four blocks and
+// the die makes up for it (fp32 97 keys 147 / 158).
+template <int MODE> static int64_t ragged_die_end(const SoftmaxGeom &g, const SoftmaxPlan &pl, int64_t nblocks) {
+  return MODE == kModeBias && g.batch_inner && pl.lpr == kWave ? 0 : nblocks & ~(int64_t)63;
+}
+
 // ... and the builds that it can come out with
 template <typename T, int MODE>
 constexpr bool ragged_plan_reaches(int vpl, int lpr, RaggedPass pass) {
@@ -1961,7 +1972,7 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
       softmax_waves_per_cu<T, MODE>(pl, g.sk, false, drop, g.causal, ragged, g.batch_inner != 0),
       threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
-  if (ragged) g.die_end = nblocks & ~(int64_t)63;
+  if (ragged) g.die_end = ragged_die_end<MODE>(g, pl, nblocks);
 #define OSLO_SM_FWD(VPL, RPW, LPR_)                                  \
   if constexpr (VPL * RPW * E <= (MODE == kModeBias ? kBiasMaxElems : kFwdMaxElems)) { \
     if (drop)                                                        \
@@ -2076,7 +2087,7 @@ int launch_softmax_bwd(const void *dy, const void *y,
   const unsigned occ = occupancy_lds(
       softmax_waves_per_cu<T, MODE>(pl, g.sk, true, false, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
-  if (ragged) g.die_end = nblocks & ~(int64_t)63;
+  if (ragged) g.die_end = ragged_die_end<MODE>(g, pl, nblocks);
 #define OSLO_SM_BWD(VPL, RPW, LPR_)                        \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_))       \
     softmax_bwd_kernel<T, VPL, RPW, MODE, LPR_>            \
@@ -2152,7 +2163,7 @@ int launch_softmax_dropout_bwd(const void *dy, const void *x,
   const unsigned occ = occupancy_lds(
       softmax_waves_per_cu<T, MODE>(pl, g.sk, true, true, g.causal, ragged), threads, nblocks);
   const int64_t per_launch = max_workgroups(threads);
-  if (ragged) g.die_end = nblocks & ~(int64_t)63;
+  if (ragged) g.die_end = ragged_die_end<MODE>(g, pl, nblocks);
 #define OSLO_SM_DBWD(VPL, RPW, LPR_)                                \
   if constexpr (bwd_plan_reaches<T>(VPL, RPW, LPR_) && (MODE != kModeBias || RPW <= 2)) \
     softmax_dropout_bwd_kernel<T, VPL, RPW, MODE, LPR_>             \

@@ -1,0 +1,19 @@
+"""The lines of the launch rules that row counts, the mask and the type move:
+each side of them against the float64 oracle, through the checks (and
+tolerances) of the per-op tests."""
+import pytest
+import torch
+
+from test_gpu_softmax_bias import test_bias_softmax as check_bias
+from test_gpu_softmax_bias import test_bias_softmax_dropout as check_bias_dropout
+
+pytestmark = pytest.mark.gpu
+
+F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
+
+
+@pytest.mark.parametrize("dtype,sk", [(F32, 97), (F32, 397), (F32, 1111), (BF16, 389), (BF16, 1003), (F16, 2049)])
+def test_blocks_of_a_term_shared_by_the_batch(device, dtype, sk):
+    """More than 64 blocks of ragged rows, in lane groups and in whole waves."""
+    check_bias(device, 3, 2, 96, sk, dtype, 0.25, "t5", False)
+    check_bias_dropout(device, 3, 2, 96, sk, dtype, 0.25, "t5", False, 0.1)
