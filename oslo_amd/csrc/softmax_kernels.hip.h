@@ -1504,9 +1504,10 @@ struct SoftmaxPlan {
 };
 
 // Rows that do not fill two chunks per lane of 8, 16 or 32 lanes and take them
-// all the same: the most chunks for each, and the fewest altogether.
+// all the same: the most chunks for each, the fewest altogether, and the row sets
+// of a wave then.
 struct TwoChunks {
-  int most8, most16, most32, from;
+  int most8, most16, most32, from, rpw;
 };
 
 // max_elems: elements of one operand a lane may hold (register budget).
@@ -1553,7 +1554,8 @@ static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
                       nchunks <= (q == 8 ? two->most8 : q == 16 ? two->most16 : two->most32);
     if (q != 0 && (nchunks == 2 * q || part)) {
       // one row set per wave without a mask tensor, two with one (measured)
-      int want = g_tune.softmax_rows_per_wave > 0 ? g_tune.softmax_rows_per_wave : default_rpw;
+      int want = g_tune.softmax_rows_per_wave > 0 ? g_tune.softmax_rows_per_wave
+                                                  : (part ? two->rpw : default_rpw);
       p.vpl = 2;
       p.rpw = want >= 2 && 2 * 2 * E <= max_elems ? 2 : 1;
       p.wpr = 1;
@@ -1776,6 +1778,7 @@ static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bo
   } else {
     kb = MODE == kModeMasked ? 112 : 64;
     if (MODE == kModeBias && pl.rpw > 1) kb = 96;
+    if (MODE == kModeBias && !k16 && !drop && pl.rpw == 2 && pl.vpl == 2 && pl.lpr < kWave) return 18;
     if (drop) kb = 96;
     if (pl.wpr > 1 && kb < 96) kb = 96;
     if (ragged && pl.vpl == 3 && pl.lpr < kWave && drop && MODE == kModeCausal)
@@ -1927,7 +1930,11 @@ int launch_softmax_fwd(const void *x, const uint8_t *mask, void *y,
   //  93; 176: 98, 83 / 83, 82.  Longer rows gain behind a key mask with the diagonal,
   //  504 bf16 keys 106, 86 / 88, 83, but add in the order of the key mask alone)
   constexpr bool k16 = sizeof(T) == 2;
-  constexpr TwoChunks two = {k16 ? 9 : 8, k16 ? 20 : 16, 44, k16 ? 9 : 34};
+  // (with a term, fp32 takes two row sets then: in one the two chunks wait for each
+  //  other, 140 keys 117 us by one chunk, 128 / 114 with one / two sets, 164: 105, 119
+  //  / 106, with dropout 163, 130 / 123)
+  const TwoChunks two = {k16 ? 9 : 8, k16 ? 20 : 16, 44, k16 ? 9 : 34,
+                         MODE == kModeBias && !k16 ? 2 : default_rpw};
   SoftmaxPlan pl = plan_softmax(g.sk, E, cap, default_rpw, 4, &two);
   if (!pl.ok && cap < kFwdMaxElems && MODE != kModeBias)
     pl = plan_softmax(g.sk, E, kFwdMaxElems, default_rpw, 4);

@@ -12,6 +12,15 @@ pytestmark = pytest.mark.gpu
 F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
 
 
+@pytest.mark.parametrize("sk", [132, 136, 140, 156, 172, 176, 180])
+@pytest.mark.parametrize("sq", [1, 7])
+def test_fp32_rows_with_a_term_in_two_row_sets(device, sq, sk):
+    """34 to 44 chunks: two sets of rows to a wave, the last one partly empty."""
+    check_bias(device, 3, 1, sq, sk, F32, 0.25, "t5", False)
+    check_bias(device, 1, 3, sq, sk, F32, 0.25, "perq", True)
+    check_bias_dropout(device, 3, 1, sq, sk, F32, 0.25, "t5", False, 0.1)
+
+
 @pytest.mark.parametrize("dtype,sk", [(F32, 97), (F32, 397), (F32, 1111), (BF16, 389), (BF16, 1003), (F16, 2049)])
 def test_blocks_of_a_term_shared_by_the_batch(device, dtype, sk):
     """More than 64 blocks of ragged rows, in lane groups and in whole waves."""
