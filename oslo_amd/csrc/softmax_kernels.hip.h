@@ -1760,11 +1760,14 @@ static inline unsigned ragged_keep_lds(const SoftmaxPlan &pl) {
 // -> 144).  Behind a key mask three chunks in 8 or 16 lanes take 24 to 28 waves
 // (bf16 133 keys 160 -> 146, with dropout 167 -> 152; 305: 124 -> 111, fp32 173: 112
 // -> 108), but not 16 lanes in 16 bits with dropout (373 keys: 111, with 24 waves
-// 118).  A term that the batch shares is served by the L2s if fewer rows are under
-// way: 16 waves with dropout (bf16 133 keys 278 -> 249, 345: 191 -> 179, fp32 153:
-// 179 -> 156).
+// 118), nor fp32 under the diagonal while a third of the chunks is empty (131 keys:
+// 107, with 28 waves 108).  A term that the batch shares is served by the L2s if
+// fewer rows are under way: 16 waves with dropout (bf16 133 keys 278 -> 249, 345: 191
+// -> 179, fp32 153: 179 -> 156), in 16 bits of full groups of 16 lanes (261 keys: 194
+// without a limit, 205 with 16, 186 with 23).
 // Additive terms with several rows to a wave, which waits for both operands: 96 KB
-// (bf16 392 keys 373 -> 327 us, fp16 352 keys 387 -> 362 at 900 MB).
+// (bf16 392 keys 373 -> 327 us, fp16 352 keys 387 -> 362 at 900 MB), in fp32 lane
+// groups 72 KB (140 keys 122 -> 114, 172: 114 -> 107).
 template <typename T, int MODE>
 static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bool drop,
                                 bool causal, bool ragged, bool shared_term = false) {
@@ -1785,9 +1788,12 @@ static int softmax_waves_per_cu(const SoftmaxPlan &pl, int sk, bool backward, bo
       return (int)((k16 && pl.lpr == 32 ? 24 : 20) * (int64_t)pl.vpl * pl.lpr /
                    ceil_div(sk, io<T>::EPV));
     if (ragged && pl.vpl == 3 && pl.lpr < 32) {
+      const int nchunks = (int)ceil_div(sk, io<T>::EPV);
+      if (MODE == kModeMasked && !k16 && causal && !drop && nchunks <= 38) return 0;
       if (MODE == kModeMasked && !drop) return k16 && !causal ? 24 : 28;
-      if (MODE == kModeMasked && (!k16 || pl.lpr == 8)) return k16 && causal ? 28 : 24;
-      if (MODE == kModeBias && drop && shared_term) return 16;
+      if (MODE == kModeMasked && (!k16 || pl.lpr == 8)) return k16 && !causal ? 24 : 28;
+      if (MODE == kModeBias && drop && shared_term)
+        return k16 && pl.lpr == 16 ? 16 * 48 / nchunks : 16;
     }
     if (ragged && pl.vpl == 2 && pl.lpr < kWave && !drop && MODE != kModeMasked)
       return (int)((pl.lpr == 8 ? 18 : 24) * (int64_t)pl.vpl * pl.lpr / ceil_div(sk, io<T>::EPV));
