@@ -1623,7 +1623,9 @@ static SoftmaxPlan plan_softmax(int64_t sk, int E, int max_elems,
 // Plain and dropout forward of a row hold it alike, so that they add in one order.
 // The plain backward has neither Philox rounds nor a row to cut twice, and takes
 // two chunks only where one leaves nearly half of the lanes idle: bf16 133 keys
-// 161 -> 140, 261: 161 -> 121, 341: 127 -> 118, but 181: 131 -> 140, 443: 110 -> 116;
+// 161 -> 140, 261: 161 -> 121, 341: 127 -> 118, but 181: 131 -> 140, 443: 110 -> 116
+// (without a diagonal, whose rows need all their chunks, 129: 180 -> 193, 143: 175 ->
+// 182, 341: 160 -> 165, but 317: 168 -> 162);
 // fp32 67: 146 -> 139, 131: 146 -> 120, 171: 121 -> 116, but 189: 114 -> 116.
 // Two rows (of waves or sets of lane groups) to a workgroup: the line that two
 // rows share is then written through one L2 (bf16 1003 keys: causal backward
@@ -1650,6 +1652,8 @@ static SoftmaxPlan plan_softmax_ragged(int64_t sk, RaggedPass pass, bool shared_
   // (16-bit rows behind a mask or with a term: up to where three of 8 lanes
   //  remain the better)
   const bool shared = term && shared_term;
+  // (16-bit plain backward of rows that are not cut off by a diagonal)
+  constexpr bool whole16 = k16 && MODE == kModeDense;
   const int three8 = !k16 || plain ? 0 : fwd ? (term || masked ? 20 : 0) : (term ? 18 : 0);
   if (nchunks <= 8) {
     group(1, 8);
@@ -1659,13 +1663,13 @@ static SoftmaxPlan plan_softmax_ragged(int64_t sk, RaggedPass pass, bool shared_
     group(1, 16);
   } else if (nchunks <= three8) {
     group(3, 8);
-  } else if (nchunks <= (plain ? 18 : shared ? 24 : k16 ? 32 : 28)) {
+  } else if (nchunks <= (plain ? (whole16 ? 16 : 18) : shared ? 24 : k16 ? 32 : 28)) {
     group(2, 16);
   } else if (nchunks <= 32) {
     group(1, 32);
   } else if (nchunks <= (k16 || masked ? 48 : 40) && !plain) {
     group(3, 16);
-  } else if (nchunks <= (plain ? 44 : 64)) {
+  } else if (nchunks <= (plain ? (whole16 ? 42 : 44) : 64)) {
     group(2, 32);
   } else if (nchunks > 64 && nchunks <= 96 && !plain) {
     group(3, 32);
@@ -1695,7 +1699,7 @@ constexpr bool ragged_plan_reaches(int vpl, int lpr, RaggedPass pass) {
   if (lpr == kWave) return vpl > 1 || plain;
   if (vpl == 3 && lpr == 8) return k16 && (term || (masked && pass == kRaggedFwd)) && !plain;
   if (vpl == 3) return !plain;
-  if (vpl == 2) return !plain || lpr != 8;
+  if (vpl == 2) return !plain || (lpr != 8 && !(lpr == 16 && k16 && MODE == kModeDense));
   return lpr != 32 || plain || !k16 || term;
 }
 #define OSLO_SM_RAGGED_CASES(LAUNCH)       \

@@ -4,8 +4,10 @@ tolerances) of the per-op tests."""
 import pytest
 import torch
 
+from test_gpu_softmax import test_masked as check_masked
 from test_gpu_softmax_bias import test_bias_softmax as check_bias
 from test_gpu_softmax_bias import test_bias_softmax_dropout as check_bias_dropout
+from test_gpu_softmax_causal_masked import test_causal_masked as check_causal_masked
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +21,14 @@ def test_fp32_rows_with_a_term_in_two_row_sets(device, sq, sk):
     check_bias(device, 3, 1, sq, sk, F32, 0.25, "t5", False)
     check_bias(device, 1, 3, sq, sk, F32, 0.25, "perq", True)
     check_bias_dropout(device, 3, 1, sq, sk, F32, 0.25, "t5", False, 0.1)
+
+
+@pytest.mark.parametrize("sk", [121, 128, 129, 137, 143, 145, 329, 336, 337, 343, 345])
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_backward_of_ragged_rows_without_a_diagonal(device, dtype, sk):
+    """16, 18, 42 and 43 chunks, which rows under the diagonal hold otherwise."""
+    check_masked(device, 2, 2, 9, sk, dtype, 0.25, "padding")
+    check_causal_masked(device, 2, 2, 9, sk, dtype, 0.25, "padding")
 
 
 @pytest.mark.parametrize("dtype,sk", [(F32, 97), (F32, 397), (F32, 1111), (BF16, 389), (BF16, 1003), (F16, 2049)])
