@@ -198,6 +198,24 @@ def test_norm_launch_table(device, tuned, name, chunks):
     assert _under_each(settings, lambda s: run()) >= 1
 
 
+# A launch of few rows takes fewer chunks per lane (two waves per SIMD at most): the
+# rows above find those builds, these the ones of large batches under the defaults.
+MANY_ROWS = {100: 2100, 128: 2100, 160: 1100, 200: 1100, 256: 1100, 300: 800, 320: 800, 384: 800, 512: 600, 640: 500,
+             768: 450, 1000: 300, 1024: 300, 1536: 200, 2048: 140}
+
+
+@pytest.mark.parametrize("name", ["f32-f32", "f16-f16", "bf16-bf16", "f32-f16", "f32-bf16"])
+@pytest.mark.parametrize("chunks", sorted(MANY_ROWS))
+def test_norms_of_many_rows(device, name, chunks):
+    tin, tout = (DTYPE[n] for n in name.split("-"))
+    n1, n2 = MANY_ROWS[chunks], chunks * (8 if "16" in name else 4)
+    check_layer_norm(device, n1, n2, tin, tout, True)
+    check_rms_norm(device, n1, n2, tin, tout, True)
+    if tin == tout:
+        check_fused(device, n1, n2, tin, 0.1, False)
+        check_fused(device, n1, n2, tin, 0.1, True)
+
+
 # ------------------------------------------------------------------ element-wise kernels
 ELTWISE_SETTINGS = [{"eltwise_unroll": v} for v in (1, 2, 4, 8)] + [
     {"eltwise_fwd_steps": 4}, {"eltwise_tile_max": 256}, {"eltwise_tile_min": 64},
