@@ -1021,19 +1021,19 @@ static int launch_norm_fwd(const void *x, const void *gamma, const void *beta,
       sp = split_row(n2 / E, 32 / E, kVpl, 4, waves);
   }
   // The fused build holds two more packed operands per chunk: at most 16
-  // elements per lane.  Measured on MI355X: 16-bit, 16 per lane while a row then
-  // fits four waves, else 8 per lane over up to twelve waves, else 16 per lane.
-  // fp32, 8 per lane (16 only where a row would not fit): 16 spill in the builds
-  // for more than four waves ([8886, 7552] 337 -> 182 us, [2164, 4672] 65.7 ->
-  // 33.2) and are slower below ([2006, 4096] 27.6 -> 25.2, [8192, 1024] 27.6 ->
-  // 25.0, and no faster at [16384, 4096]).
+  // elements per lane.  Measured on MI355X: 16 per lane while a row then fits four
+  // waves, else 8 per lane: fp32 always (16 only where a row would not fit: they
+  // spill in the builds for more than four waves, [8886, 7552] 337 -> 182 us, [2164,
+  // 4672] 65.7 -> 33.2), 16-bit over up to twelve waves, else 16 per lane.  (fp32 with
+  // 8 per lane in rows of up to four waves of 16: [8192, 1024] 27.6 -> 25.0, but [3000,
+  // 1536] 15.1 -> 18.3, [1500, 3072] 15.8 -> 18.2, RMSNorm [3000, 640] 7.2 -> 8.9.)
   bool fused_big = false;
   if (fused && vec_ok) {
     const int waves = g_tune.norm_fwd_waves > 0 ? g_tune.norm_fwd_waves : 4;
     if (g_tune.norm_fwd_vpl > 0) {
       const int cap = g_tune.norm_fwd_vpl < 16 / E ? g_tune.norm_fwd_vpl : 16 / E;
       sp = split_row(n2 / E, cap, kVpl, 4, waves);
-    } else if (E == 4) {
+    } else if (E == 4 && n2 / E > kWave * 4 * 4) {
       sp = split_row(n2 / E, few_rows_chunks(2, n1, n2 / E), kVpl, 4,
                      g_tune.norm_fwd_waves > 0 ? waves : 8);
       if (!sp.ok) sp = split_row(n2 / E, 4, kVpl, 4, waves);
