@@ -1069,16 +1069,24 @@ static int launch_norm_fwd(const void *x, const void *gamma, const void *beta,
   // are spread over that many rows
   // (LayerNorm: two groups, the second one prefetched; RMSNorm is fastest
   // with short-lived workgroups)
-  // A launch of up to three workgroups per CU takes one group in each: the
-  // second would wait for the first while the chip has room ([2048, 768] bf16
-  // 4.6 -> 3.9 us, [3048, 1024] 4.8 -> 4.2, with the fused prologue and dropout
-  // 6.9 -> 5.1 and 8.9 -> 7.4; [2006, 4096], four workgroups, the same).
-  auto iters_of = [&](int64_t groups) {
+  // A launch of up to three workgroups of four waves per CU takes one group in
+  // each: the second would wait for the first while the chip has room ([2048, 768]
+  // bf16 4.6 -> 3.9 us, [3048, 1024] 4.8 -> 4.2, with the fused prologue and
+  // dropout 6.9 -> 5.1 and 8.9 -> 7.4; [2006, 4096], four workgroups, the same).
+  // Rows that take a whole workgroup, more than one and up to two to a CU, go two
+  // to a workgroup, with the second one's loads in flight: one to each leaves some
+  // CUs with two in turn ([300, 8192] fp32 LayerNorm
+  // 7.4 -> 5.8 us, [512, 12288] 10.9 -> 9.1, fused 42.9 -> 30.8; LayerNorm from six
+  // waves a row on, RMSNorm and the fused build, which gain from the room, from nine).
+  const int64_t cus = device_cu_count();
+  auto iters_of = [&](int64_t groups, int waves) {
     if (g_tune.norm_fwd_iters > 0) return g_tune.norm_fwd_iters;
-    if (groups <= (int64_t)device_cu_count() * 3) return 1;
+    if (groups <= cus) return 1;
+    if (sp.rpb == 1 && groups <= 2 * cus && waves >= (RMS || fused ? 9 : 6)) return 2;
+    if (groups * waves <= 12 * cus) return 1;
     return (RMS && !(E == 8 && n2 / E > kWave * 4 * 4)) ? 1 : 2;
   };
-  int iters = iters_of(ceil_div(n1, sp.rpb));
+  int iters = iters_of(ceil_div(n1, sp.rpb), sp.wpr * sp.rpb);
   int64_t grid = ceil_div(ceil_div(n1, sp.rpb), iters);
   const int64_t maxgrid = (int64_t)device_cu_count() * 64;
   if (grid > maxgrid) grid = maxgrid;
@@ -1087,7 +1095,7 @@ static int launch_norm_fwd(const void *x, const void *gamma, const void *beta,
   if (const int l3 = lanes_per_row_x3(n2 / E)) {
     const int threads3 = 256;
     const int rpb3 = (threads3 / kWave) * (kWave / l3);
-    iters = iters_of(ceil_div(n1, rpb3));
+    iters = iters_of(ceil_div(n1, rpb3), threads3 / kWave);
     int64_t grid3 = ceil_div(ceil_div(n1, rpb3), iters);
     if (grid3 > maxgrid) grid3 = maxgrid;
 #define OSLO_FWD_X3(LPR_)                                                    \
@@ -1124,7 +1132,7 @@ static int launch_norm_fwd(const void *x, const void *gamma, const void *beta,
     const int threads_l = kWave * waves_l;
     const int rpb_eff = waves_l * (kWave / lpr);
     const bool even_l = (n2 / E) == lpr;
-    iters = iters_of(ceil_div(n1, rpb_eff));
+    iters = iters_of(ceil_div(n1, rpb_eff), waves_l);
     int64_t grid_l = ceil_div(ceil_div(n1, rpb_eff), iters);
     if (grid_l > maxgrid) grid_l = maxgrid;
     if constexpr (kCanFuse) {

@@ -4,6 +4,9 @@ tolerances) of the per-op tests."""
 import pytest
 import torch
 
+from test_gpu_norm import test_layer_norm as check_layer_norm
+from test_gpu_norm import test_rms_norm as check_rms_norm
+from test_gpu_residual_norm import test_fused_vs_oracle as check_fused
 from test_gpu_softmax import test_masked as check_masked
 from test_gpu_softmax_bias import test_bias_softmax as check_bias
 from test_gpu_softmax_bias import test_bias_softmax_dropout as check_bias_dropout
@@ -36,3 +39,13 @@ def test_blocks_of_a_term_shared_by_the_batch(device, dtype, sk):
     """More than 64 blocks of ragged rows, in lane groups and in whole waves."""
     check_bias(device, 3, 2, 96, sk, dtype, 0.25, "t5", False)
     check_bias_dropout(device, 3, 2, 96, sk, dtype, 0.25, "t5", False, 0.1)
+
+
+# rows of a whole workgroup, one and up to two of them to a CU, and beyond
+@pytest.mark.parametrize("n1,n2,dtype", [
+    (255, 6144, F32), (257, 6144, F32), (511, 8192, F32), (513, 8192, F32), (300, 12288, BF16), (515, 12288, BF16)])
+def test_two_rows_to_a_workgroup(device, n1, n2, dtype):
+    check_layer_norm(device, n1, n2, dtype, dtype, True)
+    check_rms_norm(device, n1, n2, dtype, dtype, True)
+    check_fused(device, n1, n2, dtype, 0.1, False)
+    check_fused(device, n1, n2, dtype, 0.1, True)
