@@ -590,7 +590,7 @@ int64_t colsum_parts_eltwise(int64_t rows, int64_t cols) {
 // (bf16 [269, 2048], finalize included: bias-GeLU 9.0 -> 7.1 us, bias-dropout-add
 // 8.2 -> 6.9; fp32 [108, 768] 5.9 -> 5.3 and 6.5 -> 5.5.)
 static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int *unroll, int E,
-                                       int per_cu = kBwdWorkgroupsPerCu) {
+                                       int per_cu = kBwdWorkgroupsPerCu, bool even = false) {
   EltGeom g;
   g.rows = rows;
   g.cols = cols;
@@ -601,6 +601,14 @@ static inline EltGeom eltwise_geom_bwd(int64_t rows, int64_t cols, int *unroll, 
     while (*unroll > 1 && ceil_div(rows, (int64_t)g.ty * *unroll) < most) *unroll /= 2;
   const int64_t nsteps = ceil_div(rows, (int64_t)g.ty * *unroll);
   g.slots = most < nsteps ? most : nsteps;
+  // One or two steps in finer slots: as many in each (bias-dropout-add bf16 [1500,
+  // 5120], 188 steps: 11.7 us in 94 slots of at least 16 rows, 12.9 in 128, of which
+  // 60 take a second step.  fp32 and bias-GeLU, with less to do per step and more,
+  // are faster in the uneven slots: [1000, 5120] 11.4 against 12.5, bf16 [600, 5120]
+  // 8.7 against 9.4.)
+  if (even && g_tune.eltwise_unroll == 0 && nsteps <= 2 * g.slots &&
+      g.slots > colsum_parts_eltwise_e(rows, cols, E, false, per_cu))
+    g.slots = ceil_div(nsteps, ceil_div(nsteps, g.slots));
   return g;
 }
 
@@ -840,7 +848,7 @@ static int run_bda_bwd(const void *gr, void *dx, void *dbias, void *ws,
     return generic_colsum_of_stored<T>(dx, dbias, ws, ws_bytes, rows, cols, st);
   }
   int unroll = eltwise_unroll(4);
-  EltGeom g = eltwise_geom_bwd(rows, cols, &unroll, kE);
+  EltGeom g = eltwise_geom_bwd(rows, cols, &unroll, kE, kBwdWorkgroupsPerCu, sizeof(T) == 2);
   float *part = nullptr;
   if (dbias != nullptr) {
     const int64_t need = fit_workspace(&g, kE, kBwdWorkgroupsPerCu, ws, ws_bytes);

@@ -4,6 +4,10 @@ tolerances) of the per-op tests."""
 import pytest
 import torch
 
+from helpers import check, f64, randn
+from oracle import closed_form as cf
+from oracle import philox
+from oslo_amd.torch import _C
 from test_gpu_norm import test_layer_norm as check_layer_norm
 from test_gpu_norm import test_rms_norm as check_rms_norm
 from test_gpu_residual_norm import test_fused_vs_oracle as check_fused
@@ -49,3 +53,15 @@ def test_two_rows_to_a_workgroup(device, n1, n2, dtype):
     check_rms_norm(device, n1, n2, dtype, dtype, True)
     check_fused(device, n1, n2, dtype, 0.1, False)
     check_fused(device, n1, n2, dtype, 0.1, True)
+
+
+# bias-dropout-add: steps that fill the finer slots, one too many, two each
+@pytest.mark.parametrize("rows,cols,dtype", [
+    (256, 5120, BF16), (258, 5120, BF16), (300, 6144, F16), (800, 5120, BF16), (1500, 5120, BF16), (1500, 5120, F32)])
+def test_column_sums_of_a_few_steps(device, rows, cols, dtype):
+    g = randn((rows, cols), dtype, rows + cols)
+    dx, db = _C.get_fused_elementwise_kernel().bias_dropout_add_backward(g.to(device), 0.2, 9, 4)
+    keep = torch.from_numpy(philox.keep_mask(rows * cols, 0.2, 9, 4)).view(rows, cols).bool()
+    check(dx, cf.bias_dropout_add_bwd(f64(g), keep.numpy(), 0.2)[0], "dx", atol=1e-6)
+    # (the sum of dx as stored, in float32: relative 2^-24 of each of `rows` terms of order one)
+    check(db, dx.double().sum(0).cpu().numpy(), "dbias", atol=1e-5 * rows ** 0.5 + 1e-6, min_exact=0.97)
