@@ -122,9 +122,11 @@ __global__ __launch_bounds__(256) void bias_gelu_fwd_kernel(
 
 // Folds the per-lane column sums of the ty rows of the workgroup and writes
 // the partial row of this slot.  Bound: the latency of the LDS reads, at the end
-// of every workgroup.  Each thread adds kE values whatever the shape of the tile:
-// by the first row of lanes alone, tiles of 16 lanes added 128 values in each
-// (whole backward, finalize included, bf16 [59, 448] 9.5 -> 5.3 us, [512, 768] 8.1
+// of every workgroup: a column has ty = 256 / tx values, and one thread adds them
+// one after the other; the kE * tx columns of the tile are dealt out over all 256
+// threads (in tiles of fewer columns than that some idle).  By the first row of
+// lanes alone a thread did kE columns, 128 values in tiles of 16 lanes, where 16 are
+// left now (whole backward, finalize included, bf16 [59, 448] 9.5 -> 5.3 us, [512, 768] 8.1
 // -> 5.9, [27294, 704] 28.3 -> 24.3).  sh is [ty][kE][tx] floats, with eight
 // columns of padding from 32 lanes on, so that the lanes that read kE values of
 // neighbouring chunks meet 64 different banks.

@@ -438,8 +438,8 @@ constexpr int keep_bytes(int lanes, int vpl) { return lanes * vpl + 2; }
 // visible key stores {0, -1 / sk}.
 //
 // LPR lanes hold a row: 64 (a row takes whole waves), or 8 / 16 / 32 for rows
-// of at most LPR chunks, where a wave works on 64 / LPR rows side by side
-// (then VPL == 1 and wpr == 1).
+// of at most LPR * VPL chunks, where a wave works on 64 / LPR rows side by side
+// (then wpr == 1 and VPL is 1 to 3).
 template <typename T, int VPL, int RPW, int MODE, bool DROP, int LPR = kWave,
           bool RAG = false>
 __global__ __launch_bounds__(1024) void softmax_fwd_kernel(
