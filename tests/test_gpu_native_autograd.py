@@ -1,8 +1,8 @@
 """The native autograd Functions against the Python ones that they stand in for
 on eager GPU calls: outputs and gradients bit for bit over operand layouts and
 requires-grad subsets, and the parts of torch that look at an autograd node
-(saved-tensor hooks, version counters, tracing, vmap, forward mode, several
-threads, a second stream)."""
+(saved-tensor hooks, version counters, second derivatives, tracing, vmap, forward
+mode, several threads, a second stream)."""
 import threading
 
 import pytest
@@ -237,8 +237,30 @@ def test_large_outputs_that_are_placed_in_a_larger_allocation(device):
     w = F._ScaledUpperTriangMaskedSoftmax.apply(z, 1.0)
     w.backward(g)
     assert torch.equal(y, w) and torch.equal(x.grad, z.grad)
-    (y * 1.0).mul_(2.0)
+    # (in place on the output itself: refused by torch for a view that a Function returns)
+    for out in (y, w):
+        with pytest.raises(RuntimeError, match="modified inplace|modified in-place"):
+            out.mul_(2.0)
     y.detach().mul_(2.0)  # (an ordinary tensor to its user)
+    small = F.scaled_upper_triang_masked_softmax(x[:1, :8, :8], 1.0)
+    assert torch.equal(small.mul_(2.0), 2.0 * F.scaled_upper_triang_masked_softmax(x[:1, :8, :8], 1.0))
+
+
+@pytest.mark.parametrize("name", sorted(OPS))
+def test_second_derivatives_are_as_absent_as_in_python(device, name):
+    """A backward pass that is asked for its own graph: the gradients, and whether
+    they carry one, as the Python Function gives them."""
+    make, native, python = OPS[name]
+    got = []
+    for call in (native, python):
+        leaves = [t.requires_grad_() for t in make(BF16, device)]
+        torch.manual_seed(11)
+        out = call(*leaves, s=random_state(device))
+        outs = list(out) if isinstance(out, tuple) else [out]
+        dys = [rnd(*o.shape, dtype=o.dtype, device=device, seed=20 + k).requires_grad_() for k, o in enumerate(outs)]
+        got.append(torch.autograd.grad(outs, leaves, dys, create_graph=True, allow_unused=True))
+    for a, b in zip(*got):
+        assert equal(a, b) and (a is None or a.requires_grad == b.requires_grad)
 
 
 def test_a_method_replaced_on_the_kernel_object_is_called(device, monkeypatch):
@@ -267,12 +289,15 @@ def test_tracing_records_the_function(device):
 
 
 def test_transforms_that_a_function_without_rules_refuses(device):
+    """The calls go to the native node, which refuses them as torch does of a C++ Function."""
     x = rnd(3, 4, 32, dtype=F32, device=device, seed=1)
-    with pytest.raises(RuntimeError):
+    with pytest.raises(RuntimeError, match="functorch transforms"):
         torch.vmap(lambda t: F.fused_rms_norm(t, (32,)))(x)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.grad(lambda t: F.fused_rms_norm(t, (32,)).sum())(x)
     import torch.autograd.forward_ad as fwad
 
-    with fwad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+    with fwad.dual_level(), pytest.raises((RuntimeError, NotImplementedError), match="jvp"):
         F.fused_rms_norm(fwad.make_dual(x.requires_grad_(), torch.ones_like(x)), (32,))
 
 
