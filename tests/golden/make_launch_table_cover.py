@@ -1,4 +1,4 @@
-"""Makes launch_table_cover.json: a smallest set of (shape, setting) runs of
+"""Makes launch_table_cover.json: a small set of (shape, setting) runs of
 tests/test_gpu_launch_table.py that between them launch every kernel build
 the full sweep launches.
 
@@ -16,8 +16,9 @@ Two steps, on a machine with the GPU (from the repository root):
 
   2. the cover: the trace is cut at the markers, every kernel of the library
      (mangled name, i.e. with its template arguments) is attributed to the
-     runs that launched it, and runs are picked greedily, the one that adds
-     the most kernels first, until every kernel is launched:
+     runs that launched it.  The runs that the table lists already stay; to
+     them runs are added greedily, the one that adds the most kernels first,
+     until every kernel is launched:
 
        python3 tests/golden/make_launch_table_cover.py <dir> <dir>/marks.json
 
@@ -110,9 +111,9 @@ def kernels_per_mark(trace_dir):
     return per_mark
 
 
-def greedy_cover(per_mark):
-    remaining = set().union(*per_mark.values())
-    chosen = []
+def greedy_cover(per_mark, kept=()):
+    chosen = list(kept)
+    remaining = set().union(*per_mark.values()) - set().union(*(per_mark.get(m, set()) for m in chosen))
     while remaining:
         best = max(per_mark, key=lambda m: (len(per_mark[m] & remaining), -m))
         gain = per_mark[best] & remaining
@@ -126,15 +127,30 @@ def greedy_cover(per_mark):
 def main(trace_dir, marks_path):
     marks = {m[0]: m for m in json.load(open(marks_path))}
     per_mark = kernels_per_mark(trace_dir)
-    chosen = greedy_cover(per_mark)
     family = {"test_softmax_launch_table": "softmax", "test_norm_launch_table": "norm",
               "test_elementwise_launch_table": "eltwise"}
-    table = {name: collections.defaultdict(list) for name in family.values()}
-    for m in chosen:
-        _, nodeid, setting = marks[m][:3]
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "launch_table_cover.json")
+
+    def entry(mark):
+        _, nodeid, setting = mark[:3]
         test, params = re.match(r".*::(\w+)\[(.*)\]", nodeid).groups()
         dtype, size = params.rsplit("-", 1)          # "f32-f16-4096" -> "f32-f16", "4096"
-        table[family[test]]["%s:%s" % (dtype, size)].append(setting)
+        return family[test], "%s:%s" % (dtype, size), setting
+
+    listed = {}
+    if os.path.exists(path):
+        with open(path) as f:
+            listed = json.load(f)
+    kept = []
+    for m in sorted(marks):
+        fam, key, setting = entry(marks[m])
+        if setting in listed.get(fam, {}).get(key, []):
+            kept.append(m)
+    chosen = greedy_cover(per_mark, kept)
+    table = {name: collections.defaultdict(list) for name in family.values()}
+    for m in chosen:
+        fam, key, setting = entry(marks[m])
+        table[fam][key].append(setting)
 
     def shape_order(key):
         dtype, size = key.split(":")
@@ -150,12 +166,11 @@ def main(trace_dir, marks_path):
             lines.append('  "%s": %s%s' % (key, json.dumps(settings, sort_keys=True), "," if j + 1 < len(items) else ""))
         lines.append(" }" + ("," if i + 1 < len(out) else ""))
     lines.append("}")
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "launch_table_cover.json")
     with open(path, "w") as f:
         f.write("\n".join(lines) + "\n")
     kernels = set().union(*per_mark.values())
-    print("%d runs in the sweep, %d kernels launched, %d runs chosen over %d shapes -> %s"
-          % (len(marks), len(kernels), len(chosen), sum(len(t) for t in out.values()), path))
+    print("%d runs in the sweep, %d kernels launched, %d runs kept and %d added over %d shapes -> %s"
+          % (len(marks), len(kernels), len(kept), len(chosen) - len(kept), sum(len(t) for t in out.values()), path))
 
 
 if __name__ == "__main__":
