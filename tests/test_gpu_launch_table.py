@@ -216,6 +216,21 @@ def test_norms_of_many_rows(device, name, chunks):
         check_fused(device, n1, n2, tin, 0.1, True)
 
 
+# Builds that only an override reaches at row lengths that the sweeps leave out.
+@pytest.mark.parametrize("tout", [F16, BF16])
+def test_mixed_layer_norm_of_three_chunks_in_eight_waves(device, tuned, tout):
+    _C.tune("norm_fwd_vpl", 3)
+    check_layer_norm(device, 5, 1536 * 8, F32, tout, True)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_two_rows_of_32_lanes_with_a_term(device, tuned, dtype):
+    _C.tune("softmax_lanes_per_row", 32)
+    _C.tune("softmax_rows_per_wave", 2)
+    check_bias(device, 2, 2, 5, 40, dtype, 0.25, "t5", False, rows_per_wave=(2, 2))
+    check_bias_dropout(device, 2, 2, 5, 40, dtype, 0.25, "perq", True, 0.1)
+
+
 # ------------------------------------------------------------------ element-wise kernels
 ELTWISE_SETTINGS = [{"eltwise_unroll": v} for v in (1, 2, 4, 8)] + [
     {"eltwise_fwd_steps": 4}, {"eltwise_tile_max": 256}, {"eltwise_tile_min": 64},
